@@ -199,18 +199,25 @@ struct vb_batch {
       for (size_t l = 0; l < rec[m].size(); ++l)
         if (solves[(size_t)M[m]->lanes[l]]->record_pair(rec[m][l]) == 0) return false;
     }
-    const auto& s0 = rec[0][0].seq;
+    // The members share their stage combines, in order; between two of them
+    // each runs its own launches (sizes differ in the prefix kernels they use).
+    // pos[m]: the combines' positions in member m's sequence
+    std::vector<std::vector<size_t>> pos(M.size());
     for (size_t m = 0; m < M.size(); ++m) {
       const auto& g0 = rec[m][0].seq;
+      for (size_t k = 0; k < g0.size(); ++k)
+        if (vb::zstage_multi_op(g0[k].op)) pos[m].push_back(k);
+      if (pos[m].size() != pos[0].size()) return false;
+      for (size_t i = 0; i < pos[m].size(); ++i)
+        if (g0[pos[m][i]].op != rec[0][0].seq[pos[0][i]].op) return false;
       for (size_t l = 0; l < rec[m].size(); ++l) {
         const auto& sl = rec[m][l].seq;
-        if (sl.size() != s0.size()) return false;
-        for (size_t k = 0; k < s0.size(); ++k) {
-          if (sl[k].op != s0[k].op) return false;   // every lane of every member: the same ops in order
-          if (sl[k].launch_tab != g0[k].launch_tab || sl[k].args.size() != g0[k].args.size() ||
-              sl[k].grid.x != g0[k].grid.x || sl[k].grid.y != g0[k].grid.y || sl[k].block.x != g0[k].block.x)
+        if (sl.size() != g0.size()) return false;
+        for (size_t k = 0; k < g0.size(); ++k)
+          if (sl[k].op != g0[k].op || sl[k].launch_tab != g0[k].launch_tab ||
+              sl[k].args.size() != g0[k].args.size() || sl[k].grid.x != g0[k].grid.x ||
+              sl[k].grid.y != g0[k].grid.y || sl[k].block.x != g0[k].block.x)
             return false;   // within a group: the same launches
-        }
       }
     }
     auto upload = [&](const std::vector<unsigned char>& h) {
@@ -223,40 +230,43 @@ struct vb_batch {
     // the tables: per member and launch for the group launches; per stage
     // combine, the argument structs, first column groups and lengths of all
     // solves of all members
-    std::vector<std::vector<unsigned char*>> gtab(M.size(), std::vector<unsigned char*>(s0.size(), nullptr));
-    std::vector<vb::ZsMultiArgs> margs(s0.size());
-    std::vector<unsigned> mblocks(s0.size(), 0);
-    for (size_t k = 0; k < s0.size(); ++k) {
-      if (vb::zstage_multi_op(s0[k].op)) {
-        std::vector<unsigned char> args;
-        std::vector<int> first, len;
-        int acc = 0;
-        for (size_t m = 0; m < M.size(); ++m)
-          for (size_t l = 0; l < rec[m].size(); ++l) {
-            const auto& x = rec[m][l].seq[k];
-            if (x.block.x != 256 || x.grid.y != 1) return false;
-            args.insert(args.end(), x.args.begin(), x.args.end());
-            first.push_back(acc);
-            len.push_back(solves[(size_t)M[m]->lanes[l]]->p.nx);
-            acc += (int)x.grid.x;
-          }
-        std::vector<unsigned char> hf(first.size() * sizeof(int)), hn(len.size() * sizeof(int));
-        std::memcpy(hf.data(), first.data(), hf.size());
-        std::memcpy(hn.data(), len.data(), hn.size());
-        margs[k].args = upload(args);
-        margs[k].first = reinterpret_cast<const int*>(upload(hf));
-        margs[k].n = reinterpret_cast<const int*>(upload(hn));
-        margs[k].nsolve = (int)first.size();
-        mblocks[k] = (unsigned)acc;
-      } else {
-        for (size_t m = 0; m < M.size(); ++m) {
-          const size_t a = rec[m][0].seq[k].args.size();
-          std::vector<unsigned char> h(a * rec[m].size());
-          for (size_t l = 0; l < rec[m].size(); ++l)
-            std::copy(rec[m][l].seq[k].args.begin(), rec[m][l].seq[k].args.end(), h.begin() + l * a);
-          gtab[m][k] = upload(h);
-        }
+    std::vector<std::vector<unsigned char*>> gtab(M.size());
+    for (size_t m = 0; m < M.size(); ++m) {
+      gtab[m].assign(rec[m][0].seq.size(), nullptr);
+      for (size_t k = 0; k < gtab[m].size(); ++k) {
+        if (vb::zstage_multi_op(rec[m][0].seq[k].op)) continue;
+        const size_t a = rec[m][0].seq[k].args.size();
+        std::vector<unsigned char> h(a * rec[m].size());
+        for (size_t l = 0; l < rec[m].size(); ++l)
+          std::copy(rec[m][l].seq[k].args.begin(), rec[m][l].seq[k].args.end(), h.begin() + l * a);
+        gtab[m][k] = upload(h);
       }
+    }
+    const size_t nst = pos[0].size();
+    std::vector<vb::ZsMultiArgs> margs(nst);
+    std::vector<unsigned> mblocks(nst, 0);
+    for (size_t i = 0; i < nst; ++i) {
+      std::vector<unsigned char> args;
+      std::vector<int> first, len;
+      int acc = 0;
+      for (size_t m = 0; m < M.size(); ++m)
+        for (size_t l = 0; l < rec[m].size(); ++l) {
+          const auto& x = rec[m][l].seq[pos[m][i]];
+          if ((x.block.x != 256 && x.block.x != 64) || x.grid.y != 1) return false;
+          const unsigned per = 256 / x.block.x;   // column groups per shared workgroup
+          args.insert(args.end(), x.args.begin(), x.args.end());
+          first.push_back(acc);
+          len.push_back(solves[(size_t)M[m]->lanes[l]]->p.nx);
+          acc += (int)((x.grid.x + per - 1) / per);
+        }
+      std::vector<unsigned char> hf(first.size() * sizeof(int)), hn(len.size() * sizeof(int));
+      std::memcpy(hf.data(), first.data(), hf.size());
+      std::memcpy(hn.data(), len.data(), hn.size());
+      margs[i].args = upload(args);
+      margs[i].first = reinterpret_cast<const int*>(upload(hf));
+      margs[i].n = reinterpret_cast<const int*>(upload(hn));
+      margs[i].nsolve = (int)first.size();
+      mblocks[i] = (unsigned)acc;
     }
     hipStream_t main = streams[(size_t)M[0]->stream];
     std::vector<hipStream_t> others;
@@ -280,17 +290,17 @@ struct vb_batch {
     hipGraph_t gr = nullptr;
     try {
       fork();
-      for (size_t k = 0; k < s0.size(); ++k) {
-        if (vb::zstage_multi_op(s0[k].op)) {
-          join();
-          vb::launch_zstage_multi(s0[k].op, margs[k], mblocks[k], main);
-          fork();
-        } else {
-          for (size_t m = 0; m < M.size(); ++m) {
-            const auto& x = rec[m][0].seq[k];
-            x.launch_tab(x.op, gtab[m][k], x.grid, x.block, (int)rec[m].size(), streams[(size_t)M[m]->stream]);
-          }
+      for (size_t i = 0; i <= nst; ++i) {
+        for (size_t m = 0; m < M.size(); ++m) {
+          const auto& sq = rec[m][0].seq;
+          for (size_t k = i ? pos[m][i - 1] + 1 : 0; k < (i < nst ? pos[m][i] : sq.size()); ++k)
+            sq[k].launch_tab(sq[k].op, gtab[m][k], sq[k].grid, sq[k].block, (int)rec[m].size(),
+                             streams[(size_t)M[m]->stream]);
         }
+        if (i == nst) break;
+        join();
+        vb::launch_zstage_multi(rec[0][0].seq[pos[0][i]].op, margs[i], mblocks[i], main);
+        fork();
       }
       join();
     } catch (...) {

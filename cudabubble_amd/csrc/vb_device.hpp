@@ -120,19 +120,67 @@ struct alignas(64) Coef {
 // moves the targets, alpha -= V - alpha0, beta -= A - beta0
 // (belastic.cpp:680-688), then computes the multipliers with them.
 enum { FIN_PLAIN = 0, FIN_DRIFT = 1 };
+// what else the finalize does in the penalty-drift double step: save the new
+// scalars (the state's, for the second evaluation), or put the saved ones back
+// under the targets just moved
+enum { FOLD_NONE = 0, FOLD_KEEP = 1, FOLD_RETARGET = 2 };
 
 __device__ __forceinline__ int fold(int k, int n) { return k < n - k ? k : n - k; }
 __device__ __forceinline__ int sgnk(int k, int n) { return k < n - k ? k : k - n; }
+
+// A double from another lane by a DPP control (two 32-bit moves in the VALU;
+// a shuffle would take two LDS permutes); lanes without a source, or outside
+// the row mask, get 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_get(double v) {
+  const unsigned long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(unsigned(b)), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(unsigned(b >> 32)), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((unsigned long long)unsigned(lo) | ((unsigned long long)unsigned(hi) << 32));
+}
+// K sums over a wave, the totals in every lane: prefix sums within each row of
+// 16 lanes, the rows' totals passed on to the last lane, which is broadcast.
+template <int K>
+__device__ __forceinline__ void wave_sum(double (&acc)[K]) {
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    double v = acc[q];
+    v += dpp_get<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8
+    v += dpp_get<0x112, 0xf>(v);
+    v += dpp_get<0x114, 0xf>(v);
+    v += dpp_get<0x118, 0xf>(v);
+    v += dpp_get<0x142, 0xa>(v);   // row_bcast:15 into rows 1, 3
+    v += dpp_get<0x143, 0xc>(v);   // row_bcast:31 into rows 2, 3
+    const unsigned long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane(int(unsigned(b)), 63);
+    const unsigned hi = __builtin_amdgcn_readlane(int(unsigned(b >> 32)), 63);
+    acc[q] = __longlong_as_double((unsigned long long)lo | ((unsigned long long)hi << 32));
+  }
+}
+
+// K sums over a workgroup of NT threads: wave_part stores each wave's sums to
+// red[K * (NT / 64)] before a barrier of the caller, wave_total adds them
+// after it (threads 0..K-1).
+template <int K, int NT>
+__device__ __forceinline__ void wave_part(double (&acc)[K], double* red) {
+  wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < K; ++q) red[q * (NT / 64) + (threadIdx.x >> 6)] = acc[q];
+  }
+}
+template <int NT>
+__device__ __forceinline__ double wave_total(const double* red, int q) {
+  double s = 0.0;
+  for (int i = 0; i < NT / 64; ++i) s += red[q * (NT / 64) + i];
+  return s;
+}
 
 // block-wide deterministic sum of K doubles; thread 0..K-1 write out[q].
 // Uses LDS scratch of K * (NT / 64) doubles (declared by the caller).
 template <int K, int NT>
 __device__ __forceinline__ void block_sum_store(double (&acc)[K], double* red, double* out) {
-#pragma unroll
-  for (int q = 0; q < K; ++q) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc[q] += __shfl_xor(acc[q], off, 64);
-  }
+  wave_sum(acc);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   if (l == 0) {
 #pragma unroll
@@ -174,8 +222,10 @@ struct FinArgs {
   const double* dc;   // k = 0 coefficient of the field (its mean)
   const double* dcpart;   // FP32-mixed: the x kernel's sums of tmp1 and eps^3 s (2 per block), or nullptr
   Scal* sc;
+  Scal* keep;         // see fold
   FinScratch* fs;
-  int nxb, nzb, mode, pad;
+  int nxb, nzb, mode;
+  int fold;           // FOLD_KEEP: also stored in *keep; FOLD_RETARGET: only the targets of *keep move
   Geo g;
   Phys ph;
 };
@@ -189,10 +239,24 @@ struct FinArgs {
 // and 473-479), and with dcpart the means of tmp1 and eps^3 s.  red holds
 // 6 * (NT / 64) doubles and tot 7 doubles of LDS.
 // UN accumulator sets per thread keep UN loads in flight (fewer registers in
-// kernels that carry this as a side branch).
-template <int NT, int UN = 4>
+// kernels that carry this as a side branch).  RT: FOLD_RETARGET may be asked for.
+template <int NT, int UN = 4, bool RT = false>
 __device__ __forceinline__ void finalize_body(const FinArgs& a, double* red, double* tot, int b, int nb) {
   static_assert(NT % 64 == 0, "whole waves");
+  // what the result needs of the old scalars (and, for a retarget, all of the
+  // kept ones), loaded beside the partials
+  double tg[4] = {}, dc0 = 0.0;
+  Scal k;
+  if (threadIdx.x == 0) {
+    tg[0] = a.sc->alpha;
+    tg[1] = a.sc->beta;
+    tg[2] = a.sc->alpha0;
+    tg[3] = a.sc->beta0;
+    dc0 = a.dc[0];
+    if constexpr (RT) {
+      if (a.fold == FOLD_RETARGET) k = *a.keep;
+    }
+  }
   const int xs = (a.nxb + nb - 1) / nb, zs = (a.nzb + nb - 1) / nb;
   const int x0 = b * xs, x1 = min(a.nxb, x0 + xs);
   const int z0 = b * zs, z1 = min(a.nzb, z0 + zs);
@@ -245,7 +309,6 @@ __device__ __forceinline__ void finalize_body(const FinArgs& a, double* red, dou
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    Scal c = *a.sc;
     const double N = double(a.g.nr);
     const double L3 = a.g.L3;
     const double eps = a.ph.eps;
@@ -253,14 +316,19 @@ __device__ __forceinline__ void finalize_body(const FinArgs& a, double* red, dou
     // s = eps/2 |grad d|^2 + (d^2-1)^2/(4 eps); elastic: intf(f^2, 0, 1/(2 eps)).
     // mean(d) is the k = 0 coefficient of the FP64 spectrum (Parseval gives
     // mean |grad d|^2 the same way); the spatial sum is kept as sum_v.
-    const double V = (a.dc[0] + 1.0) * (0.5 * L3);
+    const double V = (dc0 + 1.0) * (0.5 * L3);
     const double ms = 0.5 * eps * tot[3] + 0.25 / eps * (tot[1] / N);
     const double A = ms * (3.0 / (2.0 * sqrt(2.0)) * L3);
     const double Eb = (tot[2] / N) * (1.0 / (eps * 2) * L3);
     if (a.mode == FIN_DRIFT) {
-      c.alpha -= (V - c.alpha0);
-      c.beta -= (A - c.beta0);
+      tg[0] -= (V - tg[2]);
+      tg[1] -= (A - tg[3]);
     }
+    Scal c;
+    c.alpha = tg[0];
+    c.beta = tg[1];
+    c.alpha0 = tg[2];
+    c.beta0 = tg[3];
     c.V = V;
     c.A = A;
     c.Eb = Eb;
@@ -271,10 +339,24 @@ __device__ __forceinline__ void finalize_body(const FinArgs& a, double* red, dou
     if (a.dcpart) {
       c.dc_t1 = tot[4] / N;
       c.dc_s = tot[5] / N;
+    } else {
+      c.dc_t1 = a.sc->dc_t1;
+      c.dc_s = a.sc->dc_s;
     }
+    c.pad = 0;
     c.nonfinite = !(isfinite(V) && isfinite(A) && isfinite(Eb)) ? 1 : 0;
     apply_targets(c, a.ph);
-    *a.sc = c;
+    if (RT && a.fold == FOLD_RETARGET) {
+      k.alpha = c.alpha;
+      k.beta = c.beta;
+      k.alpha0 = c.alpha0;
+      k.beta0 = c.beta0;
+      apply_targets(k, a.ph);
+      *a.sc = k;
+    } else {
+      *a.sc = c;
+      if (a.fold == FOLD_KEEP) *a.keep = c;
+    }
   }
 }
 

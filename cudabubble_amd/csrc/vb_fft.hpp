@@ -71,6 +71,8 @@ template <> struct Plan<256, 1> { static constexpr int E = 16, NP = 2; static co
 template <> struct Plan<128, 1> { static constexpr int E = 16, NP = 2; static constexpr int R[2] = {16, 8}; };
 template <> struct Plan<512, 1> { static constexpr int E = 16, NP = 3; static constexpr int R[3] = {16, 8, 4}; };
 template <> struct Plan<192, 1> { static constexpr int E = 24, NP = 2; static constexpr int R[2] = {24, 8}; };
+template <> struct Plan<48, 3>  { static constexpr int E = 12, NP = 2; static constexpr int R[2] = {12, 4}; };
+template <> struct Plan<96, 3>  { static constexpr int E = 12, NP = 3; static constexpr int R[3] = {12, 4, 2}; };
 template <> struct Plan<192, 3> { static constexpr int E = 12, NP = 3; static constexpr int R[3] = {12, 4, 4}; };
 
 template <int N, int V = 0> constexpr int TFof() { return N / Plan<N, V>::E; }
@@ -298,10 +300,10 @@ struct Pass {
 #pragma unroll
       for (int e = 0; e < E; ++e) x[e] = y[e];
     } else {
-      __syncthreads();
+      lds.sync();
 #pragma unroll
       for (int e = 0; e < E; ++e) x[e] = lds(j + TF * e);
-      __syncthreads();
+      lds.sync();
       Pass<T, N, S, P + 1, V>::run(x, j, tw, lds);
     }
   }
@@ -327,21 +329,22 @@ struct Pass2 {
         x1[e] = y1[e];
       }
     } else {
-      __syncthreads();
+      l0.sync();
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         x0[e] = l0(j + TF * e);
         x1[e] = l1(j + TF * e);
       }
-      __syncthreads();
+      l0.sync();
       Pass2<T, N, S, P + 1, V>::run(x0, x1, j, tw, l0, l1);
     }
   }
 };
 
 // Full 1-D transform (unnormalised): S = -1 forward, +1 inverse.
-// Contains (NP - 1) * 2 workgroup barriers; every thread of the workgroup
-// must call it the same number of times.
+// Contains (NP - 1) * 2 barriers of the view's scope (Lds::sync): with a
+// workgroup view every thread of the workgroup must call it the same number of
+// times, with a wave view every lane of the wave.
 template <typename T, int N, int S, int V = 0, class Lds>
 __device__ __forceinline__ void fft(cpx<T>* x, int j, const cpx<T>* __restrict__ tw, Lds& lds) {
   Pass<T, N, S, 0, V>::run(x, j, tw, lds);
@@ -360,15 +363,45 @@ template <typename T>
 struct RowLds {
   cpx<T>* base;
   __device__ __forceinline__ cpx<T>& operator()(int pos) const { return base[pos + (pos >> 3)]; }
+  __device__ __forceinline__ void sync() const { __syncthreads(); }
 };
 template <int N> constexpr int row_lds_len() { return N + N / 8; }
 
+// Order of one wave's LDS accesses: a wave's LDS instructions execute in
+// order, so its lanes exchange data without a workgroup barrier as long as the
+// compiler keeps that order.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // LDS view for column tiles (y and z kernels): TB interleaved transforms,
-// column index fastest.
-template <typename T, int TB>
+// column index fastest.  WAVE: the tile's lanes are one wave.
+template <typename T, int TB, bool WAVE = false>
 struct ColLds {
   cpx<T>* base;  // already offset by the column index
   __device__ __forceinline__ cpx<T>& operator()(int pos) const { return base[pos * TB]; }
+  __device__ __forceinline__ void sync() const {
+    if constexpr (WAVE) wave_sync();
+    else __syncthreads();
+  }
+};
+
+// Views of a plane of rows held in LDS (vb_plane.hpp), each transform carried
+// by lanes of one wave: a row (one pad slot every 2^PS entries), and a column
+// (one slot of every row, LL apart).
+template <typename T, int PS>
+struct PlaneRow {
+  cpx<T>* base;
+  __device__ __forceinline__ cpx<T>& operator()(int pos) const { return base[pos + (pos >> PS)]; }
+  __device__ __forceinline__ void sync() const { wave_sync(); }
+};
+template <typename T, int LL>
+struct PlaneCol {
+  cpx<T>* base;
+  __device__ __forceinline__ cpx<T>& operator()(int pos) const { return base[pos * LL]; }
+  __device__ __forceinline__ void sync() const { wave_sync(); }
 };
 
 }  // namespace vb

@@ -80,8 +80,7 @@ hipStream_t make_queue_stream();
 // finalize kernel's launcher (vb_solver.hip)
 FinArgs fin_args(const double* xpart, int nxb, const double* zpart, const double* dc, int nzb, Scal* sc,
                  FinScratch* fs, const Geo& g, const Phys& ph, int mode);
-void launch_finalize(const double* xpart, int nxb, const double* zpart, const double* dc, int nzb, Scal* sc,
-                     const Geo& g, const Phys& ph, int mode, hipStream_t s);
+void launch_finalize(const FinArgs& a, hipStream_t s);
 void launch_fill_scal(Scal* sc, double alpha, double beta, double alpha0, double beta0, hipStream_t s);
 
 // device-side accept of adaptive attempts (vb_chain.hip): the control kernels

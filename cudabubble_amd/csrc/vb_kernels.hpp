@@ -20,8 +20,26 @@
 #include <type_traits>
 
 #include "vb_device.hpp"
+#ifndef VB_XREV
+#define VB_XREV true
+#endif
 
 namespace vb {
+
+// Workgroups go to the chip's XCDs in turn (workgroup b to XCD b mod 8), and
+// each XCD has its own L2: lines that an XCD wrote are read back by the same
+// XCD in the next kernel at L2 speed, by another one far slower (16 MB rewritten
+// in place by the next kernel: 5.2 us on the same XCD, 12.5 us shifted by one),
+// and a line that two XCDs write in parts is worse still.  So the prefix kernels
+// give plane z to XCD (z / 2) mod 8 in all of them, and the column groups that
+// share 128-byte lines (two planes of a group-major spectrum, two 8-column tiles
+// of a row) run on one XCD.
+constexpr int kXcds = 8;
+// item of workgroup b (of n) when items 2i and 2i + 1 are to share an XCD; a
+// permutation of [0, n), the identity past the last whole sixteen
+__device__ __forceinline__ int pair_item(int b, int n) {
+  return b < (n & ~15) ? (b & ~15) | ((b & 7) << 1) | ((b >> 3) & 1) : b;
+}
 
 constexpr int XWG = 64;   // threads per x-kernel workgroup: one wave (measured best at 256^3: 64 < 128 < 256)
 
@@ -45,27 +63,31 @@ template <typename T, int N> constexpr int colplan() {
 // Column tile width of the y passes and the z Laplacian (columns that are
 // contiguous in memory): enough columns for >= 128-byte segments and >= 256
 // threads, except FP32 at 64, 16 columns (128 threads): a 64^3 solve's y pass
-// is then 1056 workgroups instead of 528 (9.6 -> 7.7 us, a step 0.236 -> 0.209
-// ms; 32 columns at 32 changed nothing).
+// is then 1056 workgroups instead of 528 (9.6 -> 7.7 us), and 16 at 96, which
+// divides its 48 columns (aligned rows).
 template <typename T, int N> constexpr int colw() {
-  if (sizeof(T) == 4 && N == 64) return 16;
+  if ((sizeof(T) == 4 && N == 64) || N == 96) return 16;
   constexpr int seg = 128 / int(sizeof(cpx<T>));
   constexpr int occ = 256 / TFof<N>();
   return seg > occ ? seg : occ;
 }
 
 // Column tile of the z stage kernels (stage combines, z-prep, plain z
-// passes): the column width, except FP32 at 256 and 512, 8 columns.  At 256
-// (256-thread workgroups, two or three per CU) 8 measured 6-14 % faster per
-// stage than 16: their inputs are group-major, so only their P, Q outputs are
-// written in 64-byte pieces.  At 512, 16 columns make 1024-thread workgroups,
-// whose 128-register budget spilled 160-412 bytes per lane in the stage
-// combines; 8 took the combines from 1410-2358 to 1118-1440 us (the forward y
-// pass, which writes the 8-column groups, from 483 to 590 us) and a step from
-// 25.7 to 23.2 ms.  FP32 at 64 keeps 32 (256 threads, the shared stage
-// launches' workgroup), though its y passes use 16 columns.
+// passes).  Up to 96, one wave's columns, so that the combines need no
+// workgroup barrier and a short grid spreads over more CUs (a 32^3 FP64 combine
+// was 9 workgroups of 256 threads): with the combine's operands and
+// coefficients loaded before its transforms (EARLY), 9.4 -> 6.4 us at 32^3 FP64
+// and 10.5 -> 8.6 us (stage 1 9.6 -> 6.4) at 64^3 FP32.  Above, the column
+// width, except FP32 at 256 and 512, 8 columns.  At 256 (256-thread workgroups,
+// two or three per CU) 8 measured 6-14 % faster per stage than 16: their inputs
+// are group-major, so only their P, Q outputs are written in 64-byte pieces.  At
+// 512, 16 columns make 1024-thread workgroups, whose 128-register budget
+// spilled 160-412 bytes per lane in the stage combines; 8 took the combines
+// from 1410-2358 to 1118-1440 us (the forward y pass, which writes the
+// 8-column groups, from 483 to 590 us) and a step from 25.7 to 23.2 ms.
 template <typename T, int N> constexpr int tbw() {
-  return (sizeof(T) == 4 && (N == 256 || N == 512)) ? 8 : (sizeof(T) == 4 && N == 64) ? 32 : colw<T, N>();
+  if (N <= 96) return 64 / TFof<N>();
+  return (sizeof(T) == 4 && (N == 256 || N == 512)) ? 8 : colw<T, N>();
 }
 // The other z tile a kernel schedule can select: the column width where tbw
 // is narrower, else half of it.
@@ -101,6 +123,17 @@ struct Rows {
     return (long long)q * pp + (nq >= 0 ? nq + m : (long long)m * pitch + half);
   }
 };
+
+// Row group of this workgroup of an x kernel with RL rows per workgroup, in the
+// solver's row layout: planes on their XCDs (see kXcds), last ones first, so
+// that the planes the y pass wrote last, still in L2, are read first.
+template <int RL>
+__device__ __forceinline__ unsigned xgroup(const Rows& rl, long long nrows) {
+  const unsigned ny = unsigned(rl.ny), nz = unsigned(nrows) / ny, b = blockIdx.x;
+  if (rl.nq < 0 || ny % RL || nz % (2 * kXcds)) return b;
+  const unsigned w = ny / RL, q = gridDim.x / kXcds - 1 - b / kXcds, q2 = q % (2 * w);
+  return (((q / (2 * w)) * kXcds + b % kXcds) * 2 + q2 % 2) * w + q2 / 2;
+}
 
 // After a forward transform of Z = a + i b (a, b real rows), write the half
 // spectra of a and b, times s (and b's times sb as well); SCALE = false writes
@@ -393,7 +426,7 @@ __global__ void __launch_bounds__((xrthreads<T, N, XP>()), (xrwaves<T, N>())) k_
   const int lane = threadIdx.x / TF, j = threadIdx.x % TF;
   RowLds<T> lds{sm + lane * LL};
   const long long nrows = 2 * a.npairs;
-  long long row = (long long)blockIdx.x * RL + lane;
+  long long row = (long long)xgroup<RL>(a.rl, nrows) * RL + lane;
   const bool valid = row < nrows;
   if (!valid) row = nrows - 1;
   const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps;
@@ -599,10 +632,12 @@ __device__ __forceinline__ YIdx yidx(const Geo& g, long long t) {
     // the Nyquist groups (uncoalesced, slower) come first so they overlap
     // with the main groups instead of trailing them
     const int tpr = (g.nx / 2) / TB;
-    const long long nnyq = (g.nz + TB - 1) / TB;
+    const int nnyq = (g.nz + TB - 1) / TB;
     if (t >= nnyq) {
-      z = int((t - nnyq) / tpr);
-      kx = int((t - nnyq) % tpr) * TB + c;
+      // two planes at a time per XCD, their tiles alternating
+      const unsigned i = unsigned(t - nnyq), q = i / kXcds, t2 = 2 * unsigned(tpr), q2 = q % t2;
+      z = int(((q / t2) * kXcds + i % kXcds) * 2 + q2 % 2);
+      kx = int(q2 / 2) * TB + c;
       r.valid = true;
     } else {   // Nyquist column of TB planes
       z = int(t * TB + c);
@@ -638,6 +673,7 @@ struct YArgs {
   Geo g;
   FinArgs fin;  // workgroups [0, fin_on) of blockIdx.y = 0 evaluate these integrals
   int fin_on;
+  int pad;
   cpx<T>* o0;   // GM: out-of-place outputs in the z kernels' group-major layout
   cpx<T>* o1;
   int ztb;      // GM: the z kernels' column tile
@@ -689,7 +725,8 @@ __global__ void __launch_bounds__((TB * TFof<N, V>())) k_ypass(YArgs<T> a0, cons
   cpx<T>* buf = blockIdx.y ? a.b1 : a.b0;
   const int j = threadIdx.x / TB;
   ColLds<T, TB> lds{sm + threadIdx.x % TB};
-  const YIdx id = yidx<TB>(g, (long long)blockIdx.x - a.fin_on);
+  const YIdx id = yidx<TB>(g, (long long)blockIdx.x - a.fin_on - a.pad);
+  if ((int)blockIdx.x < a.fin_on + a.pad) return;
   cpx<T>* col = buf + id.base;
   cpx<T> x[E];
 #pragma unroll
@@ -886,6 +923,7 @@ template <typename T, int N, int TB, int V, bool PONLY = false, class Lds>
 __device__ __forceinline__ void next_field_tail(cpx<T>* x, cpx<T>* y, double acc, int j, const ZIdx& id,
                                                 const Geo& g, Lds& lds, Lds& lds2, const cpx<T>* __restrict__ tw,
                                                 cpx<T>* P, cpx<T>* Q, double* part, double* red, int tile) {
+  constexpr bool WAVE = TB * TFof<N, V>() == 64;
   constexpr int E = Plan<N, V>::E, TF = N / E;
   const long long plane = g.pp;
   if constexpr (PONLY)
@@ -900,7 +938,12 @@ __device__ __forceinline__ void next_field_tail(cpx<T>* x, cpx<T>* y, double acc
     }
   }
   double s[1] = {acc};
-  block_sum_store<1, TB * TF>(s, red, part + tile);
+  if constexpr (WAVE) {
+    wave_sum(s);
+    if ((threadIdx.x & 63) == 0) part[tile] = s[0];
+  } else {
+    block_sum_store<1, TB * TF>(s, red, part + tile);
+  }
 }
 
 template <typename T>
@@ -924,11 +967,13 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zprep(ZprArgs<T> a0, const
   __shared__ cpx<T> sm[2 * N * TB];
   __shared__ double red[(TB * TF) / 64];
   const int j = threadIdx.x / TB;
-  ColLds<T, TB> lds{sm + threadIdx.x % TB};
-  ColLds<T, TB> lds2{sm + N * TB + threadIdx.x % TB};
-  const ZIdx id = zidx<TB>(g);
+  constexpr bool WAVE = TB * TF == 64;
+  ColLds<T, TB, WAVE> lds{sm + threadIdx.x % TB};
+  ColLds<T, TB, WAVE> lds2{sm + N * TB + threadIdx.x % TB};
+  const int tile = pair_item(int(blockIdx.x), int(gridDim.x));
+  const ZIdx id = zidx<TB>(g, tile);
   // the state spectrum is group-major (see k_zstage)
-  const long long ib0 = (long long)blockIdx.x * N * TB + threadIdx.x % TB;
+  const long long ib0 = (long long)tile * N * TB + threadIdx.x % TB;
   cpx<double> u[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) u[e] = id.valid ? vh[ib0 + (long long)(j + TF * e) * TB] : mk<double>(0.0, 0.0);
@@ -937,7 +982,7 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zprep(ZprArgs<T> a0, const
   double acc = 0.0;
 #pragma unroll
   for (int e = 0; e < E; ++e) next_field_elem<T>(u[e].x, u[e].y, j + TF * e, id, g, acc, x[e], y[e]);
-  next_field_tail<T, N, TB, 0>(x, y, acc, j, id, g, lds, lds2, tw, a.P, a.Q, a.part, red, int(blockIdx.x));
+  next_field_tail<T, N, TB, 0>(x, y, acc, j, id, g, lds, lds2, tw, a.P, a.Q, a.part, red, tile);
 }
 
 template <typename T>
@@ -961,6 +1006,16 @@ struct ZsArgs {
   const double4* c2;      // per m: ETDRK4 {e2, A s, 2 B s, C s}; ETDRK2 {c2, 0, 0, 0}
   const cpx<T>* tw;
   Geo g;
+  // The stage field's integrals, where no other kernel evaluated them (nxb >
+  // 0): the partial sums of k_plane (xpart, dcpart: nxb sets) and of the kernel
+  // that prepared the field (zin: nzb, dcin), from which each workgroup forms
+  // lambda1 and lambda2 under the targets of sc, with penalties M1, M2.
+  const double* xpart;
+  const double* dcpart;
+  const double* zin;
+  const double* dcin;
+  int nxb, nzb;
+  double M1, M2;
 };
 
 // SCH = 4 (ETDRK4, belastic.cpp:519-552 / Calc.cu:488-577) or 2 (ETDRK2,
@@ -993,7 +1048,7 @@ template <typename T, int N> constexpr int zsplan() { return (sizeof(T) == 4 && 
 template <typename T, int N, int SCH, int STG, int TB, int V>
 constexpr int zs_lds_bytes() {
   return (2 * N * TB * int(sizeof(cpx<T>))) >
-                 ((SCH == 4 && STG != 2) ? TB * (N / 2 + 1) * int(STG == 4 ? sizeof(double4) : sizeof(double2)) : 0)
+                 ((SCH == 4 && STG != 2 && !(TB * TFof<N, V>() == 64 && Plan<N, V>::E <= 8)) ? TB * (N / 2 + 1) * int(STG == 4 ? sizeof(double4) : sizeof(double2)) : 0)
              ? 2 * N * TB * int(sizeof(cpx<T>))
              : TB * (N / 2 + 1) * int(STG == 4 ? sizeof(double4) : sizeof(double2));
 }
@@ -1002,9 +1057,16 @@ constexpr int zs_lds_bytes() {
 // workgroup's LDS passed in (smraw: zs_lds_bytes, red: (TB * TF) / 64
 // doubles), so that a launch can run the groups of solves of several sizes.
 template <typename T, int N, int SCH, int STG, int TB, int V, bool PROBE>
-__device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsigned char* smraw, double* red) {
+__device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, int tid, unsigned char* smraw, double* red,
+                                            double* fred) {
   static_assert(!PROBE || (SCH == 4 && STG == 4), "the probe form is the last ETDRK4 stage");
   constexpr int E = Plan<N, V>::E, TF = N / E;
+  constexpr bool WAVE = TB * TF == 64;   // the tile is one wave's (the workgroup may run several)
+  // A wave tile has the registers for all its operands at once (up to 290 in
+  // FP64): loaded before the transforms, with the coefficients per element,
+  // they cost one memory latency instead of three in a row.  Not at 48 and 96,
+  // whose 12 elements per thread would need over 400.
+  constexpr bool EARLY = WAVE && E <= 8;
   // ETDRK4 stages 1, 3 and 4 read their coefficient records from a
   // per-workgroup table in LDS: TB columns x (N/2 + 1) folded kz, gathered once
   // after the forward transforms.  Gathered per element, the 64 lanes of a load
@@ -1012,19 +1074,19 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
   // requests of their streams; staged, stages 1, 3, 4 and the probe ran 120,
   // 123, 161, 126 -> 112, 107, 148, 122 us at 256^3 FP32.  Stage 2 keeps the
   // gathers: the table cost it a wave per SIMD and time.
-  constexpr bool STAGED = SCH == 4 && STG != 2;
+  constexpr bool STAGED = SCH == 4 && STG != 2 && !EARLY;
   using Rec = typename std::conditional<STG == 4, double4, double2>::type;
   constexpr int NQ = N / 2 + 1;
   cpx<T>* sm = reinterpret_cast<cpx<T>*>(smraw);
-  const int j = threadIdx.x / TB;
-  ColLds<T, TB> lds{sm + threadIdx.x % TB};
-  ColLds<T, TB> lds2{sm + N * TB + threadIdx.x % TB};
+  const int j = tid / TB;
+  ColLds<T, TB, WAVE> lds{sm + tid % TB};
+  ColLds<T, TB, WAVE> lds2{sm + N * TB + tid % TB};
   const Geo g = a.g;
-  const ZIdx id = zidx<TB>(g, tile);
+  const ZIdx id = zidx<TB>(g, tile, tid % TB);
   // The state and U, U2, pre, Na, Nb, Vh are kept group-major: this
   // workgroup's TB columns of all N planes are one contiguous run (see
   // zs_private); the strided z traffic of a stage is only P, Q
-  const long long ib0 = (long long)tile * N * TB + threadIdx.x % TB;
+  const long long ib0 = (long long)tile * N * TB + tid % TB;
   // (lanes past the last column of a Nyquist group have no input written;
   // they transform zeros and store nothing)
   cpx<T> x[E], x2[E];
@@ -1040,9 +1102,84 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
   // spectra of tmp1 and s are dead before the combine's operands load:
   // N^ = Np + Av v^ with Av = -lambda2 3/(2 sqrt 2) (eps |k|^2 + kappa/eps).
   // Np stays FP64: near an equilibrium f^ is small and its two parts cancel.
+  constexpr bool USES_U = !(SCH == 4 && STG == 3);
+  // The operands of the combine (EH elements at a time, see below)
+  constexpr int NH = (!EARLY && (sizeof(T) == 8 || E >= 12 || PROBE) && STG == SCH) ? 2 : 1, EH = E / NH;
+  constexpr bool C1 = SCH == 2 || STG != 4, C2 = STG == SCH;
+  cpx<double> ur[USES_U ? EH : 1];
+  cpx<T> pa[(SCH == 4 && STG >= 3) || (SCH == 2 && STG == 2) ? EH : 1];
+  cpx<T> pb[(SCH == 4 && STG == 4) ? EH : 1];
+  cpx<T> pv[STG > 1 ? EH : 1];
+  double2 k1[EARLY && C1 ? E : 1];
+  double4 k2[EARLY && C2 ? E : 1];
+  auto load = [&](int hh) {
+#pragma unroll
+    for (int iq = 0; iq < EH; ++iq) {
+      const int e = hh * EH + iq;
+      const long long ib = ib0 + (long long)(j + TF * e) * TB;
+      if constexpr (USES_U) ur[iq] = id.valid ? ld_nt(a.uh + ib) : mk<double>(0.0, 0.0);
+      if constexpr (SCH == 4 && STG == 3) pa[iq] = ld_nt(a.pre + ib);
+      if constexpr (SCH == 4 && STG == 4) { pa[iq] = ld_nt(a.Na + ib); pb[iq] = ld_nt(a.Nb + ib); }
+      if constexpr (SCH == 2 && STG == 2) pa[iq] = ld_nt(a.Na + ib);
+      if constexpr (STG > 1) pv[iq] = ld_nt(a.Vh + ib);
+    }
+  };
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int m = mindex(g, id.kx, id.ky, j + TF * e);
+      if constexpr (C1) k1[e] = a.c1[m];
+      if constexpr (C2) k2[e] = a.c2[m];
+    }
+    load(0);
+  }
+  constexpr int NTZ = TB * TF, KF = sizeof(T) == 4 ? 4 : 2;
+  double ftot[KF] = {};
+  if (a.nxb > 0) {
+    double fs[KF] = {};
+    for (int i = tid; i < a.nxb; i += NTZ) {
+      fs[0] += a.xpart[3 * i + 1];
+      if constexpr (KF == 4) {
+        fs[2] += a.dcpart[2 * i];
+        fs[3] += a.dcpart[2 * i + 1];
+      }
+    }
+    for (int i = tid; i < a.nzb; i += NTZ) fs[1] += a.zin[i];
+    if constexpr (WAVE) {
+      wave_sum(fs);
+#pragma unroll
+      for (int q = 0; q < KF; ++q) ftot[q] = fs[q];
+    } else {
+      wave_part<KF, NTZ>(fs, fred);   // read after the transforms' barriers
+    }
+  }
   fft2<T, N, -1, V>(x, x2, j, a.tw, lds, lds2);   // spectra of tmp1 and eps^3 s (stored units)
-  const double l1h = 0.5 * a.sc->l1;
-  const double l2c = a.sc->l2 * (3.0 / (2.0 * sqrt(2.0)));
+  double lam1, lam2, dct1 = 0.0, dcs = 0.0;
+  if (a.nxb > 0) {
+    if constexpr (!WAVE) {
+#pragma unroll
+      for (int q = 0; q < KF; ++q) ftot[q] = wave_total<NTZ>(fred, q);
+    }
+    // as finalize_body
+    const double V0 = (a.dcin[0] + 1.0) * (0.5 * g.L3);
+    const double ms = 0.5 * a.eps * ftot[1] + 0.25 / a.eps * (ftot[0] / double(g.nr));
+    const double A0 = ms * (3.0 / (2.0 * sqrt(2.0)) * g.L3);
+    lam1 = a.M1 * (V0 - a.sc->alpha);
+    lam2 = a.M2 * (A0 - a.sc->beta);
+    if constexpr (KF == 4) {
+      dct1 = ftot[2] / double(g.nr);
+      dcs = ftot[3] / double(g.nr);
+    }
+  } else {
+    lam1 = a.sc->l1;
+    lam2 = a.sc->l2;
+    if constexpr (KF == 4) {
+      dct1 = a.sc->dc_t1;
+      dcs = a.sc->dc_s;
+    }
+  }
+  const double l1h = 0.5 * lam1;
+  const double l2c = lam2 * (3.0 / (2.0 * sqrt(2.0)));
   const double ie = 1.0 / a.eps;
   // the x kernel stores 2 N F(tmp1) and 2 N F(eps^3 s) (F normalised): hu and
   // hs turn them into F(tmp1) and F(s)
@@ -1059,8 +1196,8 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
       // the k = 0 coefficients summed in FP64 by the x kernel (k_xrow), the
       // means of tmp1 and eps^3 s, in stored units
       if (e == 0 && id.q == 0 && j == 0) {
-        tr = a.sc->dc_t1 / hu;
-        sr = a.sc->dc_s / hu;
+        tr = dct1 / hu;
+        sr = dcs / hu;
       }
     }
     double pr = at * tr - etas * sr;
@@ -1068,20 +1205,29 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
     if (id.q == 0 && kz == 0) pr -= l1h;
     np[e] = mk<double>(pr, pi);
   }
-  const Rec* tbl = reinterpret_cast<const Rec*>(smraw);
+  [[maybe_unused]] const Rec* tbl = reinterpret_cast<const Rec*>(smraw);
   if constexpr (STAGED) {
     // the transforms' last LDS reads are behind their last barrier
     Rec* w = reinterpret_cast<Rec*>(smraw);
-    for (int i = threadIdx.x; i < TB * NQ; i += TB * TF) {
+    for (int i = tid; i < TB * NQ; i += TB * TF) {
       const int c = i / NQ, q = i % NQ;
       const ZIdx ic = zidx<TB>(g, tile, c);
       const int m = mindex(g, ic.kx, ic.ky, q);
       if constexpr (STG == 4) w[i] = a.c2[m]; else w[i] = a.c1[m];
     }
-    __syncthreads();
+    lds.sync();
   }
-  const int tcol = int(threadIdx.x % TB);
-  constexpr bool USES_U = !(SCH == 4 && STG == 3);
+  const int tcol = int(tid % TB);
+  auto coef1 = [&](int e, int kz, int m) -> double2 {
+    if constexpr (EARLY) return k1[C1 ? e : 0];
+    else if constexpr (STAGED && STG != 4) return tbl[tcol * NQ + (kz <= N / 2 ? kz : N - kz)];
+    else return a.c1[m];
+  };
+  auto coef2 = [&](int e, int kz, int m) -> double4 {
+    if constexpr (EARLY) return k2[C2 ? e : 0];
+    else if constexpr (STAGED && STG == 4) return tbl[tcol * NQ + (kz <= N / 2 ? kz : N - kz)];
+    else return a.c2[m];
+  };
   // The last stage loads and combines its operands in two halves in FP64, and
   // in FP32 with 12 elements per thread (192, 384): all at once they need 256
   // registers and more in AGPRs, one wave per SIMD; in halves two (4 x 192^3
@@ -1089,25 +1235,11 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
   // 256 (198 -> 166 registers, two waves per SIMD -> three, 121 -> 118 us);
   // the full FP32 stage 4 stays at two waves either way and ran slower split
   // (149 -> 154 us).
-  constexpr int NH = ((sizeof(T) == 8 || E >= 12 || PROBE) && STG == SCH) ? 2 : 1, EH = E / NH;
   cpx<T> y[E];
   double acc = 0.0, dc0 = 0.0;
 #pragma unroll
   for (int hh = 0; hh < NH; ++hh) {
-    cpx<double> ur[USES_U ? EH : 1];
-    cpx<T> pa[(SCH == 4 && STG >= 3) || (SCH == 2 && STG == 2) ? EH : 1];
-    cpx<T> pb[(SCH == 4 && STG == 4) ? EH : 1];
-    cpx<T> pv[STG > 1 ? EH : 1];
-#pragma unroll
-    for (int iq = 0; iq < EH; ++iq) {
-      const int e = hh * EH + iq;
-      const long long ib = ib0 + (long long)(j + TF * e) * TB;
-      if constexpr (USES_U) ur[iq] = id.valid ? ld_nt(a.uh + ib) : mk<double>(0.0, 0.0);
-      if constexpr (SCH == 4 && STG == 3) pa[iq] = ld_nt(a.pre + ib);
-      if constexpr (SCH == 4 && STG == 4) { pa[iq] = ld_nt(a.Na + ib); pb[iq] = ld_nt(a.Nb + ib); }
-      if constexpr (SCH == 2 && STG == 2) pa[iq] = ld_nt(a.Na + ib);
-      if constexpr (STG > 1) pv[iq] = ld_nt(a.Vh + ib);
-    }
+    if constexpr (!EARLY) load(hh);
 #pragma unroll
     for (int iq = 0; iq < EH; ++iq) {
       const int e = hh * EH + iq;
@@ -1127,25 +1259,25 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
       x[e] = mk<T>(T(nr), T(ni));
       double fr, fi;   // next field
       if constexpr (SCH == 4 && STG == 1) {
-        const double2 c = STAGED ? tbl[tcol * NQ + (kz <= N / 2 ? kz : N - kz)] : a.c1[m];   // e1, q
+        const double2 c = coef1(e, kz, m);              // e1, q
         const cpx<double> u = ur[iq];
         fr = c.x * u.x + c.y * nr;                      // etd41: a^
         fi = c.x * u.y + c.y * ni;
         if (id.valid) st_nt(a.pre + ib, mk<T>(T(c.x * fr - c.y * nr), T(c.x * fi - c.y * ni)));
       } else if constexpr (SCH == 4 && STG == 2) {
-        const double2 c = STAGED ? tbl[tcol * NQ + (kz <= N / 2 ? kz : N - kz)] : a.c1[m];
+        const double2 c = coef1(e, kz, m);
         const cpx<double> u = ur[iq];
         fr = c.x * u.x + c.y * nr;                      // etd42: b^
         fi = c.x * u.y + c.y * ni;
         if (id.valid) st_nt(a.Na + ib, x[e]);
       } else if constexpr (SCH == 4 && STG == 3) {
-        const double q = STAGED ? tbl[tcol * NQ + (kz <= N / 2 ? kz : N - kz)].y : a.c1[m].y;
+        const double q = coef1(e, kz, m).y;
         const cpx<T> p = pa[iq];
         fr = double(p.x) + 2.0 * q * nr;                // etd43: c^ = e1 F(a) + q (2 N^b - N^u)
         fi = double(p.y) + 2.0 * q * ni;
         if (id.valid) st_nt(a.Nb + ib, x[e]);
       } else if constexpr (SCH == 4 && STG == 4) {
-        const double4 c = STAGED ? tbl[tcol * NQ + (kz <= N / 2 ? kz : N - kz)] : a.c2[m];   // e2, A s, 2 B s, C s
+        const double4 c = coef2(e, kz, m);              // e2, A s, 2 B s, C s
         const cpx<double> u = ur[iq];
         const cpx<T> na = pa[iq], nb = pb[iq];
         // etd44: e2 u^ + [N^a A + 2 (N^a + N^b) B + N^c C] s  (first term N^a as in Calc.cu:559)
@@ -1153,14 +1285,14 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
         fi = c.x * u.y + (double(na.y) * c.y + (double(na.y) + double(nb.y)) * c.z + ni * c.w);
         if (id.valid && !PROBE) st_nt(a.uout + ib, mk<double>(fr, fi));
       } else if constexpr (SCH == 2 && STG == 1) {
-        const double2 c = a.c1[m];                      // e^z, q1
+        const double2 c = coef1(e, kz, m);              // e^z, q1
         const cpx<double> u = ur[iq];
         fr = c.x * u.x + c.y * nr;                      // etd1: a^
         fi = c.x * u.y + c.y * ni;
         if (id.valid) st_nt(a.Na + ib, x[e]);
       } else {                                          // SCH == 2 && STG == 2
-        const double2 c = a.c1[m];
-        const double c2 = a.c2[m].x;
+        const double2 c = coef1(e, kz, m);
+        const double c2 = coef2(e, kz, m).x;
         const cpx<double> u = ur[iq];
         const cpx<T> nu = pa[iq];
         // etd2: u^+ = F(a) + c2 (N^a - N^u), a^ = e^z u^ + q1 N^u
@@ -1177,7 +1309,7 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, unsign
     }
   }
   if (id.valid && id.q == 0 && j == 0) a.dc[0] = dc0;
-  if constexpr (STAGED) __syncthreads();   // the table's last reads before the transforms reuse LDS
+  if constexpr (STAGED) lds.sync();   // the table's last reads before the transforms reuse LDS
   next_field_tail<T, N, TB, V, PROBE>(x, y, acc, j, id, g, lds, lds2, a.tw, a.P, a.Q, a.part, red, tile);
 }
 
@@ -1187,7 +1319,9 @@ __global__ void __launch_bounds__((TB * TFof<N, V>())) k_zstage(ZsArgs<T> a0, co
   const ZsArgs<T> a = TAB ? tab[blockIdx.z] : a0;
   __shared__ __align__(16) unsigned char smraw[zs_lds_bytes<T, N, SCH, STG, TB, V>()];
   __shared__ double red[(TB * TFof<N, V>()) / 64];
-  zstage_body<T, N, SCH, STG, TB, V, PROBE>(a, int(blockIdx.x), smraw, red);
+  __shared__ double fred[4 * ((TB * TFof<N, V>()) / 64)];
+  zstage_body<T, N, SCH, STG, TB, V, PROBE>(a, pair_item(int(blockIdx.x), int(gridDim.x)), int(threadIdx.x), smraw,
+                                                red, fred);
 }
 
 // Copy of a half spectrum between layouts, widened to FP64: tb_in / tb_out =

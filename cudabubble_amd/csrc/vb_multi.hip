@@ -2,10 +2,10 @@
 // one launch (the batched form's shared stage launches).
 //
 // Workgroup b of a launch runs column group b - first[s] of solve s, the last
-// solve with first[s] <= b; the solve's grid length selects the stage body
-// compiled for it (the same body the single-size kernels run, so a solve
-// computes exactly what it computes alone).  Every size carried here runs its
-// default column tile in 256-thread workgroups.  192 is left out: its bodies
+// solve with first[s] <= b, or four of them, one per wave (the short lengths);
+// the solve's grid length selects the stage body compiled for it (the same
+// body the single-size kernels run, so a solve computes exactly what it
+// computes alone).  192 is left out: its bodies
 // need 205-226 registers, and one launch takes the largest register count of
 // the bodies it carries (two waves per SIMD instead of three for the other
 // sizes' stages 1-3).
@@ -19,16 +19,20 @@ namespace {
 
 constexpr int kMultiThreads = 256;
 
+// threads of a size's column tile, and its tiles per workgroup: one, or the
+// wave tiles of the short lengths, each run by one wave
 template <int N>
-constexpr bool multi_size_ok() {
-  return tbw<float, N>() * TFof<N, zsplan<float, N>()>() == kMultiThreads;
-}
+constexpr int tile_threads() { return tbw<float, N>() * TFof<N, zsplan<float, N>()>(); }
+template <int N>
+constexpr int tiles_per_wg() { return kMultiThreads / tile_threads<N>(); }
+template <int N>
+constexpr bool multi_size_ok() { return tile_threads<N>() == kMultiThreads || tile_threads<N>() == 64; }
 static_assert(multi_size_ok<32>() && multi_size_ok<64>() && multi_size_ok<128>() && multi_size_ok<256>(),
-              "every size of the shared stage launch runs 256-thread workgroups");
+              "every size of the shared stage launch runs whole 256-thread workgroups or waves");
 
 template <int SCH, int STG, int N>
 constexpr int lds_of() {
-  return zs_lds_bytes<float, N, SCH, STG, tbw<float, N>(), zsplan<float, N>()>();
+  return tiles_per_wg<N>() * zs_lds_bytes<float, N, SCH, STG, tbw<float, N>(), zsplan<float, N>()>();
 }
 template <int SCH, int STG>
 constexpr int multi_lds() {
@@ -36,6 +40,20 @@ constexpr int multi_lds() {
                 d = lds_of<SCH, STG, 256>();
   constexpr int ab = a > b ? a : b, cd = c > d ? c : d;
   return ab > cd ? ab : cd;
+}
+
+// workgroup wg of one solve of length N
+template <int N, int SCH, int STG, bool PROBE>
+__device__ __forceinline__ void run_size(const ZsArgs<float>& a, int wg, unsigned char* smraw, double* red, double* fred) {
+  constexpr int TB = tbw<float, N>(), V = zsplan<float, N>();
+  if constexpr (tiles_per_wg<N>() == 1) {
+    zstage_body<float, N, SCH, STG, TB, V, PROBE>(a, wg, int(threadIdx.x), smraw, red, fred);
+  } else {
+    const int sub = int(threadIdx.x) / 64, tile = wg * tiles_per_wg<N>() + sub;
+    if (tile < zgroups(a.g, TB))
+      zstage_body<float, N, SCH, STG, TB, V, PROBE>(a, tile, int(threadIdx.x) % 64,
+                                                    smraw + sub * zs_lds_bytes<float, N, SCH, STG, TB, V>(), red, fred);
+  }
 }
 
 template <int SCH, int STG, bool PROBE>
@@ -49,18 +67,15 @@ __global__ void __launch_bounds__(kMultiThreads) k_zstage_multi(ZsMultiArgs m) {
     else hi = mid - 1;
   }
   const ZsArgs<float> a = static_cast<const ZsArgs<float>*>(m.args)[lo];
-  const int tile = b - m.first[lo];
+  const int wg = b - m.first[lo];
   __shared__ __align__(16) unsigned char smraw[multi_lds<SCH, STG>()];
   __shared__ double red[kMultiThreads / 64];
+  __shared__ double fred[4 * (kMultiThreads / 64)];
   switch (m.n[lo]) {
-    case 32: zstage_body<float, 32, SCH, STG, tbw<float, 32>(), zsplan<float, 32>(), PROBE>(a, tile, smraw, red); break;
-    case 64: zstage_body<float, 64, SCH, STG, tbw<float, 64>(), zsplan<float, 64>(), PROBE>(a, tile, smraw, red); break;
-    case 128:
-      zstage_body<float, 128, SCH, STG, tbw<float, 128>(), zsplan<float, 128>(), PROBE>(a, tile, smraw, red);
-      break;
-    case 256:
-      zstage_body<float, 256, SCH, STG, tbw<float, 256>(), zsplan<float, 256>(), PROBE>(a, tile, smraw, red);
-      break;
+    case 32: run_size<32, SCH, STG, PROBE>(a, wg, smraw, red, fred); break;
+    case 64: run_size<64, SCH, STG, PROBE>(a, wg, smraw, red, fred); break;
+    case 128: run_size<128, SCH, STG, PROBE>(a, wg, smraw, red, fred); break;
+    case 256: run_size<256, SCH, STG, PROBE>(a, wg, smraw, red, fred); break;
     default: break;
   }
 }

@@ -18,13 +18,16 @@ namespace vb {
 // group, with the solves' argument structs in a device table.
 enum PipeOp {
   OP_XA_RS, OP_XA_F, OP_XA_S, OP_XA_SUMS, OP_Y_FWD, OP_Y_INV, OP_Y_FWD_GM, OP_ZLAP, OP_ZPREP,
-  OP_ZS41, OP_ZS42, OP_ZS43, OP_ZS44, OP_ZS21, OP_ZS22, OP_FIN, OP_KEEP, OP_RETARGET, OP_ZS44P, OP_RELAYOUT
+  OP_ZS41, OP_ZS42, OP_ZS43, OP_ZS44, OP_ZS21, OP_ZS22, OP_FIN, OP_KEEP, OP_ZS44P, OP_RELAYOUT,
+  OP_PL_ETD, OP_PL_SUMS, OP_PL_ROWSUMS
 };
 // x-kernel outputs: the partial sums of v, (v^2-1)^2 and f^2 only (k_xrow
 // without its forward transform: the integrals of a field), tmp1 and f
 // (Euler), tmp1 and s (spectral N), the partial sums of v and (v^2-1)^2 only
 // (from P alone: k_xsums)
 enum XaMode { XA_ROWSUMS = 0, XA_WITHF = 1, XA_WITHS = 2, XA_SUMS = 3 };
+// modes of the plane kernel (k_plane)
+enum PlaneMode { PL_ETD = 0, PL_SUMS = 1, PL_ROWSUMS = 2 };
 struct RecLaunch {
   // issues the table form of the recorded kernel over `lanes` solves
   void (*launch_tab)(int op, const void* tab, dim3 grid, dim3 block, int lanes, hipStream_t s);
@@ -48,6 +51,20 @@ inline void record_launch(void (*tabfn)(int, const void*, dim3, dim3, int, hipSt
   r.block = block;
   g_recorder->seq.push_back(std::move(r));
 }
+
+template <typename T>
+struct PlaneArgs {
+  const cpx<T>* P;   // z-inverse of v^
+  const cpx<T>* Q;   // z-inverse of -|k|^2 v^ (PL_SUMS: unused)
+  cpx<T>* U;         // PL_ETD out: x,y-forward of tmp1 and eps^3 s (k_xrow's units),
+  cpx<T>* U2;        // in the z kernels' group-major layout, column tile ztb
+  double* part;      // [workgroup][3]
+  double* dcpart;    // FP32 PL_ETD: [workgroup][2], or nullptr
+  const cpx<T>* tw;
+  Geo g;
+  int ztb, pad;
+  double eps, kappa, D;
+};
 
 template <typename T> struct XaArgs;
 template <typename T> struct XeArgs;
@@ -84,6 +101,10 @@ struct SizeOps {
   // stg 1..sch; 5: the probe form of ETDRK4 stage 4 (V and A of the result
   // only: no state store, P alone)
   void (*zstage)(const ZsArgs<T>& a, int sch, int stg, hipStream_t s);
+  // the prefix with a whole xy plane in LDS (vb_plane.hpp), mode: PlaneMode;
+  // nullptr where a plane does not fit.  Its partials are one set per
+  // workgroup: nz of them (PL_SUMS: nz / 2).
+  void (*plane)(const PlaneArgs<T>& a, int mode, hipStream_t s);
 };
 
 // launch table of kernel schedule sc of length N (nullptr if not compiled),

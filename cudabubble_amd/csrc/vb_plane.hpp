@@ -1,0 +1,207 @@
+// vb_plane.hpp -- the ETD prefix of one field with a whole xy plane in LDS.
+//
+// For grids whose plane of v and lap v (as half spectra: N x (N + 2) complex
+// values) fits the 160 KB of LDS, the y-inverse, the x kernel (k_xrow) and the
+// y-forward run as one kernel, one workgroup per z: P and Q are read once and
+// the spectra of tmp1 and s written once, instead of three kernels that each
+// read and write both arrays.
+//
+// What bounds it: the chain of its phases at the short lengths (one workgroup
+// per CU at most), VALU issue at 128 (42 000 cycles for 16 waves).  So the
+// transforms stay inside a wave (no workgroup barrier but between the three
+// phases), the twiddles are read from LDS, the Nyquist columns have a wave of
+// their own, and the sums go through DPP moves.  Measured: 32^3 FP64 6.2 us
+// against 13.1 for the three kernels, 64^3 FP32 8.7 against 14.7, 128^3 FP32
+// 23 against 33; a penalty-drift step 173 -> 104, 195 -> 138, 489 -> 416 us
+// (with the combines evaluating the integrals and their wave tiles), batches of
+// 16 x 32^3, 16 x 64^3, 12 x 128^3 302 -> 186, 712 -> 617, 3465 -> 2835 us.
+#pragma once
+#include "vb_kernels.hpp"
+
+namespace vb {
+
+template <typename T, int N>
+struct PlaneCfg {
+  // plans with every transform inside one wave: the two-pass plan at 128, 12 x
+  // 4 (x 2) at 48 and 96, else the default
+  static constexpr int V = N == 128 ? 1 : (N == 48 || N == 96) ? 3 : 0;
+  static constexpr int E = N <= 128 ? Plan<N, V>::E : 8;
+  static constexpr int TF = N / E;
+  static constexpr int NT = N * TF;                 // TF lanes per row, and per column of P and Q but Nyquist
+  // the two Nyquist columns are a wave's of their own, so that no wave runs
+  // two column transforms one after the other, where there is room for one
+  static constexpr int XW = NT + 64 <= 1024 ? 1 : 0;
+  static constexpr int NA = NT + 64 * XW;           // threads of the workgroup
+  static constexpr int PS = (N == 96 || N == 128) ? 4 : 3;
+  // a row holds the N points of its transform, or its N + 2 half-spectrum
+  // modes: P[0, N/2), Q[0, N/2), then the two Nyquist modes
+  static constexpr int LL = N + 2 + ((N + 1) >> PS);
+  static constexpr int bytes = N * LL * int(sizeof(cpx<T>));
+  static constexpr bool ok = N <= 128 && NT <= 1024 && bytes + N * int(sizeof(cpx<T>)) + 1024 <= 160 * 1024;
+};
+
+// Element (ky, kx) of a plane of half-spectrum rows (see Geo).
+__device__ __forceinline__ int plane_pos(const Geo& g, int ky, int kx) {
+  return (g.nq >= 0 && kx == g.nx / 2) ? int(g.nq) + ky : ky * g.pitch + kx;
+}
+
+// PL_ETD: the prefix of a stage (k_ypass, k_xrow and the group-major k_ypass
+// in one; the same terms and units as k_xrow).  PL_ROWSUMS: the partial sums
+// of v, (v^2-1)^2 and f^2 only.  PL_SUMS: the partial sums of v and (v^2-1)^2
+// from P alone, two planes per workgroup, the second in Q's place.
+template <typename T, int N, int MODE, bool TAB = false>
+__global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0, const PlaneArgs<T>* tab) {
+  using C = PlaneCfg<T, N>;
+  constexpr int E = C::E, TF = C::TF, LL = C::LL, PS = C::PS, V = C::V, NT = C::NT, NA = C::NA, CW = 64 / TF,
+                H = N / 2;
+  static_assert(64 % TF == 0 && N % CW == 0, "whole lane groups per wave");
+  const PlaneArgs<T> a = TAB ? tab[blockIdx.z] : a0;
+  const Geo& g = a.g;
+  __shared__ cpx<T> sm[N * LL];
+  __shared__ cpx<T> tw[N];
+  __shared__ double red[5 * (NA / 64)];
+  const int z = MODE == PL_SUMS ? 2 * int(blockIdx.x) : pair_item(int(blockIdx.x), int(gridDim.x));
+  const cpx<T>* const pA = a.P + (long long)z * g.pp;
+  const cpx<T>* const pB = MODE == PL_SUMS ? pA + g.pp : a.Q + (long long)z * g.pp;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  // columns: CW consecutive ones per wave; column c of [0, N) is P's kx = c,
+  // then Q's; the two Nyquist columns are the extra wave's, or (XW = 0) the
+  // first wave's second ones
+  const int cj = lane / CW, cc = wave * CW + lane % CW;
+  auto slot = [](int c) { return c + (c >> PS); };
+  // which array a column is of: by wave where no wave has both
+  auto second = [&](int c) { return H % CW == 0 && c < N ? wave * CW >= H : c < N ? c >= H : c > N; };
+  auto load = [&](cpx<T>* x, int c) {
+    const cpx<T>* const p = second(c) ? pB : pA;
+    const int kx = c < N ? c % H : H;
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = p[unsigned(plane_pos(g, cj + TF * e, kx))];
+  };
+  auto inv = [&](cpx<T>* x, int c) {
+    PlaneCol<T, LL> col{sm + slot(c)};
+    fft<T, N, +1, V>(x, cj, tw, col);
+#pragma unroll
+    for (int e = 0; e < E; ++e) col(cj + TF * e) = x[e];
+  };
+  const bool main = wave < NT / 64, act = main || lane % CW < 2;
+  {
+    cpx<T> x[E];
+    if (act) load(x, cc);
+    // the twiddles from LDS: a pass's loads of them would be a round trip to L2
+    if (threadIdx.x < N) tw[threadIdx.x] = a.tw[threadIdx.x];
+    __syncthreads();
+    if (act) inv(x, cc);
+    if (!C::XW && wave == 0 && lane % CW < 2) {
+      load(x, N + lane % CW);
+      inv(x, N + lane % CW);
+    }
+  }
+  __syncthreads();
+  constexpr int K = (MODE == PL_ETD && sizeof(T) == 4) ? 5 : 3;
+  double acc[K] = {};
+  if (main) {
+    const int r = threadIdx.x / TF, j = threadIdx.x % TF;
+    PlaneRow<T, PS> row{sm + r * LL};
+    cpx<T> x[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      // pack2 over the row's slots
+      const int p = j + TF * e;
+      const bool mir = p > H;
+      const int k = mir ? N - p : p;
+      cpx<T> u = row(k == H ? N : k), w = row(k == H ? N + 1 : H + k);
+      if (k == 0 || k == H) { u.y = T(0); w.y = T(0); }
+      if (mir) { u.y = -u.y; w.y = -w.y; }
+      x[e] = mk<T>(u.x - w.y, u.y + w.x);
+    }
+    row.sync();
+    fft<T, N, +1, V>(x, j, tw, row);
+    const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps, D = a.D;
+    T ts[5] = {T(0), T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if constexpr (MODE == PL_SUMS) {
+        const T v0 = x[e].x, v1 = x[e].y;
+        const double w0 = double(v0 * v0 - T(1)), w1 = double(v1 * v1 - T(1));
+        acc[0] += double(v0) + double(v1);
+        acc[1] += w0 * w0 + w1 * w1;
+      } else {
+        const T v = x[e].x, lv = x[e].y;
+        const T w = v * v - T(1);
+        const T f = -lv * T(eps) + w * v * T(ieps);                               // f_kernel, Calc.cu:160
+        const T t1 = v * (w - T(kappa));                                          // nld_kernel1, Calc.cu:270
+        const T sv = T(D) * t1 + (T(3 * eps) * v * v - T(eps * (D + 1))) * f;     // Calc.cu:282, times eps^3
+        if constexpr (sizeof(T) == 4) {
+          ts[0] += v; ts[1] += w * w; ts[2] += f * f; ts[3] += t1; ts[4] += sv;
+        } else {
+          acc[0] += double(v); acc[1] += double(w) * double(w); acc[2] += double(f) * double(f);
+        }
+        x[e] = mk<T>(t1, sv);
+      }
+    }
+    if constexpr (MODE != PL_SUMS && sizeof(T) == 4) {
+#pragma unroll
+      for (int q = 0; q < K; ++q) acc[q] = double(ts[q]);
+    }
+    if constexpr (MODE == PL_ETD) {
+      constexpr int NH = H + 1, U = (NH + TF - 1) / TF;
+      fft<T, N, -1, V>(x, j, tw, row);
+#pragma unroll
+      for (int e = 0; e < E; ++e) row(j + TF * e) = x[e];
+      row.sync();
+      // unpack_store without SCALE, over the row's own slots
+      cpx<T> ua[U], ub[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int k = j + TF * i;
+        if (k < NH) {
+          const cpx<T> zk = row(k), zm = row(k == 0 ? 0 : N - k);
+          ua[i] = mk<T>(zk.x + zm.x, zk.y - zm.y);
+          ub[i] = mk<T>(zk.y + zm.y, zm.x - zk.x);
+        }
+      }
+      row.sync();
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int k = j + TF * i;
+        if (k < NH) {
+          row(k == H ? N : k) = ua[i];
+          row(k == H ? N + 1 : H + k) = ub[i];
+        }
+      }
+    }
+  }
+  wave_part<K, NA>(acc, red);
+  __syncthreads();
+  if (threadIdx.x < K) {
+    const double s = wave_total<NA>(red, threadIdx.x);
+    if (threadIdx.x < 3) a.part[3 * (long long)blockIdx.x + threadIdx.x] = s;
+    else if (a.dcpart) a.dcpart[2 * (long long)blockIdx.x + threadIdx.x - 3] = s;
+  }
+  if constexpr (MODE == PL_ETD) {
+    auto fwd = [&](int c) {
+      PlaneCol<T, LL> col{sm + slot(c)};
+      cpx<T> x[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = col(cj + TF * e);
+      col.sync();
+      fft<T, N, -1, V>(x, cj, tw, col);
+      const int kx = c < N ? c % H : H;
+      cpx<T>* const out = second(c) ? a.U2 : a.U;
+      if (g.aligned && c < N) {
+        // ky = cj + TF e: one ky step is one row of column groups of all z
+        const unsigned o = unsigned(gm_index(g, a.ztb, z, cj, kx)),
+                       st = unsigned(((H >> __builtin_ctz((unsigned)a.ztb)) * TF) * g.nz * a.ztb);
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[o + e * st] = x[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[unsigned(gm_index(g, a.ztb, z, cj + TF * e, kx))] = x[e];
+      }
+    };
+    if (act) fwd(cc);
+    if (!C::XW && wave == 0 && lane % CW < 2) fwd(N + lane % CW);
+  }
+}
+
+}  // namespace vb

@@ -5,6 +5,7 @@
 
 #include "vb_kernels.hpp"
 #include "vb_ops.hpp"
+#include "vb_plane.hpp"
 
 namespace vb {
 
@@ -70,11 +71,15 @@ struct Launch {
   static void xe(const XeArgs<T>& a, hipStream_t s) {
     hipLaunchKernelGGL((k_xe<T, N>), dim3(xgrid(a.npairs)), dim3(XWG), 0, s, a);
   }
+  static int ypad(const Geo& g, int nf) {
+    return g.aligned ? (kXcds - (nf + (g.nz + CB - 1) / CB) % kXcds) % kXcds : 0;
+  }
   static void ypass(cpx<T>* b0, cpx<T>* b1, int narr, int sign, const Geo& g, const cpx<T>* tw, const FinArgs* fin,
                     hipStream_t s) {
     const int nf = fin_groups(fin);
-    const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf), unsigned(narr)), bl(CT);
-    YArgs<T> a{b0, b1, tw, g, fin ? *fin : FinArgs{}, nf};
+    const int pad = ypad(g, nf);
+    const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf + pad), unsigned(narr)), bl(CT);
+    YArgs<T> a{b0, b1, tw, g, fin ? *fin : FinArgs{}, nf, pad};
     if (g_recorder) return record_launch(&launch_tab, sign < 0 ? OP_Y_FWD : OP_Y_INV, a, grid, bl);
     if (sign < 0)
       hipLaunchKernelGGL((k_ypass<T, N, -1, CB, false, CV>), grid, bl, 0, s, a, nullptr);
@@ -86,8 +91,9 @@ struct Launch {
   static void ypass_gm(const cpx<T>* b0, const cpx<T>* b1, cpx<T>* o0, cpx<T>* o1, int ztb, const Geo& g,
                        const cpx<T>* tw, const FinArgs* fin, hipStream_t s) {
     const int nf = fin_groups(fin);
-    const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf), 2u), bl(CT);
-    YArgs<T> a{const_cast<cpx<T>*>(b0), const_cast<cpx<T>*>(b1), tw, g, fin ? *fin : FinArgs{}, nf, o0, o1, ztb};
+    const int pad = ypad(g, nf);
+    const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf + pad), 2u), bl(CT);
+    YArgs<T> a{const_cast<cpx<T>*>(b0), const_cast<cpx<T>*>(b1), tw, g, fin ? *fin : FinArgs{}, nf, pad, o0, o1, ztb};
     if (g_recorder) return record_launch(&launch_tab, OP_Y_FWD_GM, a, grid, bl);
     hipLaunchKernelGGL((k_ypass<T, N, -1, CB, false, CV, true>), grid, bl, 0, s, a, nullptr);
   }
@@ -141,6 +147,24 @@ struct Launch {
     zs_dispatch<false>(sch, stg, gr, a, nullptr, s);
   }
 
+  template <bool TAB>
+  static void pl_launch(int mode, dim3 gr, const PlaneArgs<T>& a, const PlaneArgs<T>* tab, hipStream_t s) {
+    if constexpr (PlaneCfg<T, N>::ok) {
+      const dim3 bl(PlaneCfg<T, N>::NA);
+      if (mode == PL_ETD)
+        hipLaunchKernelGGL((k_plane<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
+      else if (mode == PL_SUMS)
+        hipLaunchKernelGGL((k_plane<T, N, PL_SUMS, TAB>), gr, bl, 0, s, a, tab);
+      else
+        hipLaunchKernelGGL((k_plane<T, N, PL_ROWSUMS, TAB>), gr, bl, 0, s, a, tab);
+    }
+  }
+  static void plane(const PlaneArgs<T>& a, int mode, hipStream_t s) {
+    const dim3 gr(unsigned(mode == PL_SUMS ? a.g.nz / 2 : a.g.nz));
+    if (g_recorder) return record_launch(&launch_tab, OP_PL_ETD + mode, a, gr, dim3(PlaneCfg<T, N>::NA));
+    pl_launch<false>(mode, gr, a, nullptr, s);
+  }
+
   // the table form of a recorded launch, over `lanes` solves (blockIdx.z)
   static void launch_tab(int op, const void* tab, dim3 gr, dim3 bl, int lanes, hipStream_t s) {
     gr.z = unsigned(lanes);
@@ -173,6 +197,9 @@ struct Launch {
       case OP_ZS41: case OP_ZS42: case OP_ZS43: case OP_ZS44:
         zs_dispatch<true>(4, op - OP_ZS41 + 1, gr, ZsArgs<T>{}, (const ZsArgs<T>*)tab, s);
         break;
+      case OP_PL_ETD: case OP_PL_SUMS: case OP_PL_ROWSUMS:
+        pl_launch<true>(op - OP_PL_ETD, gr, PlaneArgs<T>{}, (const PlaneArgs<T>*)tab, s);
+        break;
       case OP_ZS44P: zs_dispatch<true>(4, 5, gr, ZsArgs<T>{}, (const ZsArgs<T>*)tab, s); break;
       case OP_ZS21: case OP_ZS22:
         zs_dispatch<true>(2, op - OP_ZS21 + 1, gr, ZsArgs<T>{}, (const ZsArgs<T>*)tab, s);
@@ -203,6 +230,7 @@ struct Launch {
     o.zlap = &zlap;
     o.zprep = &zprep;
     o.zstage = &zstage;
+    o.plane = PlaneCfg<T, N>::ok ? &plane : nullptr;
     return o;
   }
 };

@@ -36,17 +36,16 @@ __global__ void __launch_bounds__(kFinThreads) k_finalize(FinArgs a0, const FinA
   const FinArgs a = TAB ? tab[blockIdx.z] : a0;
   __shared__ double red[6 * (kFinThreads / 64)];
   __shared__ double tot[7];
-  finalize_body<kFinThreads>(a, red, tot, 0, 1);
+  finalize_body<kFinThreads, 4, true>(a, red, tot, 0, 1);
 }
 
-// Across the penalty-drift double step: KEEP saves the scalars of the
-// current state (its integrals do not depend on the targets); RETARGET puts
-// them back under the current (drifted) targets, which is what the finalize
-// kernel would write for that state's partial sums.
+// Copy of the scalars of one field: the state's, kept for the second
+// evaluation of the penalty-drift double step, or the targets of the FP64
+// integrals of FP32-mixed mode.  Inside a recurring step the finalize kernel
+// keeps and retargets them itself (FinArgs::fold).
 struct KeepArgs {
-  Scal* sc;
+  const Scal* sc;
   Scal* keep;
-  Phys ph;
 };
 
 template <bool TAB>
@@ -55,36 +54,15 @@ __global__ void k_keep_scal(KeepArgs a0, const KeepArgs* tab) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *a.keep = *a.sc;
 }
 
-template <bool TAB>
-__global__ void k_retarget(KeepArgs a0, const KeepArgs* tab) {
-  const KeepArgs a = TAB ? tab[blockIdx.z] : a0;
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    Scal c = *a.keep;
-    c.alpha = a.sc->alpha;
-    c.beta = a.sc->beta;
-    c.alpha0 = a.sc->alpha0;
-    c.beta0 = a.sc->beta0;
-    apply_targets(c, a.ph);
-    *a.sc = c;
-  }
-}
-
-static void keep_tab(int op, const void* tab, dim3 gr, dim3 bl, int lanes, hipStream_t s) {
+static void keep_tab(int, const void* tab, dim3 gr, dim3 bl, int lanes, hipStream_t s) {
   gr.z = unsigned(lanes);
-  if (op == OP_KEEP)
-    hipLaunchKernelGGL(k_keep_scal<true>, gr, bl, 0, s, KeepArgs{}, (const KeepArgs*)tab);
-  else
-    hipLaunchKernelGGL(k_retarget<true>, gr, bl, 0, s, KeepArgs{}, (const KeepArgs*)tab);
+  hipLaunchKernelGGL(k_keep_scal<true>, gr, bl, 0, s, KeepArgs{}, (const KeepArgs*)tab);
 }
 
-// op: OP_KEEP or OP_RETARGET
-static void launch_keep(int op, Scal* sc, Scal* keep, const Phys& ph, hipStream_t s) {
-  const KeepArgs a{sc, keep, ph};
-  if (g_recorder) return record_launch(&keep_tab, op, a, dim3(1), dim3(64));
-  if (op == OP_KEEP)
-    hipLaunchKernelGGL(k_keep_scal<false>, dim3(1), dim3(64), 0, s, a, nullptr);
-  else
-    hipLaunchKernelGGL(k_retarget<false>, dim3(1), dim3(64), 0, s, a, nullptr);
+static void launch_keep(const Scal* sc, Scal* keep, hipStream_t s) {
+  const KeepArgs a{sc, keep};
+  if (g_recorder) return record_launch(&keep_tab, OP_KEEP, a, dim3(1), dim3(64));
+  hipLaunchKernelGGL(k_keep_scal<false>, dim3(1), dim3(64), 0, s, a, nullptr);
 }
 
 __global__ void k_fill_scal(Scal* sc, double alpha, double beta, double alpha0, double beta0) {
@@ -115,19 +93,18 @@ FinArgs fin_args(const double* xpart, int nxb, const double* zpart, const double
   a.dc = dc;
   a.dcpart = nullptr;
   a.sc = sc;
+  a.keep = nullptr;
   a.fs = fs;
   a.nxb = nxb;
   a.nzb = nzb;
   a.mode = mode;
-  a.pad = 0;
+  a.fold = FOLD_NONE;
   a.g = g;
   a.ph = ph;
   return a;
 }
 
-void launch_finalize(const double* xpart, int nxb, const double* zpart, const double* dc, int nzb, Scal* sc,
-                     const Geo& g, const Phys& ph, int mode, hipStream_t s) {
-  const FinArgs a = fin_args(xpart, nxb, zpart, dc, nzb, sc, nullptr, g, ph, mode);
+void launch_finalize(const FinArgs& a, hipStream_t s) {
   if (g_recorder) return record_launch(&finalize_tab, OP_FIN, a, dim3(1), dim3(kFinThreads));
   hipLaunchKernelGGL(k_finalize<false>, dim3(1), dim3(kFinThreads), 0, s, a, nullptr);
 }
@@ -185,6 +162,11 @@ struct Solver final : SolverBase {
   Scal* hs = nullptr;   // pinned host copy
   DBuf<double> rpart;   // block sums of the Euler residual
   int nxb = 0, nzb = 0;
+  // partial-sum sets of the last prefix's x (or plane) kernel, and which half
+  // of zpart and dc the prepared field's are in: the stage combines alternate
+  // (zprep and the last stage of either scheme use half 0), because one that
+  // evaluates the integrals itself reads one half while it writes the other
+  int nxlast = 0, zhalf = 0;
   long long npairs = 0;
   int mmax = 0;
   // ETD coefficient tables: a fixed pool of slots allocated with the solver.
@@ -211,6 +193,8 @@ struct Solver final : SolverBase {
   int cur = 0;
   bool prepped = false;     // P, Q hold zprep of uh[cur]
   bool prefixed = false;    // ETD prefix of uh[cur] done (scal; Tt, Ts: x,y-forward of tmp1, s)
+  bool kept = false;        // scal_keep holds scal of uh[cur] (the drift double step starts from it)
+  bool fin_pending = false; // the last prefix left its integrals to the next stage combine
   bool prefixed_f = false;  // Euler prefix of uh[cur] done (scal; v, f; W: x-spectra of lap f)
   // driver state
   bool started = false;
@@ -235,11 +219,11 @@ struct Solver final : SolverBase {
   // so theirs are replayed whatever dt is.
   struct PipeState {
     int cur;
-    bool prepped, prefixed, prefixed_f;
+    bool prepped, prefixed, prefixed_f, kept;
     double dt;
     bool operator==(const PipeState& o) const {
       return cur == o.cur && prepped == o.prepped && prefixed == o.prefixed && prefixed_f == o.prefixed_f &&
-             dt == o.dt;
+             kept == o.kept && dt == o.dt;
     }
   };
   enum { kFixedPair = 0, kAttempt = 1, kChain = 2, kShapeAttempt = 3, kEulerAttempt = 4, kShapeChain = 5 };
@@ -314,14 +298,15 @@ struct Solver final : SolverBase {
       v.alloc(nr);
       f.alloc(nr);
     }
-    dc.alloc(1);
+    dc.alloc(2);
     phid.alloc(nr);
     npairs = (long long)g.nz * g.ny / 2;
     nxb = int((npairs + ox->xlanes - 1) / ox->xlanes);
     nzb = int(zgroups(g, oz->ytile));
-    xpart.alloc((size_t)nxb * 3);
-    if (kMixed) xdc.alloc((size_t)nxb * 2);
-    zpart.alloc((size_t)nzb);
+    const size_t nxp = (size_t)std::max(nxb, g.nz);   // k_plane writes one set per plane
+    xpart.alloc(nxp * 3);
+    if (kMixed) xdc.alloc(nxp * 2);
+    zpart.alloc(2 * (size_t)nzb);
     scal.alloc(1);
     scal_keep.alloc(1);
     fin_scratch.alloc(1);
@@ -503,6 +488,12 @@ struct Solver final : SolverBase {
     L("zprep", [&] { oz->zprep(vh, P.p, Q.p, zpart.p, dc.p, g, twz.p, st); });
     check_launch();
     prepped = true;
+    zhalf = 0;
+  }
+
+  // the integrals of the prepared field from nx sets of x partials
+  FinArgs fin_of(int nx, int mode) {
+    return fin_args(xpart.p, nx, zpart.p + (size_t)zhalf * nzb, dc.p + zhalf, nzb, scal.p, fin_scratch.p, g, ph, mode);
   }
 
   // fin: integrals to evaluate in the same launch as the z pass (extra
@@ -513,6 +504,31 @@ struct Solver final : SolverBase {
     L("y_inv", [&] { ox->ypass(b, nullptr, 1, +1, g, twx.p, nullptr, st); });
   }
 
+  void fold_keep(FinArgs& fin) {
+    fin.fold = FOLD_KEEP;
+    fin.keep = scal_keep.p;
+    kept = true;
+  }
+
+  // one plane kernel over the prepared field (PlaneMode)
+  void plane(int mode, cpx<T>* tt, cpx<T>* ts) {
+    PlaneArgs<T> a{};
+    a.P = P.p;
+    a.Q = Q.p;
+    a.U = tt;
+    a.U2 = ts;
+    a.part = xpart.p;
+    a.dcpart = (kMixed && mode == PL_ETD) ? xdc.p : nullptr;
+    a.tw = twx.p;
+    a.g = g;
+    a.ztb = oz->ytile;
+    a.eps = p.eps;
+    a.kappa = p.kappa;
+    a.D = p.D;
+    nxlast = mode == PL_SUMS ? g.nz / 2 : g.nz;
+    L(mode == PL_SUMS ? "plane_sums" : "plane", [&] { ox->plane(a, mode, st); });
+  }
+
   // The prefix of the prepared stage field (P, Q: its z-inverse spectra and
   // those of its Laplacian): the integrals in scal, and
   //  - ETD (withf = false): Tt, Ts = x,y-forward of tmp1 and s, from which the
@@ -520,9 +536,30 @@ struct Solver final : SolverBase {
   //  - Euler (withf = true): v, f and W = x-spectra of lap f (k_xe).
   // set 0: the prefix of the state (stage 1), kept in Tt, Ts; set 1: of a
   // later stage, in Tt1, Ts1 (so the state's survives an evaluation)
-  void prefix(int mode, bool withf, int set = 0) {
+  // defer (the stages inside an evaluation, where the next kernel is a stage
+  // combine): with a plane kernel the combine evaluates the integrals it needs.
+  // keep: the scalars also go to scal_keep.
+  void prefix(int mode, bool withf, int set = 0, bool defer = false, bool keep = false) {
     cpx<T>* tt = set ? Tt1.p : Tt.p;
     cpx<T>* ts = set ? Ts1.p : Ts.p;
+    kept = false;
+    if (ox->plane && !withf) {
+      plane(PL_ETD, tt, ts);
+      if (defer) {
+        fin_pending = true;
+      } else {
+        FinArgs fin = fin_of(nxlast, mode);
+        fin.dcpart = kMixed ? xdc.p : nullptr;
+        if (keep) fold_keep(fin);
+        L("finalize", [&] { launch_finalize(fin, st); });
+      }
+      check_launch();
+      prepped = false;
+      prefixed = true;
+      prefixed_f = false;
+      return;
+    }
+    nxlast = nxb;
     L("y_inv2", [&] { ox->ypass(P.p, Q.p, 2, +1, g, twx.p, nullptr, st); });
     XaArgs<T> a{};
     a.P = P.p;
@@ -547,8 +584,9 @@ struct Solver final : SolverBase {
     L(withf ? "xa_f" : "xa", [&] { ox->xa(a, withf ? XA_WITHF : XA_WITHS, st); });
     // the integrals of this field (xa's and the z kernel's partials) are
     // evaluated by extra workgroups of the next column pass
-    FinArgs fin = fin_args(xpart.p, nxb, zpart.p, dc.p, nzb, scal.p, fin_scratch.p, g, ph, mode);
+    FinArgs fin = fin_of(nxb, mode);
     fin.dcpart = a.dcpart;
+    if (keep) fold_keep(fin);
     if (withf) {
       spectral_lap(W.p, &fin);
     } else {
@@ -563,7 +601,13 @@ struct Solver final : SolverBase {
   // V and A of the prepared stage field alone (no stage data, and no E_b):
   // y-inverse of P, the partial sums of v and (v^2-1)^2, and the finalize
   // kernel.  Used where only the targets' drift is needed.
-  void prefix_integrals(int mode) {
+  void prefix_integrals(int mode, int fold) {
+    if (ox->plane) {
+      plane(PL_SUMS, nullptr, nullptr);
+      refinalize(mode, nxlast, fold);
+      prepped = prefixed = prefixed_f = false;
+      return;
+    }
     L("y_inv", [&] { ox->ypass(P.p, nullptr, 1, +1, g, twx.p, nullptr, st); });
     XaArgs<T> a{};
     a.P = P.p;
@@ -577,16 +621,20 @@ struct Solver final : SolverBase {
     a.inv_n = 1.0 / double(g.nr);
     a.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
     L("xa_sums", [&] { ox->xa(a, XA_SUMS, st); });
-    refinalize(mode, (nxb + kXsLoop - 1) / kXsLoop);
+    refinalize(mode, (nxb + kXsLoop - 1) / kXsLoop, fold);
     prepped = false;
     prefixed = false;
     prefixed_f = false;
   }
 
-  // nx_parts: the x partials written by the last x kernel (k_xsums writes fewer)
-  void refinalize(int mode, int nx_parts = -1) {
-    const int nxp = nx_parts < 0 ? nxb : nx_parts;
-    L("finalize", [&] { launch_finalize(xpart.p, nxp, zpart.p, dc.p, nzb, scal.p, g, ph, mode, st); });
+  // nx_parts: the x partials written by the last x kernel (k_xsums writes
+  // fewer); fold: FOLD_*
+  void refinalize(int mode, int nx_parts = -1, int fold = FOLD_NONE) {
+    FinArgs fin = fin_of(nx_parts < 0 ? nxlast : nx_parts, mode);
+    fin.fold = fold;
+    fin.keep = scal_keep.p;
+    kept = false;
+    L("finalize", [&] { launch_finalize(fin, st); });
     check_launch();
   }
 
@@ -610,8 +658,18 @@ struct Solver final : SolverBase {
     z.uout = uh[out].p;
     z.P = P.p;
     z.Q = Q.p;
-    z.part = zpart.p;
-    z.dc = dc.p;
+    z.xpart = xpart.p;
+    z.dcpart = xdc.p;
+    z.zin = zpart.p + (size_t)zhalf * nzb;
+    z.dcin = dc.p + zhalf;
+    z.nxb = fin_pending ? nxlast : 0;
+    z.nzb = nzb;
+    z.M1 = p.M1;
+    z.M2 = p.M2;
+    fin_pending = false;
+    zhalf = stg & 1;
+    z.part = zpart.p + (size_t)zhalf * nzb;
+    z.dc = dc.p + zhalf;
     z.c1 = lt ? lt->c1 : chain_c1.p;
     z.c2 = lt ? lt->c2 : chain_c2.p;
     z.tw = twz.p;
@@ -647,7 +705,7 @@ struct Solver final : SolverBase {
     const int out = 1 - cur;
     ensure_prefixed();
     for (int stg = 1; stg <= sch; ++stg) {
-      if (stg > 1) prefix(FIN_PLAIN, false, 1);
+      if (stg > 1) prefix(FIN_PLAIN, false, 1, true);
       suffix(sch, stg, lt, out, probe);
     }
     // after the last stage P, Q belong to uh[out]
@@ -694,22 +752,22 @@ struct Solver final : SolverBase {
   int fixed_body() {
     if (drift_mode()) {
       ensure_prefixed();
-      launch_keep(OP_KEEP, scal.p, scal_keep.p, ph, st);
+      if (!kept) launch_keep(scal.p, scal_keep.p, st);
       int out = eval(time_step, true);
       const int keep = cur;
       cur = out;
-      prefix_integrals(FIN_DRIFT);   // only the drift of the targets is used
+      // only the drift of the targets is used.  The second evaluation starts
+      // again from the kept state with the new targets.  Its prefix data (Tt,
+      // Ts) does not depend on the targets and is still there; only lambda1,
+      // lambda2 and E change (FOLD_RETARGET).
+      prefix_integrals(FIN_DRIFT, FOLD_RETARGET);
       cur = keep;
-      // The second evaluation starts again from the kept state with the new
-      // targets.  Its prefix data (Tt, Ts) does not depend on the targets and
-      // is still there; only lambda1, lambda2 and E change.
-      launch_keep(OP_RETARGET, scal.p, scal_keep.p, ph, st);
       prepped = false;
       prefixed = true;
       prefixed_f = false;
       out = eval(time_step);
       cur = out;
-      prefix(FIN_DRIFT, false);
+      prefix(FIN_DRIFT, false, 0, false, true);   // and keep the new state's scalars
       return 2;
     }
     ensure_prefixed();
@@ -717,12 +775,13 @@ struct Solver final : SolverBase {
     return 1;
   }
 
-  PipeState pipe_state() const { return PipeState{cur, prepped, prefixed, prefixed_f, time_step}; }
+  PipeState pipe_state() const { return PipeState{cur, prepped, prefixed, prefixed_f, kept, time_step}; }
   void set_pipe_state(const PipeState& q) {
     cur = q.cur;
     prepped = q.prepped;
     prefixed = q.prefixed;
     prefixed_f = q.prefixed_f;
+    kept = q.kept;
   }
 
   // Records the launches of `body` (returning its evaluation count) from the
@@ -1040,7 +1099,7 @@ struct Solver final : SolverBase {
       launch_chain_table(chain.p, chain_c1.p, chain_c2.p, mmax + 1, st);
       const int keep = cur, out = 1 - cur;
       for (int stg = 1; stg <= sch; ++stg) {
-        if (stg > 1) prefix(FIN_PLAIN, false, 1);
+        if (stg > 1) prefix(FIN_PLAIN, false, 1, true);
         suffix(sch, stg, nullptr, out);
       }
       cur = out;
@@ -1066,7 +1125,7 @@ struct Solver final : SolverBase {
     const PipeState now = pipe_state();
     for (auto& G : graphs)
       if (G.x && G.kind == kind && G.evals == K && G.pre.cur == now.cur && G.pre.prepped == now.prepped &&
-          G.pre.prefixed == now.prefixed && G.pre.prefixed_f == now.prefixed_f)
+          G.pre.prefixed == now.prefixed && G.pre.prefixed_f == now.prefixed_f && G.pre.kept == now.kept)
         return &G;
     return nullptr;
   }
@@ -1200,7 +1259,10 @@ struct Solver final : SolverBase {
   }
 
   // ---- drivers ----------------------------------------------------------------
-  void set_targets_device() { launch_fill_scal(scal.p, alpha, beta, alpha0, beta0, st); }
+  void set_targets_device() {
+    kept = false;
+    launch_fill_scal(scal.p, alpha, beta, alpha0, beta0, st);
+  }
 
   // One Euler attempt of the shape-adjust and run_static loops: the update of
   // uh[cur] with step t into uh[out], and the prefix of the candidate (its
@@ -1226,7 +1288,7 @@ struct Solver final : SolverBase {
     const PipeState now = pipe_state();
     for (auto& H : graphs)
       if (H.x && H.kind == kind && H.pre.cur == now.cur && H.pre.prepped == now.prepped &&
-          H.pre.prefixed == now.prefixed && H.pre.prefixed_f == now.prefixed_f)
+          H.pre.prefixed == now.prefixed && H.pre.prefixed_f == now.prefixed_f && H.pre.kept == now.kept)
         G = &H;
     if (!G) G = &capture(kind, [&] {
       body(true);
@@ -1474,7 +1536,7 @@ struct Solver final : SolverBase {
     scal64.alloc(1);
     nxb64 = int((npairs + oxd->xlanes - 1) / oxd->xlanes);
     nzb64 = int(zgroups(g, ozd->ytile));
-    xpart64.alloc((size_t)nxb64 * 3);
+    xpart64.alloc((size_t)std::max(nxb64, g.nz) * 3);
     zpart64.alloc((size_t)nzb64);
   }
 
@@ -1490,21 +1552,38 @@ struct Solver final : SolverBase {
       src = S.p;
     }
     L("zprep64", [&] { ozd->zprep(src, P64.p, Q64.p, zpart64.p, dc64.p, g, twzd.p, st); });
-    L("y_inv2_64", [&] { oxd->ypass(P64.p, Q64.p, 2, +1, g, twxd.p, nullptr, st); });
-    XaArgs<double> a{};
-    a.P = P64.p;
-    a.Q = Q64.p;
-    a.part = xpart64.p;
-    a.tw = twxd.p;
-    a.npairs = npairs;
-    a.eps = p.eps;
-    a.kappa = p.kappa;
-    a.D = p.D;
-    a.inv_n = 1.0 / double(g.nr);
-    a.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
-    L("xsums64", [&] { oxd->xa(a, XA_ROWSUMS, st); });
-    launch_keep(OP_KEEP, scal.p, scal64.p, ph, st);   // the targets
-    L("finalize64", [&] { launch_finalize(xpart64.p, nxb64, zpart64.p, dc64.p, nzb64, scal64.p, g, ph, FIN_PLAIN, st); });
+    int nx64 = nxb64;
+    if (oxd->plane) {
+      PlaneArgs<double> a{};
+      a.P = P64.p;
+      a.Q = Q64.p;
+      a.part = xpart64.p;
+      a.tw = twxd.p;
+      a.g = g;
+      a.eps = p.eps;
+      a.kappa = p.kappa;
+      a.D = p.D;
+      nx64 = g.nz;
+      L("plane_sums64", [&] { oxd->plane(a, PL_ROWSUMS, st); });
+    } else {
+      L("y_inv2_64", [&] { oxd->ypass(P64.p, Q64.p, 2, +1, g, twxd.p, nullptr, st); });
+      XaArgs<double> a{};
+      a.P = P64.p;
+      a.Q = Q64.p;
+      a.part = xpart64.p;
+      a.tw = twxd.p;
+      a.npairs = npairs;
+      a.eps = p.eps;
+      a.kappa = p.kappa;
+      a.D = p.D;
+      a.inv_n = 1.0 / double(g.nr);
+      a.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
+      L("xsums64", [&] { oxd->xa(a, XA_ROWSUMS, st); });
+    }
+    launch_keep(scal.p, scal64.p, st);   // the targets
+    L("finalize64", [&] {
+      launch_finalize(fin_args(xpart64.p, nx64, zpart64.p, dc64.p, nzb64, scal64.p, nullptr, g, ph, FIN_PLAIN), st);
+    });
     check_launch();
   }
 

@@ -1,0 +1,44 @@
+"""GPU parity of the plane kernel (an ETD prefix with a whole xy plane in LDS,
+csrc/vb_plane.hpp) and of the wave-wide column tiles of the stage combines, at
+every length that has them and at the shortest, odd and cubic depths: one
+evaluation, a penalty-drift step and the FP64 energies of a mixed state,
+against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import flush_print, rel, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", ["FP64", "FP32_MIXED"])
+@pytest.mark.parametrize("nx,nz", [(16, 16), (16, 48), (32, 16), (32, 32), (48, 48), (48, 16), (64, 16), (64, 96),
+                                   (96, 16), (96, 48), (128, 16), (128, 32)])
+def test_prefix_in_one_kernel(vb, gpu, oracle_mod, nx, nz, prec):
+    flush_print("plane", nx, nz, prec)
+    eps = 2.0 * 2 * np.pi / nx
+    phi, _ = vb.shape(vb.SHAPE_ELLIPSOID, 11, nx, nz, 1.0, eps)
+    # the reference's ETDRK4 brackets cancel at |h L^| << 1e-5: the wide interface
+    # of the 16^2 plane needs a longer step, and that one weaker penalties
+    h, M = (1e-5, 1e2) if nx == 16 else (1e-7, 1e4)
+    o = oracle_mod.Oracle(nx, nz, eps=eps, M1=M, M2=M, alpha=-1.0, beta=-1.0)
+    p = vb.params_default(nx=nx, nz=nz, eps=eps, M1=M, M2=M, alpha=-1.0, beta=-1.0, time_step=h,
+                          fixed_time_step=h, precision=getattr(vb, prec))
+    s = vb.Solver(p, phi)
+    r = s.step(3)
+    assert r["status"] == 0 and r["evaluations"] == 6
+    d = phi.copy()
+    st = o.fEIF_begin(d, h, fixed_time_step=h)
+    o.fEIF_steps(d, st, 3)
+    # FP64: as the other driver tests.  FP32-mixed: six evaluations that each add
+    # h N^ with the rounding of FP32 transforms, a few 1e-7 of h N^, which is
+    # itself below the field: 1e-6 of the field bounds it
+    tol = 1e-12 if prec == "FP64" else 1e-6
+    assert rel_l2(s.get_phi(), d) < tol
+    # V and A of the state: FP64 integrals in both precisions; their difference is
+    # that of the fields, to first order
+    E, V, A, Eb = s.query()
+    Eo, Vo, Ao, Ebo = o.energy(d)
+    assert rel(V, Vo) < 10 * tol and rel(A, Ao) < 10 * tol
+    if prec == "FP64":
+        assert rel(Eb, Ebo) < 1e-11
