@@ -2,6 +2,7 @@
 // spectral and pointwise operations (class Calc, Calc.h:8-119) on caller
 // device memory.  The fused solver does not use these entry points; they
 // exist so every reference operation can be called and checked on its own.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -35,28 +36,6 @@ __global__ void k_laplace(cpx<T>* u, Geo g) {
   const double tmp = -(x * x * c + y * y * c + z * z * c);
   u[tid].x = T(double(u[tid].x) * tmp);
   u[tid].y = T(double(u[tid].y) * tmp);
-}
-
-// gradient_kernel (Calc.cu:300-341)
-__global__ void k_gradient(const cpx<double>* u, cpx<double>* u1, cpx<double>* u2, cpx<double>* u3, Geo g) {
-  const long long tid = (long long)blockIdx.x * PW + threadIdx.x;
-  if (tid >= g.nc) return;
-  const double fac = g.kfac;
-  const int x = int(tid % g.nh);
-  if (x == g.nx / 2) u1[tid] = mk(0.0, 0.0);
-  else u1[tid] = mk(-(u[tid].y * fac) * x, (u[tid].x * fac) * x);
-  int y = int((tid % ((long long)g.ny * g.nh)) / g.nh);
-  if (y == g.ny / 2) u2[tid] = mk(0.0, 0.0);
-  else {
-    y = sgnk(y, g.ny);
-    u2[tid] = mk(-(u[tid].y * fac) * y, (u[tid].x * fac) * y);
-  }
-  int z = int(tid / ((long long)g.ny * g.nh));
-  if (z == g.nz / 2) u3[tid] = mk(0.0, 0.0);
-  else {
-    z = sgnk(z, g.nz);
-    u3[tid] = mk(-(u[tid].y * fac) * z, (u[tid].x * fac) * z);
-  }
 }
 
 enum { PW_F, PW_G0, PW_NLD1K, PW_NLD2K, PW_STERM, PW_MULTI, PW_PLUS, PW_NLD1, PW_NLD2 };
@@ -99,19 +78,33 @@ __global__ void k_pw(PwArgs p) {
   }
 }
 
-// Block partial sums of intf (intf_kernel, Calc.cu:224-252).  Workgroup b
-// adds the elements [b kSumChunk, (b + 1) kSumChunk) in a fixed order, so the
-// result does not depend on the number of CUs (the reference's grid is twice
-// the SM count, Calc.cu:259).
-constexpr long long kSumChunk = 256 * 256;
-inline long long sum_parts(long long n) { return (n + kSumChunk - 1) / kSumChunk; }
+// Block partial sums of intf (intf_kernel, Calc.cu:224-252).  Workgroup b adds
+// the elements [b c, (b + 1) c) in a fixed order, so the result does not depend
+// on the number of CUs (the reference's grid is twice the SM count,
+// Calc.cu:259).  The chunk c follows from the length alone: 4096 points, then
+// as many as keep the partials at 4096, up to 65536.  (65536 for every length
+// left a 128^3 sum to 32 workgroups: 64 us.)
+constexpr long long kSumParts = 16384;
+constexpr long long kSumMax = kSumParts * 65536;   // longest sum vb_intf_static takes
+inline long long sum_chunk(long long n) {
+  long long c = 4096;
+  while (c < 65536 && (n + c - 1) / c > 4096) c *= 2;
+  return c;
+}
+inline long long sum_parts(long long n) { return (n + sum_chunk(n) - 1) / sum_chunk(n); }
 
-__global__ void __launch_bounds__(256) k_sum(const double* __restrict__ u, long long n, double* __restrict__ part) {
+__global__ void __launch_bounds__(256) k_sum(const double* __restrict__ u, long long n, long long chunk,
+                                             double* __restrict__ part) {
   __shared__ double red[4];
-  double acc[1] = {0.0};
-  const long long b0 = (long long)blockIdx.x * kSumChunk;
-  const long long e = b0 + kSumChunk < n ? b0 + kSumChunk : n;
-  for (long long i = b0 + threadIdx.x; i < e; i += 256) acc[0] += u[i];
+  const long long b0 = (long long)blockIdx.x * chunk;
+  const long long e = b0 + chunk < n ? b0 + chunk : n;
+  double s[4] = {};   // four loads in flight
+  for (long long i = b0 + threadIdx.x; i < e; i += 1024) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i + 256 * k < e) s[k] += u[i + 256 * k];
+  }
+  double acc[1] = {(s[0] + s[1]) + (s[2] + s[3])};
   block_sum_store<1, 256>(acc, red, part + blockIdx.x);
 }
 
@@ -121,9 +114,15 @@ __global__ void __launch_bounds__(256) k_intf_final(const double* __restrict__ p
                                                     double addition, double mL3, double* __restrict__ out) {
   __shared__ double red[4];
   __shared__ double tot[1];
-  double acc[1] = {0.0};
-  for (int i = threadIdx.x; i < nb; i += 256) acc[0] += part[i];
+  double s[4] = {};
+  for (int i = threadIdx.x; i < nb; i += 1024) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i + 256 * k < nb) s[k] += part[i + 256 * k];
+  }
+  double acc[1] = {(s[0] + s[1]) + (s[2] + s[3])};
   block_sum_store<1, 256>(acc, red, tot);
+  __syncthreads();
   if (threadIdx.x == 0) out[0] = (tot[0] / N + addition) * mL3;
 }
 
@@ -132,7 +131,7 @@ __global__ void __launch_bounds__(256) k_intf_final(const double* __restrict__ p
 static void launch_intf(const double* u, long long n, double L, double addition, double multiply, double* part,
                         double* val, hipStream_t st) {
   const long long nb = sum_parts(n);
-  hipLaunchKernelGGL(k_sum, dim3(unsigned(nb)), dim3(256), 0, st, u, n, part);
+  hipLaunchKernelGGL(k_sum, dim3(unsigned(nb)), dim3(256), 0, st, u, n, sum_chunk(n), part);
   hipLaunchKernelGGL(k_intf_final, dim3(1), dim3(256), 0, st, part, int(nb), double(n), addition,
                      multiply * L * L * L, val);
 }
@@ -191,11 +190,12 @@ struct CalcImpl {
   const SizeOps<double>* ozd = nullptr;
   const SizeOps<float>* oxf = nullptr;
   const SizeOps<float>* ozf = nullptr;
-  DBuf<cpx<double>> c1, c2, c3, c4;
+  Geo ga{};   // layout of the transforms' scratch
+  DBuf<cpx<double>> c1, c2;
   DBuf<cpx<float>> fc1;
   DBuf<cpx<double>> twx, twz;
   DBuf<cpx<float>> twxf, twzf;
-  DBuf<double> part, val, rtmp;
+  DBuf<double> part, val;
   std::map<std::tuple<int, double, double>, std::unique_ptr<DBuf<Coef>>> luts;
   long long npairs = 0;
 
@@ -210,15 +210,27 @@ struct CalcImpl {
     ozd = get_ops<double>(nz);
     oxf = get_ops<float>(nx);
     ozf = get_ops<float>(nz);
-    const size_t nc = (size_t)g.nc;
-    c1.alloc(nc);
-    c2.alloc(nc);
-    c3.alloc(nc);
-    c4.alloc(nc);
+    // Where the x and y transforms are separate kernels, the spectra between
+    // them are rows of whole lines (see Geo); in one (k_pair) the caller's layout
+    // serves: a z pass reads and writes it in contiguous runs.
+    ga = g;
+    if (!(prec == VB_FP32_MIXED ? oxf->pair_r2c != nullptr : oxd->pair_r2c != nullptr) && (nx / 2) % 16 == 0) {
+      bool tiles = true;
+      for (int t : {oxd->ctile, ozd->ctile, ozd->ytile, oxf->ctile, ozf->ytile}) tiles = tiles && (nx / 2) % t == 0;
+      if (tiles) {
+        ga.pitch = nx / 2;
+        ga.aligned = 1;
+        ga.nq = (long long)ga.ny * ga.pitch;
+        ga.pp = ga.nq + ga.ny + 16;
+        ga.ncp = (long long)ga.nz * ga.pp;
+      }
+    }
+    const size_t nc = (size_t)std::max(g.nc, ga.ncp);
     if (prec == VB_FP32_MIXED) fc1.alloc(nc);
+    c1.alloc(nc);   // the operators on FP64 fields take either precision's handle
+    c2.alloc(nc);
     part.alloc((size_t)sum_parts(g.nr));
     val.alloc(1);
-    rtmp.alloc((size_t)g.nr);
     npairs = (long long)nz * nx / 2;
     std::vector<double> t;
     build_twiddles(t, nx);
@@ -252,36 +264,58 @@ struct CalcImpl {
     VB_HIP(hipStreamSynchronize(st));
   }
 
+  // The transforms of one precision: x and y in one kernel (k_pair) or two, and
+  // a z pass between the scratch and the caller's layout, times a factor of
+  // the mode where an operator has one.
+  template <typename T>
+  struct Fft {
+    const SizeOps<T>*ox, *oz;
+    const cpx<T>*twx, *twz;
+    cpx<T>* w;   // scratch
+  };
+  Fft<double> fd() { return {oxd, ozd, twx.p, twz.p, c1.p}; }
+  Fft<float> ff() { return {oxf, ozf, twxf.p, twzf.p, fc1.p}; }
+
+  // x and y transforms of u into layout gl of s, normalised
+  template <typename T>
+  void fwd_xy(const Fft<T>& f, const T* u, cpx<T>* s, const Geo& gl) {
+    const double n = 1.0 / double(g.nr);
+    if (f.ox->pair_r2c && !gl.aligned) return f.ox->pair_r2c(u, s, n, gl, f.twx, st);
+    f.ox->xr2c(u, s, npairs, f.twx, n, gl, st);
+    f.ox->ypass(s, nullptr, 1, -1, gl, f.twx, nullptr, st);
+  }
+  template <typename T>
+  void inv_xy(const Fft<T>& f, cpx<T>* s, T* u, const Geo& gl) {   // s is overwritten
+    if (f.ox->pair_c2r && !gl.aligned) return f.ox->pair_c2r(s, u, gl, f.twx, st);
+    f.ox->ypass(s, nullptr, 1, +1, gl, f.twx, nullptr, st);
+    f.ox->xc2r(s, u, npairs, f.twx, gl, st);
+  }
+  template <typename T>
+  void r2c_t(const Fft<T>& f, const T* u, cpx<T>* s) {
+    if (!ga.aligned) {
+      fwd_xy(f, u, s, g);
+      f.oz->zpass(s, -1, g, f.twz, st);
+    } else {
+      fwd_xy(f, u, f.w, ga);
+      f.oz->zmul(f.w, s, -1, ZM_ONE, ga, g, f.twz, st);
+    }
+  }
+  // the inverse transform of op (ZmOp) times s, which is preserved
+  template <typename T>
+  void c2r_t(const Fft<T>& f, const cpx<T>* s, T* u, int op) {
+    f.oz->zmul(s, f.w, +1, op, g, ga, f.twz, st);
+    inv_xy(f, f.w, u, ga);
+  }
+
   // forward normalised R2C (r2c_3d_f + normalize_kernel, Calc.cu:88-96)
   void r2c(const void* u, void* s) {
-    if (prec == VB_FP32_MIXED) {
-      cpx<float>* o = (cpx<float>*)s;
-      oxf->xr2c((const float*)u, o, npairs, twxf.p, 1.0 / double(g.nr), g, st);
-      oxf->ypass(o, nullptr, 1, -1, g, twxf.p, nullptr, st);
-      ozf->zpass(o, -1, g, twzf.p, st);
-    } else {
-      cpx<double>* o = (cpx<double>*)s;
-      oxd->xr2c_d((const double*)u, o, npairs, twx.p, 1.0 / double(g.nr), g, st);
-      oxd->ypass(o, nullptr, 1, -1, g, twx.p, nullptr, st);
-      ozd->zpass(o, -1, g, twz.p, st);
-    }
+    if (prec == VB_FP32_MIXED) r2c_t(ff(), (const float*)u, (cpx<float>*)s);
+    else r2c_t(fd(), (const double*)u, (cpx<double>*)s);
   }
-  // backward C2R of a buffer that may be overwritten (c2r_3d_b, Calc.cu:99-104)
-  void c2r_destroy(cpx<double>* s, double* u) {
-    ozd->zpass(s, +1, g, twz.p, st);
-    oxd->ypass(s, nullptr, 1, +1, g, twx.p, nullptr, st);
-    oxd->xc2r_d(s, u, npairs, twx.p, g, st);
-  }
+  // backward C2R (c2r_3d_b, Calc.cu:99-104); s is preserved
   void c2r(const void* s, void* u) {
-    if (prec == VB_FP32_MIXED) {
-      VB_HIP(hipMemcpyAsync(fc1.p, s, sizeof(cpx<float>) * (size_t)g.nc, hipMemcpyDeviceToDevice, st));
-      ozf->zpass(fc1.p, +1, g, twzf.p, st);
-      oxf->ypass(fc1.p, nullptr, 1, +1, g, twxf.p, nullptr, st);
-      oxf->xc2r(fc1.p, (float*)u, npairs, twxf.p, g, st);
-    } else {
-      VB_HIP(hipMemcpyAsync(c4.p, s, sizeof(cpx<double>) * (size_t)g.nc, hipMemcpyDeviceToDevice, st));
-      c2r_destroy(c4.p, (double*)u);
-    }
+    if (prec == VB_FP32_MIXED) c2r_t(ff(), (const cpx<float>*)s, (float*)u, ZM_ONE);
+    else c2r_t(fd(), (const cpx<double>*)s, (double*)u, ZM_ONE);
   }
   void laplace(void* s) {
     if (prec == VB_FP32_MIXED)
@@ -289,21 +323,19 @@ struct CalcImpl {
     else
       hipLaunchKernelGGL(k_laplace<double>, dim3(pgrid(g.nc)), dim3(PW), 0, st, (cpx<double>*)s, g);
   }
-  void lap_spec(const void* fd, void* out) {   // Calc.cu:139-144
-    VB_HIP(hipMemcpyAsync(c1.p, fd, sizeof(cpx<double>) * (size_t)g.nc, hipMemcpyDeviceToDevice, st));
-    laplace(c1.p);
-    c2r_destroy(c1.p, (double*)out);
+  void lap_spec(const void* fds, void* out) {   // Calc.cu:139-144
+    c2r_t(fd(), (const cpx<double>*)fds, (double*)out, ZM_LAP);
   }
   void lap_real(const void* d, void* out) {    // Calc.cu:146-151
-    r2c(d, c1.p);
-    laplace(c1.p);
-    c2r_destroy(c1.p, (double*)out);
+    const Fft<double> f = fd();
+    fwd_xy(f, (const double*)d, f.w, ga);
+    f.oz->zlap(f.w, ga, f.twz, nullptr, st);
+    inv_xy(f, f.w, (double*)out, ga);
   }
-  void fftgradient(const void* fd, void* dx, void* dy, void* dz) {   // Calc.cu:344-356
-    hipLaunchKernelGGL(k_gradient, dim3(pgrid(g.nc)), dim3(PW), 0, st, (const cpx<double>*)fd, c1.p, c2.p, c3.p, g);
-    c2r_destroy(c1.p, (double*)dx);
-    c2r_destroy(c2.p, (double*)dy);
-    c2r_destroy(c3.p, (double*)dz);
+  void fftgradient(const void* fds, void* dx, void* dy, void* dz) {   // Calc.cu:344-356
+    c2r_t(fd(), (const cpx<double>*)fds, (double*)dx, ZM_DX);
+    c2r_t(fd(), (const cpx<double>*)fds, (double*)dy, ZM_DY);
+    c2r_t(fd(), (const cpx<double>*)fds, (double*)dz, ZM_DZ);
   }
   template <int OP>
   void pw(double* out, const void* a, const void* b, const void* c, const void* d, double s0, double s1 = 0,
@@ -459,8 +491,8 @@ int vb_calc_etd2(vb_calc* c, void* a, const void* fd, const void* nnld, const vo
 }
 int vb_calc_etd41(vb_calc* c, void* d_real, const void* fd, const void* nld, double eps, double h) {
   CALC_BODY({
-    k.etd<vb::ETD_41>(k.c1.p, fd, nld, nullptr, nullptr, eps, h);
-    k.c2r_destroy(k.c1.p, (double*)d_real);
+    k.etd<vb::ETD_41>(k.c2.p, fd, nld, nullptr, nullptr, eps, h);
+    k.c2r_t(k.fd(), k.c2.p, (double*)d_real, vb::ZM_ONE);
   });
 }
 int vb_calc_etd42(vb_calc* c, void* b, const void* fd, const void* nlda, double eps, double h) {
@@ -472,8 +504,8 @@ int vb_calc_etd43(vb_calc* c, void* cc, const void* nld, const void* nldb, doubl
 int vb_calc_etd44(vb_calc* c, void* d_real, const void* fd, const void* nlda, const void* nldb, const void* nldc,
                   double eps, double h) {
   CALC_BODY({
-    k.etd<vb::ETD_44>(k.c1.p, fd, nlda, nldb, nldc, eps, h);
-    k.c2r_destroy(k.c1.p, (double*)d_real);
+    k.etd<vb::ETD_44>(k.c2.p, fd, nlda, nldb, nldc, eps, h);
+    k.c2r_t(k.fd(), k.c2.p, (double*)d_real, vb::ZM_ONE);
   });
 }
 int vb_calc_sync(vb_calc* c) { CALC_BODY((void)0); }
@@ -488,8 +520,7 @@ int vb_calc_sync(vb_calc* c) { CALC_BODY((void)0); }
 // address): the address of each device's copy is looked up once per device,
 // with that device current, and kept.
 // ---------------------------------------------------------------------------
-static constexpr long long kStaticParts = 16384;   // partials: inputs of up to 16384 * 65536 = 2^30 points
-static __device__ __align__(256) double scratch[kStaticParts];
+static __device__ __align__(256) double scratch[vb::kSumParts];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -519,9 +550,9 @@ int scratch_of_current(double** out) {
 extern "C" int vb_intf_static(const double* u, long long n, double lenx, double addition, double multiply,
                               double* val, void* stream) {
   if (!u || !val || n <= 0 || !(lenx > 0)) return VB_ERR_PARAM;
-  if (vb::sum_parts(n) > kStaticParts) {
+  if (n > vb::kSumMax) {
     vb::set_last_error("vb_intf_static: " + std::to_string(n) + " points exceed its maximum of " +
-                       std::to_string(kStaticParts * vb::kSumChunk));
+                       std::to_string(vb::kSumMax));
     return VB_ERR_PARAM;
   }
   double* part = nullptr;

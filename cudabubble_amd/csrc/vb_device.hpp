@@ -125,6 +125,9 @@ enum { FIN_PLAIN = 0, FIN_DRIFT = 1 };
 // under the targets just moved
 enum { FOLD_NONE = 0, FOLD_KEEP = 1, FOLD_RETARGET = 2 };
 
+// factors of k_zmul
+enum ZmOp { ZM_ONE = 0, ZM_LAP = 1, ZM_DX = 2, ZM_DY = 3, ZM_DZ = 4 };
+
 __device__ __forceinline__ int fold(int k, int n) { return k < n - k ? k : n - k; }
 __device__ __forceinline__ int sgnk(int k, int n) { return k < n - k ? k : k - n; }
 

@@ -41,6 +41,14 @@ __device__ __forceinline__ int pair_item(int b, int n) {
   return b < (n & ~15) ? (b & ~15) | ((b & 7) << 1) | ((b >> 3) & 1) : b;
 }
 
+// the same with whole rows of w items on an XCD, one after the other, from item
+// first on (a multiple of kXcds rows; the identity before it)
+__device__ __forceinline__ int row_item(int b, int first, int w) {
+  if (b < first) return b;
+  const unsigned i = unsigned(b - first), q = i / kXcds;
+  return first + int((q / w * kXcds + i % kXcds) * w + q % w);
+}
+
 constexpr int XWG = 64;   // threads per x-kernel workgroup: one wave (measured best at 256^3: 64 < 128 < 256)
 
 // Plan variant of the x kernels (row transforms).
@@ -209,7 +217,7 @@ __global__ void __launch_bounds__(XWG) k_xr2c(const TI* __restrict__ in, cpx<T>*
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int p = j + TF * e;
-    x[e] = mk<T>(T(in[r0 * N + p]), T(in[(r0 + 1) * N + p]));
+    x[e] = mk<T>(T(__builtin_nontemporal_load(in + r0 * N + p)), T(__builtin_nontemporal_load(in + (r0 + 1) * N + p)));
   }
   fft<T, N, -1, XP>(x, j, tw, lds);
   unpack_store<T, N, XP>(x, j, lds, out + rl.off(r0), out + rl.nyq(r0, N / 2), out + rl.off(r0 + 1),
@@ -239,8 +247,8 @@ __global__ void __launch_bounds__(XWG) k_xc2r(const cpx<T>* __restrict__ in, TO*
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int p = j + TF * e;
-      out[r0 * N + p] = TO(x[e].x);
-      out[(r0 + 1) * N + p] = TO(x[e].y);
+      __builtin_nontemporal_store(TO(x[e].x), out + r0 * N + p);
+      __builtin_nontemporal_store(TO(x[e].y), out + (r0 + 1) * N + p);
     }
   }
 }
@@ -852,6 +860,61 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zpass(cpx<T>* buf, Geo g, 
   if (id.valid) {
 #pragma unroll
     for (int e = 0; e < E; ++e) col[(long long)(j + TF * e) * plane] = x[e];
+  }
+}
+
+// A z pass from one buffer and layout to another, the input times a factor of
+// the mode first (the Calc level's laplace and gradient terms): ZM_LAP -|k|^2
+// (laplace_kernel, Calc.cu:114-122), ZM_DX, DY, DZ i times the component's wave
+// number, zero at its Nyquist plane (gradient_kernel, Calc.cu:310-339).  HBM
+// bounds it.  The caller's rows (nx / 2 + 1 modes) are not whole lines, so a
+// row's tiles run one after the other on one XCD (row_item: 136 -> 129 us at
+// 384^3 FP32 into the aligned scratch, 121 -> 117 back).  The input is read past
+// the caches, so that the memory-side cache keeps the scratch that the next
+// kernel reads: with the real side of the x kernels past them too, 384^3 FP32
+// forward and back took 640 -> 562 us in kernels.
+template <typename T>
+struct ZmArgs {
+  const cpx<T>* in;
+  cpx<T>* out;
+  const cpx<T>* tw;
+  Geo gi, go;   // layouts of in and out; the tiles are those of an aligned one
+};
+
+template <typename T, int N, int S, int TB, int OP>
+__global__ void __launch_bounds__((TB * TFof<N>())) k_zmul(ZmArgs<T> a) {
+  constexpr int E = Plan<N>::E, TF = N / E;
+  __shared__ cpx<T> sm[N * TB];
+  const int j = threadIdx.x / TB;
+  ColLds<T, TB, TB * TF == 64> lds{sm + threadIdx.x % TB};
+  const Geo& g = a.go.aligned ? a.go : a.gi;
+  const ZIdx id = zidx<TB>(g, g.aligned ? row_item(int(blockIdx.x), (g.ny + TB - 1) / TB, (g.nx / 2) / TB)
+                                        : int(blockIdx.x));
+  const cpx<T>* const in = a.in + spec_pos(a.gi, 0, id.ky, id.kx);
+  cpx<T>* const out = a.out + spec_pos(a.go, 0, id.ky, id.kx);
+  cpx<T> x[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) x[e] = ld_nt(in + (long long)(j + TF * e) * a.gi.pp);
+  if constexpr (OP != ZM_ONE) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int kz = j + TF * e;
+      if constexpr (OP == ZM_LAP) {
+        const int fy = fold(id.ky, g.ny), fz = fold(kz, g.nz);
+        const double c = g.kfac2, m = -(id.kx * id.kx * c + fy * fy * c + fz * fz * c);
+        x[e] = mk<T>(T(double(x[e].x) * m), T(double(x[e].y) * m));
+      } else {
+        const int k = OP == ZM_DX ? (id.kx == g.nx / 2 ? 0 : id.kx)
+                    : OP == ZM_DY ? (id.ky == g.ny / 2 ? 0 : sgnk(id.ky, g.ny)) : (kz == g.nz / 2 ? 0 : sgnk(kz, g.nz));
+        const double f = g.kfac;
+        x[e] = mk<T>(T(-(double(x[e].y) * f) * k), T((double(x[e].x) * f) * k));
+      }
+    }
+  }
+  fft<T, N, S>(x, j, a.tw, lds);
+  if (id.valid) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) out[(long long)(j + TF * e) * a.go.pp] = x[e];
   }
 }
 

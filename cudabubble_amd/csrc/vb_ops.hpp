@@ -105,6 +105,14 @@ struct SizeOps {
   // nullptr where a plane does not fit.  Its partials are one set per
   // workgroup: nz of them (PL_SUMS: nz / 2).
   void (*plane)(const PlaneArgs<T>& a, int mode, hipStream_t s);
+  // out of place z pass of a layout gi into a layout go, the input times op
+  // (ZmOp; sign < 0: ZM_ONE only)
+  void (*zmul)(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,
+               hipStream_t s);
+  // x and y transforms of whole planes in LDS (k_pair), real rows to half
+  // spectra times scl and back; nullptr where a plane does not fit
+  void (*pair_r2c)(const T* u, cpx<T>* so, double scl, const Geo& g, const cpx<T>* tw, hipStream_t s);
+  void (*pair_c2r)(const cpx<T>* si, T* uo, const Geo& g, const cpx<T>* tw, hipStream_t s);
 };
 
 // launch table of kernel schedule sc of length N (nullptr if not compiled),

@@ -204,4 +204,145 @@ __global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0,
   }
 }
 
+// ---------------------------------------------------------------------------
+// The x and y transforms of one real plane in LDS (the Calc level's r2c and
+// c2r): two real rows travel as one complex transform, and a row pair's storage
+// holds its N points or its two half spectra.  A 3-D transform is then this
+// kernel and a z pass, two sweeps of the data instead of three: 32^3 FP64
+// forward and back 45 -> 35 us with the copy of c2r's input gone as well, an
+// FP64 c2r at 128^3 about 31 -> 25 us.
+// ---------------------------------------------------------------------------
+template <typename T, int N>
+struct PairCfg {
+  static constexpr int V = (N == 128 || N == 192) ? 1 : (N == 48 || N == 96) ? 3 : 0;
+  static constexpr bool fits = N <= 128 || (N == 192 && sizeof(T) == 4);
+  static constexpr int E = fits ? Plan<N, V>::E : 8;
+  static constexpr int TF = N / E;
+  static constexpr int CW = fits ? 64 / TF : 1;                // columns, and row pairs, per wave
+  static constexpr int NA = 64 * ((N / 2 + CW) / CW);           // lanes for N / 2 + 1 columns
+  static constexpr int PS = N >= 96 ? 4 : 3;
+  static constexpr int LL = N + 2 + ((N + 1) >> PS);
+  static constexpr int bytes = N / 2 * LL * int(sizeof(cpx<T>)) + N * int(sizeof(cpx<T>));
+  static constexpr bool ok = fits && NA <= 1024 && bytes + 512 <= 160 * 1024;
+};
+
+// column kx of a plane of row pairs: position y is row y % 2 of pair y / 2
+template <typename T, int LL>
+struct PairCol {
+  cpx<T>* base;
+  int odd;   // offset of the odd row's slot
+  __device__ __forceinline__ cpx<T>& operator()(int pos) const { return base[(pos >> 1) * LL + (pos & 1) * odd]; }
+  __device__ __forceinline__ void sync() const { wave_sync(); }
+};
+
+template <typename T>
+struct PairArgs {
+  const T* u;          // real rows [nz][ny][nx] (r2c: in)
+  T* uo;               // (c2r: out)
+  const cpx<T>* si;    // half spectra, x and y transformed (c2r: in)
+  cpx<T>* so;          // (r2c: out, times scl)
+  const cpx<T>* tw;
+  Geo g;
+  double scl;
+};
+
+template <typename T, int N, int S>
+__global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_pair(PairArgs<T> a) {
+  using C = PairCfg<T, N>;
+  constexpr int E = C::E, TF = C::TF, LL = C::LL, PS = C::PS, V = C::V, CW = C::CW, H = N / 2;
+  static_assert(64 % TF == 0, "transforms inside a wave");
+  const Geo& g = a.g;
+  __shared__ cpx<T> sm[H * LL];
+  __shared__ cpx<T> tw[N];
+  const int z = int(blockIdx.x);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int cj = lane / CW, kx = wave * CW + lane % CW;    // column
+  const int r = threadIdx.x / TF, j = threadIdx.x % TF;    // row pair
+  PlaneRow<T, PS> row{sm + (r < H ? r : 0) * LL};
+  auto slot = [](int c) { return c + (c >> PS); };
+  const PairCol<T, LL> col{sm + slot(kx < H ? kx : N), kx < H ? slot(H + kx) - slot(kx) : slot(N + 1) - slot(N)};
+  const bool isrow = r < H, iscol = kx <= H;
+  cpx<T> x[E];
+  if constexpr (S < 0) {
+    if (isrow) {
+      const T* const u = a.u + ((long long)z * N + 2 * r) * N;
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = mk<T>(u[j + TF * e], u[N + j + TF * e]);
+    }
+    for (int i = threadIdx.x; i < N; i += C::NA) tw[i] = a.tw[i];
+    __syncthreads();
+    if (isrow) {
+      fft<T, N, -1, V>(x, j, tw, row);
+      constexpr int NH = H + 1, U = (NH + TF - 1) / TF;
+#pragma unroll
+      for (int e = 0; e < E; ++e) row(j + TF * e) = x[e];
+      row.sync();
+      cpx<T> ua[U], ub[U];
+      const T h = T(0.5) * T(a.scl);
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int k = j + TF * i;
+        if (k < NH) {
+          const cpx<T> zk = row(k), zm = row(k == 0 ? 0 : N - k);
+          ua[i] = mk<T>((zk.x + zm.x) * h, (zk.y - zm.y) * h);
+          ub[i] = mk<T>((zk.y + zm.y) * h, (zm.x - zk.x) * h);
+        }
+      }
+      row.sync();
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int k = j + TF * i;
+        if (k < NH) {
+          row(k == H ? N : k) = ua[i];
+          row(k == H ? N + 1 : H + k) = ub[i];
+        }
+      }
+    }
+    __syncthreads();
+    if (iscol) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = col(cj + TF * e);
+      col.sync();
+      fft<T, N, -1, V>(x, cj, tw, col);
+      cpx<T>* const o = a.so + (long long)z * g.pp;
+#pragma unroll
+      for (int e = 0; e < E; ++e) o[unsigned(plane_pos(g, cj + TF * e, kx))] = x[e];
+    }
+  } else {
+    if (iscol) {
+      const cpx<T>* const i0 = a.si + (long long)z * g.pp;
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = i0[unsigned(plane_pos(g, cj + TF * e, kx))];
+    }
+    for (int i = threadIdx.x; i < N; i += C::NA) tw[i] = a.tw[i];
+    __syncthreads();
+    if (iscol) {
+      fft<T, N, +1, V>(x, cj, tw, col);
+#pragma unroll
+      for (int e = 0; e < E; ++e) col(cj + TF * e) = x[e];
+    }
+    __syncthreads();
+    if (isrow) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int p = j + TF * e;
+        const bool mir = p > H;
+        const int k = mir ? N - p : p;
+        cpx<T> u = row(k == H ? N : k), w = row(k == H ? N + 1 : H + k);
+        if (k == 0 || k == H) { u.y = T(0); w.y = T(0); }
+        if (mir) { u.y = -u.y; w.y = -w.y; }
+        x[e] = mk<T>(u.x - w.y, u.y + w.x);
+      }
+      row.sync();
+      fft<T, N, +1, V>(x, j, tw, row);
+      T* const u = a.uo + ((long long)z * N + 2 * r) * N;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        u[j + TF * e] = x[e].x;
+        u[N + j + TF * e] = x[e].y;
+      }
+    }
+  }
+}
+
 }  // namespace vb

@@ -104,6 +104,32 @@ struct Launch {
     else
       hipLaunchKernelGGL((k_zpass<T, N, +1, TB>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
   }
+  static void zmul(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,
+                   hipStream_t s) {
+    const ZmArgs<T> a{in, out, tw, gi, go};
+    const dim3 gr(unsigned(zgroups(go.aligned ? go : gi, TB))), bl(YT);
+    if (sign < 0) {
+      hipLaunchKernelGGL((k_zmul<T, N, -1, TB, ZM_ONE>), gr, bl, 0, s, a);
+      return;
+    }
+    switch (op) {
+      case ZM_LAP: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_LAP>), gr, bl, 0, s, a); break;
+      case ZM_DX: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DX>), gr, bl, 0, s, a); break;
+      case ZM_DY: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DY>), gr, bl, 0, s, a); break;
+      case ZM_DZ: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DZ>), gr, bl, 0, s, a); break;
+      default: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_ONE>), gr, bl, 0, s, a); break;
+    }
+  }
+  static void pair_r2c(const T* u, cpx<T>* so, double scl, const Geo& g, const cpx<T>* tw, hipStream_t s) {
+    if constexpr (PairCfg<T, N>::ok)
+      hipLaunchKernelGGL((k_pair<T, N, -1>), dim3(unsigned(g.nz)), dim3(PairCfg<T, N>::NA), 0, s,
+                         (PairArgs<T>{u, nullptr, nullptr, so, tw, g, scl}));
+  }
+  static void pair_c2r(const cpx<T>* si, T* uo, const Geo& g, const cpx<T>* tw, hipStream_t s) {
+    if constexpr (PairCfg<T, N>::ok)
+      hipLaunchKernelGGL((k_pair<T, N, +1>), dim3(unsigned(g.nz)), dim3(PairCfg<T, N>::NA), 0, s,
+                         (PairArgs<T>{nullptr, uo, si, nullptr, tw, g, 1.0}));
+  }
   static void zlap(cpx<T>* b, const Geo& g, const cpx<T>* tw, const FinArgs* fin, hipStream_t s) {
     const int nf = fin_groups(fin);
     const dim3 gr(unsigned(zgroups(g, CB)) + unsigned(nf)), bl(CT);
@@ -231,6 +257,9 @@ struct Launch {
     o.zprep = &zprep;
     o.zstage = &zstage;
     o.plane = PlaneCfg<T, N>::ok ? &plane : nullptr;
+    o.zmul = &zmul;
+    o.pair_r2c = PairCfg<T, N>::ok ? &pair_r2c : nullptr;
+    o.pair_c2r = PairCfg<T, N>::ok ? &pair_c2r : nullptr;
     return o;
   }
 };

@@ -42,3 +42,48 @@ def test_prefix_in_one_kernel(vb, gpu, oracle_mod, nx, nz, prec):
     assert rel(V, Vo) < 10 * tol and rel(A, Ao) < 10 * tol
     if prec == "FP64":
         assert rel(Eb, Ebo) < 1e-11
+
+
+@pytest.mark.parametrize("nx,nz", [(16, 16), (48, 32), (96, 16), (128, 16), (192, 16), (256, 16)])
+def test_calc_operators_per_route(vb, gpu, oracle_mod, nx, nz):
+    """The Laplacians and gradients where x and y run as one kernel, and past it
+    (192 and 256 in FP64), and the integral of a length that no chunk divides."""
+    import torch
+    flush_print("calc", nx, nz)
+    eps = 2.0 * 2 * np.pi / nx
+    d, _ = vb.shape(vb.SHAPE_TORUS, 5, nx, nz, 1.0, eps)
+    o = oracle_mod.Oracle(nx, nz, eps=eps)
+    c = vb.Calc(nx, nz)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    real = lambda: torch.empty((nz, nx, nx), dtype=torch.float64, device=gpu)
+    fd = o.r2c(d)
+    # a transform rounds at ~5e-16 of the field, white over the modes; |k|^2 raises
+    # that by at most 3 (n/2)^2 / (1/eps^2) ~ 120 relative to the result: 6e-14
+    out, src = real(), T(fd)
+    c.lap_spec(src, out)
+    ref = o.lap_real(d)
+    assert rel_l2(out.cpu().numpy(), ref) < 1e-12
+    assert np.array_equal(src.cpu().numpy(), fd)
+    c.lap_real(T(d), out)
+    assert rel_l2(out.cpu().numpy(), ref) < 1e-12
+    g = [real() for _ in range(3)]
+    c.fftgradient(src, *g)
+    for a, b in zip(g, o.fftgradient(fd)):
+        assert rel_l2(a.cpu().numpy(), b) < 1e-12
+    assert rel(c.intf(T(d), 1.0, 0.5), o.intf(d, 1.0, 0.5)) < 1e-13
+
+
+@pytest.mark.parametrize("nx,nz", [(16, 32), (48, 16), (96, 96), (192, 16), (256, 16)])
+def test_calc_fp32_round_trip_per_route(vb, gpu, oracle_mod, nx, nz):
+    import torch
+    u = np.random.default_rng(nx).standard_normal((nz, nx, nx)).astype(np.float32)
+    c = vb.Calc(nx, nz, precision=vb.FP32_MIXED)
+    ud = torch.from_numpy(u).to(gpu)
+    s = torch.empty((nz, nx, nx // 2 + 1), dtype=torch.complex64, device=gpu)
+    c.r2c(ud, s)
+    assert rel_l2(s.cpu().numpy().astype(np.complex128), oracle_mod.Oracle(nx, nz).r2c(u.astype(np.float64))) < 2e-6
+    keep = s.clone()
+    back = torch.empty_like(ud)
+    c.c2r(s, back)
+    assert rel_l2(back.cpu().numpy(), u) < 2e-6
+    assert torch.equal(s, keep)
