@@ -52,8 +52,10 @@ __device__ __forceinline__ cpx<T> rot(cpx<T> a) {
 // only where measured to pay: 256 = 16 * 16, 128 = 16 * 8 and 192 = 24 * 8
 // for the FP32 column kernels and x kernels, 512 = 16 * 8 * 4 for the FP32 x
 // kernel.
-// V = 3 keeps V = 0's elements per thread with fewer passes (192 = 12 * 4 * 4,
-// the FP32 stage combines).  (V = 2, more threads per transform and fewer
+// V = 3 keeps V = 0's elements per thread with fewer passes (192 = 12 * 4 * 4 and
+// 384 = 12 * 4 * 4 * 2 for the FP32 stage combines, 48 = 12 * 4 and 96 = 12 * 4 *
+// 2 for the plane kernels).
+// (V = 2, more threads per transform and fewer
 // registers, measured slower at 256 and is not defined.)
 template <int N, int V = 0> struct Plan;
 template <> struct Plan<16, 0>  { static constexpr int E = 4,  NP = 2; static constexpr int R[2] = {4, 4}; };
@@ -71,6 +73,7 @@ template <> struct Plan<256, 1> { static constexpr int E = 16, NP = 2; static co
 template <> struct Plan<128, 1> { static constexpr int E = 16, NP = 2; static constexpr int R[2] = {16, 8}; };
 template <> struct Plan<512, 1> { static constexpr int E = 16, NP = 3; static constexpr int R[3] = {16, 8, 4}; };
 template <> struct Plan<192, 1> { static constexpr int E = 24, NP = 2; static constexpr int R[2] = {24, 8}; };
+template <> struct Plan<384, 3> { static constexpr int E = 12, NP = 4; static constexpr int R[4] = {12, 4, 4, 2}; };
 template <> struct Plan<48, 3>  { static constexpr int E = 12, NP = 2; static constexpr int R[2] = {12, 4}; };
 template <> struct Plan<96, 3>  { static constexpr int E = 12, NP = 3; static constexpr int R[3] = {12, 4, 2}; };
 template <> struct Plan<192, 3> { static constexpr int E = 12, NP = 3; static constexpr int R[3] = {12, 4, 4}; };

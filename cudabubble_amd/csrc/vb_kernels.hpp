@@ -685,6 +685,7 @@ struct YArgs {
   cpx<T>* o0;   // GM: out-of-place outputs in the z kernels' group-major layout
   cpx<T>* o1;
   int ztb;      // GM: the z kernels' column tile
+  int nzt;      // GM: planes of the whole grid (g may be a slab of it)
 };
 
 // Position of spectral element (z, ky, kx) in the group-major layout of the z
@@ -747,15 +748,17 @@ __global__ void __launch_bounds__((TB * TFof<N, V>())) k_ypass(YArgs<T> a0, cons
   if (id.valid) {
     if constexpr (GM) {
       cpx<T>* out = blockIdx.y ? a.o1 : a.o0;
+      Geo gt = g;
+      gt.nz = a.nzt;
       if (g.aligned && id.kx != g.nx / 2) {
         // ky = j + TF e: one ky step is one row of column groups of all z
-        cpx<T>* o = out + gm_index(g, a.ztb, id.z, j, id.kx);
-        const long long s = (long long)(((g.nx / 2) >> __builtin_ctz((unsigned)a.ztb)) * TF) * g.nz * a.ztb;
+        cpx<T>* o = out + gm_index(gt, a.ztb, id.z, j, id.kx);
+        const long long s = (long long)(((g.nx / 2) >> __builtin_ctz((unsigned)a.ztb)) * TF) * a.nzt * a.ztb;
 #pragma unroll
         for (int e = 0; e < E; ++e) o[e * s] = x[e];
       } else {
 #pragma unroll
-        for (int e = 0; e < E; ++e) out[gm_index(g, a.ztb, id.z, j + TF * e, id.kx)] = x[e];
+        for (int e = 0; e < E; ++e) out[gm_index(gt, a.ztb, id.z, j + TF * e, id.kx)] = x[e];
       }
     } else {
 #pragma unroll
@@ -1101,10 +1104,12 @@ struct ZsArgs {
 // Plan variant of the stage combines (see Plan): the default plan, except
 // FP32 at 192, 12 x 4 x 4 (two exchanges instead of three, the same 12
 // elements per thread; 218-240 registers against 205-226, two waves per SIMD
-// either way; 4 x 192^3 batched 3.61 -> 3.57 ms per step).  At 256 the
+// either way; 4 x 192^3 batched 3.61 -> 3.57 ms per step), and at 384, 12 x 4 x
+// 4 x 2 (three instead of four; a 384^3 step 8.52 -> 8.34 ms, the combines 539,
+// 499, 497 -> 499, 475, 476 us).  At 256 the
 // 16 x 16 plan needs 248-256 registers there and ran slower (stage 4 158 ->
 // 182 us), and so did 4 x 4 x 4 x 4 over 64 threads (100-128 registers).
-template <typename T, int N> constexpr int zsplan() { return (sizeof(T) == 4 && N == 192) ? 3 : 0; }
+template <typename T, int N> constexpr int zsplan() { return (sizeof(T) == 4 && (N == 192 || N == 384)) ? 3 : 0; }
 
 // LDS bytes of a stage combine: two column tiles for the transforms, or the
 // staged coefficient table, whichever is larger

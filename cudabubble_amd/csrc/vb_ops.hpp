@@ -90,8 +90,9 @@ struct SizeOps {
   // fin (or nullptr): integrals evaluated by extra workgroups of the launch
   void (*ypass)(cpx<T>* b0, cpx<T>* b1, int narr, int sign, const Geo& g, const cpx<T>* tw, const FinArgs* fin,
                 hipStream_t s);
-  // forward y pass of two arrays into the z kernels' group-major layout
-  void (*ypass_gm)(const cpx<T>* b0, const cpx<T>* b1, cpx<T>* o0, cpx<T>* o1, int ztb, const Geo& g,
+  // forward y pass of two arrays into the z kernels' group-major layout of a
+  // grid of nzt planes (g: the planes of b0, b1, which start at plane 0 of o0, o1)
+  void (*ypass_gm)(const cpx<T>* b0, const cpx<T>* b1, cpx<T>* o0, cpx<T>* o1, int ztb, int nzt, const Geo& g,
                    const cpx<T>* tw, const FinArgs* fin, hipStream_t s);
   void (*zpass)(cpx<T>* b, int sign, const Geo& g, const cpx<T>* tw, hipStream_t s);
   // fin (or nullptr): integrals evaluated by one extra workgroup of the launch

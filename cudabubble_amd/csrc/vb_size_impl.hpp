@@ -79,7 +79,7 @@ struct Launch {
     const int nf = fin_groups(fin);
     const int pad = ypad(g, nf);
     const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf + pad), unsigned(narr)), bl(CT);
-    YArgs<T> a{b0, b1, tw, g, fin ? *fin : FinArgs{}, nf, pad};
+    YArgs<T> a{b0, b1, tw, g, fin ? *fin : FinArgs{}, nf, pad, nullptr, nullptr, 0, g.nz};
     if (g_recorder) return record_launch(&launch_tab, sign < 0 ? OP_Y_FWD : OP_Y_INV, a, grid, bl);
     if (sign < 0)
       hipLaunchKernelGGL((k_ypass<T, N, -1, CB, false, CV>), grid, bl, 0, s, a, nullptr);
@@ -88,12 +88,12 @@ struct Launch {
   }
   // forward y pass of two arrays, written out of place in the z kernels'
   // group-major layout (column tile ztb)
-  static void ypass_gm(const cpx<T>* b0, const cpx<T>* b1, cpx<T>* o0, cpx<T>* o1, int ztb, const Geo& g,
+  static void ypass_gm(const cpx<T>* b0, const cpx<T>* b1, cpx<T>* o0, cpx<T>* o1, int ztb, int nzt, const Geo& g,
                        const cpx<T>* tw, const FinArgs* fin, hipStream_t s) {
     const int nf = fin_groups(fin);
     const int pad = ypad(g, nf);
     const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf + pad), 2u), bl(CT);
-    YArgs<T> a{const_cast<cpx<T>*>(b0), const_cast<cpx<T>*>(b1), tw, g, fin ? *fin : FinArgs{}, nf, pad, o0, o1, ztb};
+    YArgs<T> a{const_cast<cpx<T>*>(b0), const_cast<cpx<T>*>(b1), tw, g, fin ? *fin : FinArgs{}, nf, pad, o0, o1, ztb, nzt};
     if (g_recorder) return record_launch(&launch_tab, OP_Y_FWD_GM, a, grid, bl);
     hipLaunchKernelGGL((k_ypass<T, N, -1, CB, false, CV, true>), grid, bl, 0, s, a, nullptr);
   }
