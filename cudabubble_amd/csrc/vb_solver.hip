@@ -20,6 +20,7 @@
 #include <map>
 
 #include "vb_solver.hpp"
+#include "vb_staging.hpp"
 
 namespace vb {
 
@@ -134,6 +135,7 @@ struct Solver final : SolverBase {
   Phys ph{};
   hipStream_t st = nullptr;
   bool own_stream = false;
+  bool staging_counted = false;
   const SizeOps<T>* ox = nullptr;
   const SizeOps<T>* oz = nullptr;
   // FP64 operations (state transforms, FP64 queries in mixed mode)
@@ -334,9 +336,12 @@ struct Solver final : SolverBase {
     beta0 = beta;
     set_targets_device();
     VB_HIP(hipStreamSynchronize(st));
+    staging_user(1);
+    staging_counted = true;
   }
 
   ~Solver() override {
+    if (staging_counted) staging_user(-1);
     if (st) (void)hipStreamSynchronize(st);
     for (auto& G : graphs)
       if (G.x) (void)hipGraphExecDestroy(G.x);
@@ -1660,10 +1665,22 @@ struct Solver final : SolverBase {
     L("to_rows", [&] { relayout(uh[cur].p, oz->ytile, S.p, 0); });
     L("z_inv", [&] { ozd->zpass(S.p, +1, g, twzd.p, st); });
     L("y_inv", [&] { oxd->ypass(S.p, nullptr, 1, +1, g, twxd.p, nullptr, st); });
-    L("x_c2r", [&] { oxd->xc2r_d(S.p, phid.p, npairs, twxd.p, g, st); });
-    check_launch();
-    VB_HIP(hipMemcpyAsync(host, phid.p, sizeof(double) * (size_t)g.nr, hipMemcpyDeviceToHost, st));
-    VB_HIP(hipStreamSynchronize(st));
+    // the x kernel writes to pinned memory, a chunk of planes at a time
+    struct Rows2Host final : StagingJob {
+      Solver& s;
+      explicit Rows2Host(Solver& q) : s(q) {}
+      void produce(long long z0, long long nz, void* p) override {
+        s.L("x_c2r", [&] {
+          s.oxd->xc2r_d(s.S.p + z0 * s.g.pp, static_cast<double*>(p), nz * s.g.ny / 2, s.twxd.p, s.g, s.st);
+        });
+        s.check_launch();
+      }
+    } job(*this);
+    struct Held {
+      Staging* s;
+      ~Held() { staging_release(s); }
+    } held{staging_acquire(sizeof(double) * (size_t)g.nr)};
+    staging_copy_out(held.s, job, g.nz, sizeof(double) * (size_t)g.nx * g.ny, host, st);
   }
 
   void set_phi(const double* host) override {
