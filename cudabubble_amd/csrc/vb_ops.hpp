@@ -104,7 +104,9 @@ struct SizeOps {
   void (*zstage)(const ZsArgs<T>& a, int sch, int stg, hipStream_t s);
   // the prefix with a whole xy plane in LDS (vb_plane.hpp), mode: PlaneMode;
   // nullptr where a plane does not fit.  Its partials are one set per
-  // workgroup: nz of them (PL_SUMS: nz / 2).
+  // workgroup: nz of them (PL_SUMS: nz / sums_planes).
+  int sums_planes;
+  int plane_min_nz;   // the planes from which it is used
   void (*plane)(const PlaneArgs<T>& a, int mode, hipStream_t s);
   // out of place z pass of a layout gi into a layout go, the input times op
   // (ZmOp; sign < 0: ZM_ONE only)

@@ -345,4 +345,190 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_pair(PairArgs<T> a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The plane kernel where P and Q of a plane do not fit LDS together but one of
+// them does (FP64 at 128): the plane of P goes through y and x first, its v kept
+// in registers, then Q's, then the spectra of tmp1 and of s one after the other.
+// Two rows travel as one transform (k_pair's storage).  The same modes,
+// arguments and units as k_plane, but PL_SUMS takes one plane per workgroup.
+// One workgroup per CU and its phases in a row bound it, 45 us at 128^3 whether
+// 128 or 256 planes run; the three kernels take 50, and 100 for 256 planes: a
+// 128^3 FP64 drift step 627 -> 608 us, four of them batched 2026 -> 1607.  (FP32
+// at 192 fits as well but spills 78 registers: 76 us against 75.)
+// ---------------------------------------------------------------------------
+template <typename T, int N>
+struct Plane2Cfg {
+  static constexpr bool ok = sizeof(T) == 8 && N == 128;
+};
+
+// Planes from which the plane kernels are the faster ones: a workgroup's time
+// does not shrink with fewer of them.  128 x 128 x nz drift steps, plane kernels
+// against three kernels, us: FP32 nz = 16 237 / 186, 32 264 / 256, 64 343 / 345,
+// 128 416 / 459; FP64 nz = 64 (no drift) 273 / 190, 96 650 / 644, 128 608 / 627,
+// 192 878 / 1023.  At the shorter lengths they won at every depth measured (16
+// and up).
+template <typename T, int N> constexpr int plane_min_nz() { return Plane2Cfg<T, N>::ok ? 128 : N == 128 ? 64 : 0; }
+
+template <typename T, int N, int MODE, bool TAB = false>
+__global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0, const PlaneArgs<T>* tab) {
+  using C = PairCfg<T, N>;
+  constexpr int E = C::E, TF = C::TF, LL = C::LL, PS = C::PS, V = C::V, CW = C::CW, NA = C::NA, H = N / 2;
+  const PlaneArgs<T> a = TAB ? tab[blockIdx.z] : a0;
+  const Geo& g = a.g;
+  __shared__ cpx<T> sm[H * LL];
+  __shared__ cpx<T> tw[N];
+  constexpr int K = (MODE == PL_ETD && sizeof(T) == 4) ? 5 : 3;
+  __shared__ double red[K * (NA / 64)];
+  const int z = pair_item(int(blockIdx.x), int(gridDim.x));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int cj = lane / CW, kx = wave * CW + lane % CW;    // column
+  const int r = threadIdx.x / TF, j = threadIdx.x % TF;    // row pair
+  PlaneRow<T, PS> row{sm + (r < H ? r : 0) * LL};
+  auto slot = [](int c) { return c + (c >> PS); };
+  const PairCol<T, LL> col{sm + slot(kx < H ? kx : N), kx < H ? slot(H + kx) - slot(kx) : slot(N + 1) - slot(N)};
+  const bool isrow = r < H, iscol = kx <= H;
+  const long long pz = (long long)z * g.pp;
+
+  auto col_load = [&](cpx<T>* x, const cpx<T>* src) {
+    if (iscol) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = src[unsigned(plane_pos(g, cj + TF * e, kx))];
+    }
+  };
+  auto col_inv = [&](cpx<T>* x) {
+    if (iscol) {
+      fft<T, N, +1, V>(x, cj, tw, col);
+#pragma unroll
+      for (int e = 0; e < E; ++e) col(cj + TF * e) = x[e];
+    }
+  };
+  auto row_inv = [&](cpx<T>* x) {   // two real rows, as re and im
+    if (isrow) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int p = j + TF * e;
+        const bool mir = p > H;
+        const int k = mir ? N - p : p;
+        cpx<T> u = row(k == H ? N : k), w = row(k == H ? N + 1 : H + k);
+        if (k == 0 || k == H) { u.y = T(0); w.y = T(0); }
+        if (mir) { u.y = -u.y; w.y = -w.y; }
+        x[e] = mk<T>(u.x - w.y, u.y + w.x);
+      }
+      row.sync();
+      fft<T, N, +1, V>(x, j, tw, row);
+    }
+  };
+  // the plane of two real rows per lane group through x and y into out
+  auto forward = [&](cpx<T>* x, cpx<T>* out) {
+    if (isrow) {
+      constexpr int NH = H + 1, U = (NH + TF - 1) / TF;
+      fft<T, N, -1, V>(x, j, tw, row);
+#pragma unroll
+      for (int e = 0; e < E; ++e) row(j + TF * e) = x[e];
+      row.sync();
+      cpx<T> ua[U], ub[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int k = j + TF * i;
+        if (k < NH) {
+          const cpx<T> zk = row(k), zm = row(k == 0 ? 0 : N - k);
+          ua[i] = mk<T>(zk.x + zm.x, zk.y - zm.y);
+          ub[i] = mk<T>(zk.y + zm.y, zm.x - zk.x);
+        }
+      }
+      row.sync();
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int k = j + TF * i;
+        if (k < NH) {
+          row(k == H ? N : k) = ua[i];
+          row(k == H ? N + 1 : H + k) = ub[i];
+        }
+      }
+    }
+    __syncthreads();
+    if (iscol) {
+      cpx<T> y[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) y[e] = col(cj + TF * e);
+      col.sync();
+      fft<T, N, -1, V>(y, cj, tw, col);
+      if (g.aligned && kx < H) {
+        const unsigned o = unsigned(gm_index(g, a.ztb, z, cj, kx)),
+                       st = unsigned(((H >> __builtin_ctz((unsigned)a.ztb)) * TF) * g.nz * a.ztb);
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[o + e * st] = y[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[unsigned(gm_index(g, a.ztb, z, cj + TF * e, kx))] = y[e];
+      }
+    }
+  };
+
+  cpx<T> v[E], x[E];
+  col_load(x, a.P + pz);
+  for (int i = threadIdx.x; i < N; i += NA) tw[i] = a.tw[i];
+  __syncthreads();
+  col_inv(x);
+  __syncthreads();
+  if constexpr (MODE != PL_SUMS) {
+    row_inv(v);
+    col_load(x, a.Q + pz);
+    __syncthreads();   // the rows of P are read
+    col_inv(x);
+    __syncthreads();
+  }
+  row_inv(x);          // lap v (PL_SUMS: v)
+  double acc[K] = {};
+  if (isrow) {
+    const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps, D = a.D;
+    T ts[5] = {T(0), T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      T t1[2], sv[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if constexpr (MODE == PL_SUMS) {
+          const T q = h ? x[e].y : x[e].x;
+          const double w = double(q * q - T(1));
+          acc[0] += double(q);
+          acc[1] += w * w;
+        } else {
+          const T q = h ? v[e].y : v[e].x, lq = h ? x[e].y : x[e].x;
+          const T w = q * q - T(1);
+          const T f = -lq * T(eps) + w * q * T(ieps);                               // f_kernel, Calc.cu:160
+          t1[h] = q * (w - T(kappa));                                               // nld_kernel1, Calc.cu:270
+          sv[h] = T(D) * t1[h] + (T(3 * eps) * q * q - T(eps * (D + 1))) * f;       // Calc.cu:282, times eps^3
+          if constexpr (sizeof(T) == 4) {
+            ts[0] += q; ts[1] += w * w; ts[2] += f * f; ts[3] += t1[h]; ts[4] += sv[h];
+          } else {
+            acc[0] += double(q); acc[1] += double(w) * double(w); acc[2] += double(f) * double(f);
+          }
+        }
+      }
+      if constexpr (MODE == PL_ETD) {
+        v[e] = mk<T>(sv[0], sv[1]);
+        x[e] = mk<T>(t1[0], t1[1]);
+      }
+    }
+    if constexpr (MODE != PL_SUMS && sizeof(T) == 4) {
+#pragma unroll
+      for (int q = 0; q < K; ++q) acc[q] = double(ts[q]);
+    }
+  }
+  wave_part<K, NA>(acc, red);
+  if constexpr (MODE == PL_ETD) {
+    forward(x, a.U);     // its barrier orders the sums' too
+    __syncthreads();
+    forward(v, a.U2);
+  } else {
+    __syncthreads();
+  }
+  if (threadIdx.x < K) {
+    const double s = wave_total<NA>(red, threadIdx.x);
+    if (threadIdx.x < 3) a.part[3 * (long long)blockIdx.x + threadIdx.x] = s;
+    else if (a.dcpart) a.dcpart[2 * (long long)blockIdx.x + threadIdx.x - 3] = s;
+  }
+}
+
 }  // namespace vb

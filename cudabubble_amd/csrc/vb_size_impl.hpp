@@ -175,19 +175,28 @@ struct Launch {
 
   template <bool TAB>
   static void pl_launch(int mode, dim3 gr, const PlaneArgs<T>& a, const PlaneArgs<T>* tab, hipStream_t s) {
+    const dim3 bl(kPlaneThreads);
     if constexpr (PlaneCfg<T, N>::ok) {
-      const dim3 bl(PlaneCfg<T, N>::NA);
       if (mode == PL_ETD)
         hipLaunchKernelGGL((k_plane<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
       else if (mode == PL_SUMS)
         hipLaunchKernelGGL((k_plane<T, N, PL_SUMS, TAB>), gr, bl, 0, s, a, tab);
       else
         hipLaunchKernelGGL((k_plane<T, N, PL_ROWSUMS, TAB>), gr, bl, 0, s, a, tab);
+    } else if constexpr (Plane2Cfg<T, N>::ok) {
+      if (mode == PL_ETD)
+        hipLaunchKernelGGL((k_plane2<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
+      else if (mode == PL_SUMS)
+        hipLaunchKernelGGL((k_plane2<T, N, PL_SUMS, TAB>), gr, bl, 0, s, a, tab);
+      else
+        hipLaunchKernelGGL((k_plane2<T, N, PL_ROWSUMS, TAB>), gr, bl, 0, s, a, tab);
     }
   }
+  static constexpr int kPlaneThreads = PlaneCfg<T, N>::ok ? PlaneCfg<T, N>::NA : PairCfg<T, N>::NA;
+  static constexpr int kSumsPlanes = PlaneCfg<T, N>::ok ? 2 : 1;
   static void plane(const PlaneArgs<T>& a, int mode, hipStream_t s) {
-    const dim3 gr(unsigned(mode == PL_SUMS ? a.g.nz / 2 : a.g.nz));
-    if (g_recorder) return record_launch(&launch_tab, OP_PL_ETD + mode, a, gr, dim3(PlaneCfg<T, N>::NA));
+    const dim3 gr(unsigned(mode == PL_SUMS ? a.g.nz / kSumsPlanes : a.g.nz));
+    if (g_recorder) return record_launch(&launch_tab, OP_PL_ETD + mode, a, gr, dim3(kPlaneThreads));
     pl_launch<false>(mode, gr, a, nullptr, s);
   }
 
@@ -256,7 +265,9 @@ struct Launch {
     o.zlap = &zlap;
     o.zprep = &zprep;
     o.zstage = &zstage;
-    o.plane = PlaneCfg<T, N>::ok ? &plane : nullptr;
+    o.plane = PlaneCfg<T, N>::ok || Plane2Cfg<T, N>::ok ? &plane : nullptr;
+    o.sums_planes = kSumsPlanes;
+    o.plane_min_nz = plane_min_nz<T, N>();
     o.zmul = &zmul;
     o.pair_r2c = PairCfg<T, N>::ok ? &pair_r2c : nullptr;
     o.pair_c2r = PairCfg<T, N>::ok ? &pair_c2r : nullptr;

@@ -515,6 +515,10 @@ struct Solver final : SolverBase {
     kept = true;
   }
 
+  // whether a whole plane at a time is the way (SizeOps::plane)
+  template <typename X>
+  bool by_plane(const SizeOps<X>* o) const { return o->plane && g.nz >= o->plane_min_nz; }
+
   // one plane kernel over the prepared field (PlaneMode)
   void plane(int mode, cpx<T>* tt, cpx<T>* ts) {
     PlaneArgs<T> a{};
@@ -530,7 +534,7 @@ struct Solver final : SolverBase {
     a.eps = p.eps;
     a.kappa = p.kappa;
     a.D = p.D;
-    nxlast = mode == PL_SUMS ? g.nz / 2 : g.nz;
+    nxlast = mode == PL_SUMS ? g.nz / ox->sums_planes : g.nz;
     L(mode == PL_SUMS ? "plane_sums" : "plane", [&] { ox->plane(a, mode, st); });
   }
 
@@ -548,7 +552,7 @@ struct Solver final : SolverBase {
     cpx<T>* tt = set ? Tt1.p : Tt.p;
     cpx<T>* ts = set ? Ts1.p : Ts.p;
     kept = false;
-    if (ox->plane && !withf) {
+    if (by_plane(ox) && !withf) {
       plane(PL_ETD, tt, ts);
       if (defer) {
         fin_pending = true;
@@ -635,7 +639,7 @@ struct Solver final : SolverBase {
   // y-inverse of P, the partial sums of v and (v^2-1)^2, and the finalize
   // kernel.  Used where only the targets' drift is needed.
   void prefix_integrals(int mode, int fold) {
-    if (ox->plane) {
+    if (by_plane(ox)) {
       plane(PL_SUMS, nullptr, nullptr);
       refinalize(mode, nxlast, fold);
       prepped = prefixed = prefixed_f = false;
@@ -1586,7 +1590,7 @@ struct Solver final : SolverBase {
     }
     L("zprep64", [&] { ozd->zprep(src, P64.p, Q64.p, zpart64.p, dc64.p, g, twzd.p, st); });
     int nx64 = nxb64;
-    if (oxd->plane) {
+    if (by_plane(oxd)) {
       PlaneArgs<double> a{};
       a.P = P64.p;
       a.Q = Q64.p;

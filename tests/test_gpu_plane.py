@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("prec", ["FP64", "FP32_MIXED"])
 @pytest.mark.parametrize("nx,nz", [(16, 16), (16, 48), (32, 16), (32, 32), (48, 48), (48, 16), (64, 16), (64, 96),
-                                   (96, 16), (96, 48), (128, 16), (128, 32)])
+                                   (96, 16), (96, 48), (128, 48), (128, 64), (128, 128)])
 def test_prefix_in_one_kernel(vb, gpu, oracle_mod, nx, nz, prec):
     flush_print("plane", nx, nz, prec)
     eps = 2.0 * 2 * np.pi / nx
