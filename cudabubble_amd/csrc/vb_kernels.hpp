@@ -262,7 +262,7 @@ struct XaArgs {
   const cpx<T>* Q;   // x-half-spectra of lap v
   T* v;
   T* f;
-  cpx<T>* Tt;        // out: x-forward of tmp1, times inv_n (k_xrow: doubled, unnormalised)
+  cpx<T>* Tt;        // out (k_xrow): x-forward of tmp1, doubled, unnormalised
   cpx<T>* W;         // out (Euler only): x-forward of f, times inv_n
   cpx<T>* Ts;        // out (k_xrow): x-forward of eps^3 s, doubled, unnormalised
   double* part;      // [gridDim.x][3]
@@ -276,9 +276,9 @@ struct XaArgs {
 // Every pipeline kernel takes its argument struct by value, or (TAB, a
 // batched launch over the solves of a size group) from a per-solve table in
 // device memory indexed by blockIdx.z.
-// k_xa: the x kernel of the Euler paths (WITHF: v, f and the x-forward of f
-// as well); partial sums and the x-forward of tmp1, two rows per lane.
-template <typename T, int N, bool WITHF, bool TAB = false>
+// k_xa: the x kernel of the Euler paths: v, f and the x-forward of f, and the
+// partial sums, two rows per lane.
+template <typename T, int N, bool TAB = false>
 __global__ void __launch_bounds__(XWG, (xwaves<T>())) k_xa(XaArgs<T> a0, const XaArgs<T>* tab) {
   const XaArgs<T> a = TAB ? tab[blockIdx.z] : a0;
   constexpr int XP = xplan<T, N>(), E = Plan<N, XP>::E, TF = N / E, G = xlanes<T, N>(), LL = row_lds_len<N>(), NH = N / 2 + 1;
@@ -294,11 +294,9 @@ __global__ void __launch_bounds__(XWG, (xwaves<T>())) k_xa(XaArgs<T> a0, const X
   // the pointwise terms multiply by 1/eps instead of dividing (within an ulp
   // of the reference's quotients; an FP64 division per point is a long
   // instruction sequence that these kernels cannot hide)
-  const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps;
-  const double D = a.D, ie2 = ieps * ieps, ie3 = ie2 * ieps;
+  const double eps = a.eps, ieps = 1.0 / eps;
   double acc[3] = {0.0, 0.0, 0.0};
-  T tm[2][E];
-  T ff[WITHF ? 2 : 1][E];
+  T ff[2][E];
   {
     cpx<T> x[2][E];
 #pragma unroll
@@ -318,28 +316,16 @@ __global__ void __launch_bounds__(XWG, (xwaves<T>())) k_xa(XaArgs<T> a0, const X
         const double v = double(x[h][e].x), lv = double(x[h][e].y);
         const double w = v * v - 1.0;
         const double f = -lv * eps + w * v * ieps;         // f_kernel, Calc.cu:160
-        const double t1 = v * (v * v - 1.0 - kappa);       // nld_kernel1, Calc.cu:270
         if (valid) {
           acc[0] += v; acc[1] += w * w; acc[2] += f * f;
-          if constexpr (WITHF) {   // the Euler update reads v and f back
-            a.v[r * N + p] = T(v);
-            a.f[r * N + p] = T(f);
-          }
+          a.v[r * N + p] = T(v);   // the Euler update reads v and f back
+          a.f[r * N + p] = T(f);
         }
-        tm[h][e] = T(t1);
-        if constexpr (WITHF) ff[h][e] = T(f);
+        ff[h][e] = T(f);
       }
     }
   }
   {
-    cpx<T> z[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) z[e] = mk<T>(tm[0][e], tm[1][e]);
-    fft<T, N, -1, XP>(z, j, a.tw, lds);
-    unpack_store<T, N, XP>(z, j, lds, a.Tt + a.rl.off(r0), a.Tt + a.rl.nyq(r0, N / 2), a.Tt + a.rl.off(r0 + 1),
-                           a.Tt + a.rl.nyq(r0 + 1, N / 2), T(a.inv_n), valid);
-  }
-  if constexpr (WITHF) {
     cpx<T> z[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) z[e] = mk<T>(ff[0][e], ff[1][e]);
@@ -1049,6 +1035,40 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zprep(ZprArgs<T> a0, const
 #pragma unroll
   for (int e = 0; e < E; ++e) next_field_elem<T>(u[e].x, u[e].y, j + TF * e, id, g, acc, x[e], y[e]);
   next_field_tail<T, N, TB, 0>(x, y, acc, j, id, g, lds, lds2, tw, a.P, a.Q, a.part, red, tile);
+}
+
+// After an Euler update: the z-forward of W (x and y transformed, row layout)
+// is the new state, stored widened to FP64 and group-major, and its P, Q follow
+// as in k_zprep (one kernel where the z pass, the relayout and k_zprep were
+// three).
+template <typename T, int N, int TB>
+__global__ void __launch_bounds__((TB * TFof<N>())) k_zeuler(const cpx<T>* __restrict__ W, cpx<double>* __restrict__ uh,
+                                                             ZprArgs<T> a) {
+  constexpr int E = Plan<N>::E, TF = N / E;
+  constexpr bool WAVE = TB * TF == 64;
+  const Geo& g = a.g;
+  __shared__ cpx<T> sm[2 * N * TB];
+  __shared__ double red[(TB * TF) / 64];
+  const int j = threadIdx.x / TB;
+  ColLds<T, TB, WAVE> lds{sm + threadIdx.x % TB};
+  ColLds<T, TB, WAVE> lds2{sm + N * TB + threadIdx.x % TB};
+  const int tile = pair_item(int(blockIdx.x), int(gridDim.x));
+  const ZIdx id = zidx<TB>(g, tile);
+  cpx<T> x[E], y[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) x[e] = W[id.q + (long long)(j + TF * e) * g.pp];
+  fft<T, N, -1>(x, j, a.tw, lds);
+  const long long ib0 = (long long)tile * N * TB + threadIdx.x % TB;
+  double acc = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const double re = double(x[e].x), im = double(x[e].y);
+    if (id.valid) uh[ib0 + (long long)(j + TF * e) * TB] = mk<double>(re, im);
+    if (id.valid && id.q == 0 && j == 0 && e == 0) a.dc[0] = re;
+    next_field_elem<T>(re, im, j + TF * e, id, g, acc, x[e], y[e]);
+  }
+  lds.sync();   // the forward transform's last reads
+  next_field_tail<T, N, TB, 0>(x, y, acc, j, id, g, lds, lds2, a.tw, a.P, a.Q, a.part, red, tile);
 }
 
 template <typename T>

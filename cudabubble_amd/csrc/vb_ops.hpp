@@ -27,7 +27,7 @@ enum PipeOp {
 // (from P alone: k_xsums)
 enum XaMode { XA_ROWSUMS = 0, XA_WITHF = 1, XA_WITHS = 2, XA_SUMS = 3 };
 // modes of the plane kernel (k_plane)
-enum PlaneMode { PL_ETD = 0, PL_SUMS = 1, PL_ROWSUMS = 2 };
+enum PlaneMode { PL_ETD = 0, PL_SUMS = 1, PL_ROWSUMS = 2, PL_EULER = 3 };
 struct RecLaunch {
   // issues the table form of the recorded kernel over `lanes` solves
   void (*launch_tab)(int op, const void* tab, dim3 grid, dim3 block, int lanes, hipStream_t s);
@@ -64,6 +64,10 @@ struct PlaneArgs {
   Geo g;
   int ztb, pad;
   double eps, kappa, D;
+  T* v;              // PL_EULER out: the real fields v and f, and the x,y-forward
+  T* f;              // of f times inv_n in the row layout
+  cpx<T>* W;
+  double inv_n;
 };
 
 template <typename T> struct XaArgs;
@@ -106,8 +110,15 @@ struct SizeOps {
   // nullptr where a plane does not fit.  Its partials are one set per
   // workgroup: nz of them (PL_SUMS: nz / sums_planes).
   int sums_planes;
+  bool plane_euler;   // it has the mode PL_EULER
   int plane_min_nz;   // the planes from which it is used
   void (*plane)(const PlaneArgs<T>& a, int mode, hipStream_t s);
+  // The Forward-Euler update with x and y of a plane in one kernel (nullptr
+  // where a plane does not fit; nz partials of rhs^2), and the z pass that
+  // follows it: the new state from W, and the prepared field's P, Q
+  void (*xe_plane)(const XeArgs<T>& a, const Geo& g, hipStream_t s);
+  void (*zeuler)(const cpx<T>* W, cpx<double>* uh, cpx<T>* P, cpx<T>* Q, double* part, double* dc, const Geo& g,
+                 const cpx<T>* tw, hipStream_t s);
   // out of place z pass of a layout gi into a layout go, the input times op
   // (ZmOp; sign < 0: ZM_ONE only)
   void (*zmul)(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,

@@ -46,7 +46,9 @@ __device__ __forceinline__ int plane_pos(const Geo& g, int ky, int kx) {
 }
 
 // PL_ETD: the prefix of a stage (k_ypass, k_xrow and the group-major k_ypass
-// in one; the same terms and units as k_xrow).  PL_ROWSUMS: the partial sums
+// in one; the same terms and units as k_xrow).  PL_EULER: the Euler paths'
+// (k_ypass, k_xa and the y-forward of f): v and f stored, pointwise terms in
+// FP64 as in k_xa.  PL_ROWSUMS: the partial sums
 // of v, (v^2-1)^2 and f^2 only.  PL_SUMS: the partial sums of v and (v^2-1)^2
 // from P alone, two planes per workgroup, the second in Q's place.
 template <typename T, int N, int MODE, bool TAB = false>
@@ -125,6 +127,13 @@ __global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0,
         const double w0 = double(v0 * v0 - T(1)), w1 = double(v1 * v1 - T(1));
         acc[0] += double(v0) + double(v1);
         acc[1] += w0 * w0 + w1 * w1;
+      } else if constexpr (MODE == PL_EULER) {
+        const double v = double(x[e].x), lv = double(x[e].y), w = v * v - 1.0, f = -lv * eps + w * v * ieps;
+        acc[0] += v; acc[1] += w * w; acc[2] += f * f;
+        const long long i = ((long long)z * N + r) * N + j + TF * e;
+        a.v[i] = T(v);
+        a.f[i] = T(f);
+        x[e] = mk<T>(T(f), T(0));
       } else {
         const T v = x[e].x, lv = x[e].y;
         const T w = v * v - T(1);
@@ -139,11 +148,11 @@ __global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0,
         x[e] = mk<T>(t1, sv);
       }
     }
-    if constexpr (MODE != PL_SUMS && sizeof(T) == 4) {
+    if constexpr ((MODE == PL_ETD || MODE == PL_ROWSUMS) && sizeof(T) == 4) {
 #pragma unroll
       for (int q = 0; q < K; ++q) acc[q] = double(ts[q]);
     }
-    if constexpr (MODE == PL_ETD) {
+    if constexpr (MODE == PL_ETD || MODE == PL_EULER) {
       constexpr int NH = H + 1, U = (NH + TF - 1) / TF;
       fft<T, N, -1, V>(x, j, tw, row);
 #pragma unroll
@@ -158,6 +167,7 @@ __global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0,
           const cpx<T> zk = row(k), zm = row(k == 0 ? 0 : N - k);
           ua[i] = mk<T>(zk.x + zm.x, zk.y - zm.y);
           ub[i] = mk<T>(zk.y + zm.y, zm.x - zk.x);
+          if constexpr (MODE == PL_EULER) ua[i] = scale(ua[i], T(0.5) * T(a.inv_n));
         }
       }
       row.sync();
@@ -166,7 +176,7 @@ __global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0,
         const int k = j + TF * i;
         if (k < NH) {
           row(k == H ? N : k) = ua[i];
-          row(k == H ? N + 1 : H + k) = ub[i];
+          if constexpr (MODE == PL_ETD) row(k == H ? N + 1 : H + k) = ub[i];
         }
       }
     }
@@ -177,6 +187,21 @@ __global__ void __launch_bounds__((PlaneCfg<T, N>::NA)) k_plane(PlaneArgs<T> a0,
     const double s = wave_total<NA>(red, threadIdx.x);
     if (threadIdx.x < 3) a.part[3 * (long long)blockIdx.x + threadIdx.x] = s;
     else if (a.dcpart) a.dcpart[2 * (long long)blockIdx.x + threadIdx.x - 3] = s;
+  }
+  if constexpr (MODE == PL_EULER) {
+    auto fwd = [&](int c) {   // f's columns: kx = c, or Nyquist
+      PlaneCol<T, LL> col{sm + slot(c)};
+      cpx<T> x[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = col(cj + TF * e);
+      col.sync();
+      fft<T, N, -1, V>(x, cj, tw, col);
+      cpx<T>* const o = a.W + (long long)z * g.pp;
+#pragma unroll
+      for (int e = 0; e < E; ++e) o[unsigned(plane_pos(g, cj + TF * e, c < H ? c : H))] = x[e];
+    };
+    if (act && (cc < H || cc == N)) fwd(cc);
+    if (!C::XW && wave == 0 && lane % CW == 0) fwd(N);
   }
   if constexpr (MODE == PL_ETD) {
     auto fwd = [&](int c) {
@@ -528,6 +553,125 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
     const double s = wave_total<NA>(red, threadIdx.x);
     if (threadIdx.x < 3) a.part[3 * (long long)blockIdx.x + threadIdx.x] = s;
     else if (a.dcpart) a.dcpart[2 * (long long)blockIdx.x + threadIdx.x - 3] = s;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The Forward-Euler update of a plane in LDS: the y and x inverse of W (x and y
+// spectra of lap f), k_xe's update, the x and y forward of the new field over W.
+// With PL_EULER and k_zeuler a fixed-dt Euler step is four kernels instead of
+// ten: 64^3 FP64 53 -> 33 us, 32^3 FP32 38 -> 19, 128^3 FP32 98 -> 68.
+// ---------------------------------------------------------------------------
+template <typename T, int N>
+__global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_xe_plane(XeArgs<T> a, Geo g) {
+  using C = PairCfg<T, N>;
+  constexpr int E = C::E, TF = C::TF, LL = C::LL, PS = C::PS, V = C::V, CW = C::CW, NA = C::NA, H = N / 2;
+  __shared__ cpx<T> sm[H * LL];
+  __shared__ cpx<T> tw[N];
+  __shared__ double red[NA / 64];
+  const int z = int(blockIdx.x);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int cj = lane / CW, kx = wave * CW + lane % CW;    // column
+  const int r = threadIdx.x / TF, j = threadIdx.x % TF;    // row pair
+  PlaneRow<T, PS> row{sm + (r < H ? r : 0) * LL};
+  auto slot = [](int c) { return c + (c >> PS); };
+  const PairCol<T, LL> col{sm + slot(kx < H ? kx : N), kx < H ? slot(H + kx) - slot(kx) : slot(N + 1) - slot(N)};
+  const bool isrow = r < H, iscol = kx <= H;
+  const long long r0 = ((long long)z * N + 2 * r) * N;
+  cpx<T> x[E];
+  T v[2][E], f[2][E];
+  if (iscol) {
+    const cpx<T>* const i0 = a.W + (long long)z * g.pp;
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = i0[unsigned(plane_pos(g, cj + TF * e, kx))];
+  }
+  if (isrow) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        v[h][e] = a.v[r0 + h * N + j + TF * e];
+        f[h][e] = a.f[r0 + h * N + j + TF * e];
+      }
+    }
+  }
+  const double l1 = a.sc->l1, l2 = a.sc->l2, eta = a.eta, eps = a.eps, t = a.tp ? *a.tp : a.t, ie2 = 1.0 / (eps * eps);
+  for (int i = threadIdx.x; i < N; i += NA) tw[i] = a.tw[i];
+  __syncthreads();
+  if (iscol) {
+    fft<T, N, +1, V>(x, cj, tw, col);
+#pragma unroll
+    for (int e = 0; e < E; ++e) col(cj + TF * e) = x[e];
+  }
+  __syncthreads();
+  double acc[1] = {0.0};
+  if (isrow) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int p = j + TF * e;
+      const bool mir = p > H;
+      const int k = mir ? N - p : p;
+      cpx<T> u = row(k == H ? N : k), w = row(k == H ? N + 1 : H + k);
+      if (k == 0 || k == H) { u.y = T(0); w.y = T(0); }
+      if (mir) { u.y = -u.y; w.y = -w.y; }
+      x[e] = mk<T>(u.x - w.y, u.y + w.x);
+    }
+    row.sync();
+    fft<T, N, +1, V>(x, j, tw, row);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      double nv[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double lf = double(h ? x[e].y : x[e].x), vv = double(v[h][e]), ff = double(f[h][e]);
+        const double g0 = -lf + (3.0 * vv * vv - 1.0) * ff * ie2;           // Calc.cu:178
+        const double rhs = a.shape ? g0 : l1 * 0.5 + l2 * ff + g0 * eta;    // Calc.cu:417
+        nv[h] = vv + t * rhs;                                               // Calc.cu:400
+        acc[0] += rhs * rhs;
+      }
+      x[e] = mk<T>(T(nv[0]), T(nv[1]));
+    }
+  }
+  if (a.part) {   // uniform over the grid: the residual sum only
+    block_sum_store<1, NA>(acc, red, a.part + blockIdx.x);
+    return;
+  }
+  if (isrow) {
+    fft<T, N, -1, V>(x, j, tw, row);
+    constexpr int NH = H + 1, U = (NH + TF - 1) / TF;
+#pragma unroll
+    for (int e = 0; e < E; ++e) row(j + TF * e) = x[e];
+    row.sync();
+    cpx<T> ua[U], ub[U];
+    const T h = T(0.5) * T(a.inv_n);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int k = j + TF * i;
+      if (k < NH) {
+        const cpx<T> zk = row(k), zm = row(k == 0 ? 0 : N - k);
+        ua[i] = mk<T>((zk.x + zm.x) * h, (zk.y - zm.y) * h);
+        ub[i] = mk<T>((zk.y + zm.y) * h, (zm.x - zk.x) * h);
+      }
+    }
+    row.sync();
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int k = j + TF * i;
+      if (k < NH) {
+        row(k == H ? N : k) = ua[i];
+        row(k == H ? N + 1 : H + k) = ub[i];
+      }
+    }
+  }
+  __syncthreads();
+  if (iscol) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = col(cj + TF * e);
+    col.sync();
+    fft<T, N, -1, V>(x, cj, tw, col);
+    cpx<T>* const o = a.out + (long long)z * g.pp;
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[unsigned(plane_pos(g, cj + TF * e, kx))] = x[e];
   }
 }
 

@@ -60,7 +60,7 @@ struct Launch {
       return record_launch(&launch_tab, op, a, gr, bl);
     }
     if (mode == XA_WITHF)
-      hipLaunchKernelGGL((k_xa<T, N, true>), gr, bl, 0, s, a, nullptr);
+      hipLaunchKernelGGL((k_xa<T, N>), gr, bl, 0, s, a, nullptr);
     else if (mode == XA_WITHS)
       hipLaunchKernelGGL((k_xrow<T, N, false, XR>), gr, bl, 0, s, a, nullptr);
     else if (mode == XA_SUMS)
@@ -103,6 +103,17 @@ struct Launch {
       hipLaunchKernelGGL((k_zpass<T, N, -1, TB>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
     else
       hipLaunchKernelGGL((k_zpass<T, N, +1, TB>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
+  }
+  // (FP32 at 192 would spill its 24 elements' v and f: a step 199 -> 209 us)
+  static constexpr bool kXePlane = PairCfg<T, N>::ok && N <= 128;
+  static void xe_plane(const XeArgs<T>& a, const Geo& g, hipStream_t s) {
+    if constexpr (kXePlane)
+      hipLaunchKernelGGL((k_xe_plane<T, N>), dim3(unsigned(g.nz)), dim3(PairCfg<T, N>::NA), 0, s, a, g);
+  }
+  static void zeuler(const cpx<T>* W, cpx<double>* uh, cpx<T>* P, cpx<T>* Q, double* part, double* dc, const Geo& g,
+                     const cpx<T>* tw, hipStream_t s) {
+    hipLaunchKernelGGL((k_zeuler<T, N, TB>), dim3(zgrid(g)), dim3(YT), 0, s, W, uh,
+                       (ZprArgs<T>{nullptr, P, Q, part, dc, tw, g}));
   }
   static void zmul(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,
                    hipStream_t s) {
@@ -177,6 +188,10 @@ struct Launch {
   static void pl_launch(int mode, dim3 gr, const PlaneArgs<T>& a, const PlaneArgs<T>* tab, hipStream_t s) {
     const dim3 bl(kPlaneThreads);
     if constexpr (PlaneCfg<T, N>::ok) {
+      if (!TAB && mode == PL_EULER) {
+        hipLaunchKernelGGL((k_plane<T, N, PL_EULER>), gr, bl, 0, s, a, nullptr);
+        return;
+      }
       if (mode == PL_ETD)
         hipLaunchKernelGGL((k_plane<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
       else if (mode == PL_SUMS)
@@ -207,7 +222,7 @@ struct Launch {
       case OP_XA_RS:
         hipLaunchKernelGGL((k_xrow<T, N, true, XR, true>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab);
         break;
-      case OP_XA_F: hipLaunchKernelGGL((k_xa<T, N, true, true>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab); break;
+      case OP_XA_F: hipLaunchKernelGGL((k_xa<T, N, true>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab); break;
       case OP_XA_S:
         hipLaunchKernelGGL((k_xrow<T, N, true, XR>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab);
         break;
@@ -268,6 +283,9 @@ struct Launch {
     o.plane = PlaneCfg<T, N>::ok || Plane2Cfg<T, N>::ok ? &plane : nullptr;
     o.sums_planes = kSumsPlanes;
     o.plane_min_nz = plane_min_nz<T, N>();
+    o.plane_euler = PlaneCfg<T, N>::ok;
+    o.xe_plane = kXePlane ? &xe_plane : nullptr;
+    o.zeuler = &zeuler;
     o.zmul = &zmul;
     o.pair_r2c = PairCfg<T, N>::ok ? &pair_r2c : nullptr;
     o.pair_c2r = PairCfg<T, N>::ok ? &pair_c2r : nullptr;

@@ -503,10 +503,12 @@ struct Solver final : SolverBase {
 
   // fin: integrals to evaluate in the same launch as the z pass (extra
   // workgroups of it), or nullptr
-  void spectral_lap(cpx<T>* b, const FinArgs* fin) {
-    L("y_fwd", [&] { ox->ypass(b, nullptr, 1, -1, g, twx.p, nullptr, st); });
+  // W of the Euler prefix: f's x spectra, or (y_done) x and y, to those of lap f
+  // (with k_xe_plane, which does the y-inverse, its x and y spectra)
+  void spectral_lap(cpx<T>* b, const FinArgs* fin, bool y_done) {
+    if (!y_done) L("y_fwd", [&] { ox->ypass(b, nullptr, 1, -1, g, twx.p, nullptr, st); });
     L(fin ? "z_lap_fin" : "z_lap", [&] { oz->zlap(b, g, twz.p, fin, st); });
-    L("y_inv", [&] { ox->ypass(b, nullptr, 1, +1, g, twx.p, nullptr, st); });
+    if (!ox->xe_plane) L("y_inv", [&] { ox->ypass(b, nullptr, 1, +1, g, twx.p, nullptr, st); });
   }
 
   void fold_keep(FinArgs& fin) {
@@ -534,8 +536,12 @@ struct Solver final : SolverBase {
     a.eps = p.eps;
     a.kappa = p.kappa;
     a.D = p.D;
+    a.v = v.p;
+    a.f = f.p;
+    a.W = W.p;
+    a.inv_n = 1.0 / double(g.nr);
     nxlast = mode == PL_SUMS ? g.nz / ox->sums_planes : g.nz;
-    L(mode == PL_SUMS ? "plane_sums" : "plane", [&] { ox->plane(a, mode, st); });
+    L(mode == PL_SUMS ? "plane_sums" : mode == PL_EULER ? "plane_f" : "plane", [&] { ox->plane(a, mode, st); });
   }
 
   // The prefix of the prepared stage field (P, Q: its z-inverse spectra and
@@ -585,15 +591,18 @@ struct Solver final : SolverBase {
     // FP32-mixed ETD prefix: FP64 sums of tmp1 and eps^3 s for the k = 0 modes
     fin.dcpart = (kMixed && !withf) ? xdc.p : nullptr;
     if (keep) fold_keep(fin);
-    if (withf) {
+    if (withf && by_plane(ox) && ox->plane_euler) {
+      plane(PL_EULER, nullptr, nullptr);
+      fin.nxb = nxlast;
+      spectral_lap(W.p, &fin, true);
+    } else if (withf) {
       L("y_inv2", [&] { ox->ypass(P.p, Q.p, 2, +1, g, twx.p, nullptr, st); });
       a.P = P.p;
       a.Q = Q.p;
-      a.Tt = tt;
       a.part = xpart.p;
       a.npairs = npairs;
       L("xa_f", [&] { ox->xa(a, XA_WITHF, st); });
-      spectral_lap(W.p, &fin);
+      spectral_lap(W.p, &fin, false);
     } else {
       const int ns = slabs(), nzs = g.nz / ns;
       Geo gs = g;
@@ -749,7 +758,8 @@ struct Solver final : SolverBase {
     return out;
   }
 
-  // Forward-Euler update of uh[cur] into uh[1-cur] with rhs g0 (shape) or nld1;
+  // Forward-Euler update of uh[cur] into uh[1-cur] with rhs g0 (shape) or nld1,
+  // leaving P, Q prepared for the new state;
   // tdev non-null: the step is read from there on the device instead of t
   int euler(double t, bool shape, const double* tdev = nullptr) {
     ensure_prefixed(true);
@@ -770,12 +780,16 @@ struct Solver final : SolverBase {
     e.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
     e.part = nullptr;
     e.tp = tdev;
-    L("xe", [&] { ox->xe(e, st); });
-    L("y_fwd", [&] { ox->ypass(W.p, nullptr, 1, -1, g, twx.p, nullptr, st); });
-    L("z_fwd", [&] { oz->zpass(W.p, -1, g, twz.p, st); });
-    L("widen", [&] {
-      relayout(W.p, 0, uh[out].p, oz->ytile);
-    });
+    if (ox->xe_plane) {
+      L("xe_plane", [&] { ox->xe_plane(e, g, st); });
+    } else {
+      L("xe", [&] { ox->xe(e, st); });
+      L("y_fwd", [&] { ox->ypass(W.p, nullptr, 1, -1, g, twx.p, nullptr, st); });
+    }
+    // the new state, and P, Q prepared for it
+    L("z_euler", [&] { oz->zeuler(W.p, uh[out].p, P.p, Q.p, zpart.p, dc.p, g, twz.p, st); });
+    zhalf = 0;
+    prepped = true;
     check_launch();
     prefixed_f = false;   // W was consumed
     return out;
@@ -1312,9 +1326,7 @@ struct Solver final : SolverBase {
   DBuf<double> euler_t;
   void euler_attempt(double t, bool shape) {
     auto body = [&](bool tdev) {
-      const int out = euler(t, shape, tdev ? euler_t.p : nullptr);
-      prep(uh[out].p);
-      cur = out;
+      cur = euler(t, shape, tdev ? euler_t.p : nullptr);
       prefix(FIN_PLAIN, true);
     };
     if (p.graphs < 2 || prof) return body(false);
@@ -1359,7 +1371,6 @@ struct Solver final : SolverBase {
       launch_cond_copy(&shape_ctl.p->one, 1, b, st);
       const int keep = cur;
       const int out = euler(0.0, true, &shape_ctl.p->tstep);
-      prep(uh[out].p);
       cur = out;
       prefix(FIN_PLAIN, true);
       cur = keep;
@@ -1519,8 +1530,7 @@ struct Solver final : SolverBase {
         } else {
           const int out = euler(-time_step * p.ga, false);
           r.evaluations++;
-          cur = out;
-          prepped = prefixed = prefixed_f = false;
+          cur = out;   // P, Q are prepared for it
         }
         if (time_step < 1e-23) { r.status = VB_ERR_DT_UNDERFLOW; break; }
         if (time_current > p.tmax) { r.status = VB_FINISHED; break; }
@@ -1746,7 +1756,8 @@ struct Solver final : SolverBase {
     if (!W.p) W.alloc((size_t)g.ncp);
     if (!v.p) v.alloc((size_t)g.nr);
     if (!f.p) f.alloc((size_t)g.nr);
-    if (!rpart.p) rpart.alloc((size_t)nxb);
+    const int nres = ox->xe_plane ? g.nz : nxb;
+    if (!rpart.p) rpart.alloc((size_t)nres);
     ensure_prefixed(true);
     XeArgs<T> e;
     e.W = W.p;
@@ -1764,9 +1775,12 @@ struct Solver final : SolverBase {
     e.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
     e.part = rpart.p;
     e.tp = nullptr;
-    L("xe_resid", [&] { ox->xe(e, st); });
+    L("xe_resid", [&] {
+      if (ox->xe_plane) ox->xe_plane(e, g, st);
+      else ox->xe(e, st);
+    });
     check_launch();
-    std::vector<double> h((size_t)nxb);
+    std::vector<double> h((size_t)nres);
     VB_HIP(hipMemcpyAsync(h.data(), rpart.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
     VB_HIP(hipStreamSynchronize(st));
     double sum = 0.0;
