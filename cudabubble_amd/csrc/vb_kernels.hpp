@@ -80,6 +80,21 @@ template <typename T, int N> constexpr int colw() {
   return seg > occ ? seg : occ;
 }
 
+// Plan variant of the z stage kernels (see Plan): the default plan, except
+// FP32 at 192, 12 x 4 x 4 (two exchanges instead of three, the same 12
+// elements per thread; 218-240 registers against 205-226, two waves per SIMD
+// either way; 4 x 192^3 batched 3.61 -> 3.57 ms per step), and at 384, 12 x 4 x
+// 4 x 2 (three instead of four; a 384^3 step 8.52 -> 8.34 ms, the combines 539,
+// 499, 497 -> 499, 475, 476 us), and the short lengths with four elements per
+// thread: a combine there is one or two waves per SIMD of serial FP64 work, and
+// half the elements per thread halve it (a 32^3 FP64 drift step 104 -> 96 us,
+// 8 x 64^3 FP64 batched 506 -> 487).  At 256 the
+// 16 x 16 plan needs 248-256 registers there and ran slower (stage 4 158 ->
+// 182 us), and so did 4 x 4 x 4 x 4 over 64 threads (100-128 registers).
+template <typename T, int N> constexpr int zsplan() {
+  return (sizeof(T) == 4 && (N == 192 || N == 384)) ? 3 : (N == 32 || (N == 64 && sizeof(T) == 8)) ? 4 : 0;
+}
+
 // Column tile of the z stage kernels (stage combines, z-prep, plain z
 // passes).  Up to 96, one wave's columns, so that the combines need no
 // workgroup barrier and a short grid spreads over more CUs (a 32^3 FP64 combine
@@ -94,7 +109,8 @@ template <typename T, int N> constexpr int colw() {
 // from 1410-2358 to 1118-1440 us (the forward y pass, which writes the
 // 8-column groups, from 483 to 590 us) and a step from 25.7 to 23.2 ms.
 template <typename T, int N> constexpr int tbw() {
-  if (N <= 96) return 64 / TFof<N>();
+  if (N == 64 && sizeof(T) == 8) return 8;
+  if (N <= 96) return 64 / TFof<N, zsplan<T, N>()>();
   return (sizeof(T) == 4 && (N == 256 || N == 512)) ? 8 : colw<T, N>();
 }
 // The other z tile a kernel schedule can select: the column width where tbw
@@ -833,9 +849,9 @@ __device__ __forceinline__ int mindex(const Geo& g, int kx, int ky, int kz) {
   return kx * kx + fy * fy + fz * fz;
 }
 
-template <typename T, int N, int S, int TB = tbw<T, N>()>
-__global__ void __launch_bounds__((TB * TFof<N>())) k_zpass(cpx<T>* buf, Geo g, const cpx<T>* __restrict__ tw) {
-  constexpr int E = Plan<N>::E, TF = N / E;
+template <typename T, int N, int S, int TB = tbw<T, N>(), int V = zsplan<T, N>()>
+__global__ void __launch_bounds__((TB * TFof<N, V>())) k_zpass(cpx<T>* buf, Geo g, const cpx<T>* __restrict__ tw) {
+  constexpr int E = Plan<N, V>::E, TF = N / E;
   __shared__ cpx<T> sm[N * TB];
   const int j = threadIdx.x / TB;
   ColLds<T, TB> lds{sm + threadIdx.x % TB};
@@ -845,7 +861,7 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zpass(cpx<T>* buf, Geo g, 
   cpx<T> x[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) x[e] = col[(long long)(j + TF * e) * plane];
-  fft<T, N, S>(x, j, tw, lds);
+  fft<T, N, S, V>(x, j, tw, lds);
   if (id.valid) {
 #pragma unroll
     for (int e = 0; e < E; ++e) col[(long long)(j + TF * e) * plane] = x[e];
@@ -870,9 +886,9 @@ struct ZmArgs {
   Geo gi, go;   // layouts of in and out; the tiles are those of an aligned one
 };
 
-template <typename T, int N, int S, int TB, int OP>
-__global__ void __launch_bounds__((TB * TFof<N>())) k_zmul(ZmArgs<T> a) {
-  constexpr int E = Plan<N>::E, TF = N / E;
+template <typename T, int N, int S, int TB, int OP, int V = zsplan<T, N>()>
+__global__ void __launch_bounds__((TB * TFof<N, V>())) k_zmul(ZmArgs<T> a) {
+  constexpr int E = Plan<N, V>::E, TF = N / E;
   __shared__ cpx<T> sm[N * TB];
   const int j = threadIdx.x / TB;
   ColLds<T, TB, TB * TF == 64> lds{sm + threadIdx.x % TB};
@@ -900,7 +916,7 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zmul(ZmArgs<T> a) {
       }
     }
   }
-  fft<T, N, S>(x, j, a.tw, lds);
+  fft<T, N, S, V>(x, j, a.tw, lds);
   if (id.valid) {
 #pragma unroll
     for (int e = 0; e < E; ++e) out[(long long)(j + TF * e) * a.go.pp] = x[e];
@@ -1009,9 +1025,9 @@ struct ZprArgs {
   Geo g;
 };
 
-template <typename T, int N, int TB = tbw<T, N>(), bool TAB = false>
-__global__ void __launch_bounds__((TB * TFof<N>())) k_zprep(ZprArgs<T> a0, const ZprArgs<T>* tab) {
-  constexpr int E = Plan<N>::E, TF = N / E;
+template <typename T, int N, int TB = tbw<T, N>(), bool TAB = false, int V = zsplan<T, N>()>
+__global__ void __launch_bounds__((TB * TFof<N, V>())) k_zprep(ZprArgs<T> a0, const ZprArgs<T>* tab) {
+  constexpr int E = Plan<N, V>::E, TF = N / E;
   const ZprArgs<T> a = TAB ? tab[blockIdx.z] : a0;
   const Geo& g = a.g;
   const cpx<T>* __restrict__ tw = a.tw;
@@ -1034,17 +1050,17 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zprep(ZprArgs<T> a0, const
   double acc = 0.0;
 #pragma unroll
   for (int e = 0; e < E; ++e) next_field_elem<T>(u[e].x, u[e].y, j + TF * e, id, g, acc, x[e], y[e]);
-  next_field_tail<T, N, TB, 0>(x, y, acc, j, id, g, lds, lds2, tw, a.P, a.Q, a.part, red, tile);
+  next_field_tail<T, N, TB, V>(x, y, acc, j, id, g, lds, lds2, tw, a.P, a.Q, a.part, red, tile);
 }
 
 // After an Euler update: the z-forward of W (x and y transformed, row layout)
 // is the new state, stored widened to FP64 and group-major, and its P, Q follow
 // as in k_zprep (one kernel where the z pass, the relayout and k_zprep were
 // three).
-template <typename T, int N, int TB>
-__global__ void __launch_bounds__((TB * TFof<N>())) k_zeuler(const cpx<T>* __restrict__ W, cpx<double>* __restrict__ uh,
+template <typename T, int N, int TB, int V = zsplan<T, N>()>
+__global__ void __launch_bounds__((TB * TFof<N, V>())) k_zeuler(const cpx<T>* __restrict__ W, cpx<double>* __restrict__ uh,
                                                              ZprArgs<T> a) {
-  constexpr int E = Plan<N>::E, TF = N / E;
+  constexpr int E = Plan<N, V>::E, TF = N / E;
   constexpr bool WAVE = TB * TF == 64;
   const Geo& g = a.g;
   __shared__ cpx<T> sm[2 * N * TB];
@@ -1057,7 +1073,7 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zeuler(const cpx<T>* __res
   cpx<T> x[E], y[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) x[e] = W[id.q + (long long)(j + TF * e) * g.pp];
-  fft<T, N, -1>(x, j, a.tw, lds);
+  fft<T, N, -1, V>(x, j, a.tw, lds);
   const long long ib0 = (long long)tile * N * TB + threadIdx.x % TB;
   double acc = 0.0;
 #pragma unroll
@@ -1068,7 +1084,7 @@ __global__ void __launch_bounds__((TB * TFof<N>())) k_zeuler(const cpx<T>* __res
     next_field_elem<T>(re, im, j + TF * e, id, g, acc, x[e], y[e]);
   }
   lds.sync();   // the forward transform's last reads
-  next_field_tail<T, N, TB, 0>(x, y, acc, j, id, g, lds, lds2, a.tw, a.P, a.Q, a.part, red, tile);
+  next_field_tail<T, N, TB, V>(x, y, acc, j, id, g, lds, lds2, a.tw, a.P, a.Q, a.part, red, tile);
 }
 
 template <typename T>
@@ -1121,22 +1137,20 @@ struct ZsArgs {
 // the first evaluation of a penalty-drift step (belastic.cpp:677-683): the
 // new state is not stored, and only P (its z-inverse) and the Parseval and
 // DC terms are.
-// Plan variant of the stage combines (see Plan): the default plan, except
-// FP32 at 192, 12 x 4 x 4 (two exchanges instead of three, the same 12
-// elements per thread; 218-240 registers against 205-226, two waves per SIMD
-// either way; 4 x 192^3 batched 3.61 -> 3.57 ms per step), and at 384, 12 x 4 x
-// 4 x 2 (three instead of four; a 384^3 step 8.52 -> 8.34 ms, the combines 539,
-// 499, 497 -> 499, 475, 476 us).  At 256 the
-// 16 x 16 plan needs 248-256 registers there and ran slower (stage 4 158 ->
-// 182 us), and so did 4 x 4 x 4 x 4 over 64 threads (100-128 registers).
-template <typename T, int N> constexpr int zsplan() { return (sizeof(T) == 4 && (N == 192 || N == 384)) ? 3 : 0; }
+// A tile with few elements per thread has the registers for all its operands at
+// once (up to 290 in FP64): loaded before the transforms, with the coefficients
+// per element, they cost one memory latency instead of three in a row.  Not at 48
+// and 96, whose 12 elements per thread would need over 400.
+template <int N, int TB, int V> constexpr bool zs_early() {
+  return Plan<N, V>::E <= 4 || (Plan<N, V>::E <= 8 && TB * TFof<N, V>() == 64);
+}
 
 // LDS bytes of a stage combine: two column tiles for the transforms, or the
 // staged coefficient table, whichever is larger
 template <typename T, int N, int SCH, int STG, int TB, int V>
 constexpr int zs_lds_bytes() {
   return (2 * N * TB * int(sizeof(cpx<T>))) >
-                 ((SCH == 4 && STG != 2 && !(TB * TFof<N, V>() == 64 && Plan<N, V>::E <= 8)) ? TB * (N / 2 + 1) * int(STG == 4 ? sizeof(double4) : sizeof(double2)) : 0)
+                 ((SCH == 4 && STG != 2 && !zs_early<N, TB, V>()) ? TB * (N / 2 + 1) * int(STG == 4 ? sizeof(double4) : sizeof(double2)) : 0)
              ? 2 * N * TB * int(sizeof(cpx<T>))
              : TB * (N / 2 + 1) * int(STG == 4 ? sizeof(double4) : sizeof(double2));
 }
@@ -1150,11 +1164,7 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, int ti
   static_assert(!PROBE || (SCH == 4 && STG == 4), "the probe form is the last ETDRK4 stage");
   constexpr int E = Plan<N, V>::E, TF = N / E;
   constexpr bool WAVE = TB * TF == 64;   // the tile is one wave's (the workgroup may run several)
-  // A wave tile has the registers for all its operands at once (up to 290 in
-  // FP64): loaded before the transforms, with the coefficients per element,
-  // they cost one memory latency instead of three in a row.  Not at 48 and 96,
-  // whose 12 elements per thread would need over 400.
-  constexpr bool EARLY = WAVE && E <= 8;
+  constexpr bool EARLY = zs_early<N, TB, V>();
   // ETDRK4 stages 1, 3 and 4 read their coefficient records from a
   // per-workgroup table in LDS: TB columns x (N/2 + 1) folded kz, gathered once
   // after the forward transforms.  Gathered per element, the 64 lanes of a load
@@ -1225,14 +1235,20 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, int ti
   double ftot[KF] = {};
   if (a.nxb > 0) {
     double fs[KF] = {};
-    for (int i = tid; i < a.nxb; i += NTZ) {
-      fs[0] += a.xpart[3 * i + 1];
-      if constexpr (KF == 4) {
-        fs[2] += a.dcpart[2 * i];
-        fs[3] += a.dcpart[2 * i + 1];
+    auto sum = [&](double& s, const double* p, int n, int stride) {   // four loads in flight
+      for (int i = tid; i < n; i += 4 * NTZ) {
+        double t[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[k] = i + k * NTZ < n ? p[(i + k * NTZ) * stride] : 0.0;
+        s += (t[0] + t[1]) + (t[2] + t[3]);
       }
+    };
+    sum(fs[1], a.zin, a.nzb, 1);
+    sum(fs[0], a.xpart + 1, a.nxb, 3);
+    if constexpr (KF == 4) {
+      sum(fs[2], a.dcpart, a.nxb, 2);
+      sum(fs[3], a.dcpart + 1, a.nxb, 2);
     }
-    for (int i = tid; i < a.nzb; i += NTZ) fs[1] += a.zin[i];
     if constexpr (WAVE) {
       wave_sum(fs);
 #pragma unroll

@@ -24,7 +24,7 @@ struct Launch {
   static constexpr int G = xlanes<T, N>();
   static constexpr int TB = (SC & 1) ? tbw_alt<T, N>() : tbw<T, N>();
   static constexpr int XR = (SC & 2) ? xrplan_alt<T, N>() : xrplan<T, N>();
-  static constexpr int YT = TB * TF;
+  static constexpr int YT = TB * TFof<N, zsplan<T, N>()>();
   static constexpr int CV = colplan<T, N>();          // plan of the y passes and the z Laplacian
   static constexpr int CB = colw<T, N>();             // their columns per workgroup
   static constexpr int CT = CB * TFof<N, CV>();       // and threads per workgroup
