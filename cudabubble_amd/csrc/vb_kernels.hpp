@@ -35,6 +35,7 @@ namespace vb {
 // share 128-byte lines (two planes of a group-major spectrum, two 8-column tiles
 // of a row) run on one XCD.
 constexpr int kXcds = 8;
+constexpr int kCus = 256;    // compute units
 // item of workgroup b (of n) when items 2i and 2i + 1 are to share an XCD; a
 // permutation of [0, n), the identity past the last whole sixteen
 __device__ __forceinline__ int pair_item(int b, int n) {

@@ -6,15 +6,15 @@
 // the spectra of tmp1 and s written once, instead of three kernels that each
 // read and write both arrays.
 //
-// What bounds it: the chain of its phases at the short lengths (one workgroup
-// per CU at most), VALU issue at 128 (42 000 cycles for 16 waves).  So the
-// transforms stay inside a wave (no workgroup barrier but between the three
-// phases), the twiddles are read from LDS, the Nyquist columns have a wave of
-// their own, and the sums go through DPP moves.  Measured: 32^3 FP64 6.2 us
-// against 13.1 for the three kernels, 64^3 FP32 8.7 against 14.7, 128^3 FP32
-// 23 against 33; a penalty-drift step 173 -> 104, 195 -> 138, 489 -> 416 us
-// (with the combines evaluating the integrals and their wave tiles), batches of
-// 16 x 32^3, 16 x 64^3, 12 x 128^3 302 -> 186, 712 -> 617, 3465 -> 2835 us.
+// What bounds it: the chain of its phases (one workgroup per CU at most at the
+// larger lengths).  So the transforms stay inside a wave (no workgroup barrier
+// but between the phases), the twiddles are read from LDS, the Nyquist columns
+// have a wave of their own, and the sums go through DPP moves.  Measured: 32^3
+// FP64 6.2 us against 13.1 for the three kernels, 128^3 FP32 (k_plane2) 19
+// against 33; a penalty-drift step of 32^3 FP64, 64^3 FP32, 128^3 FP32 173 -> 104,
+// 195 -> 138, 489 -> 388 us (with the combines evaluating the integrals and their
+// wave tiles), batches of 16 x 32^3, 16 x 64^3, 12 x 128^3 302 -> 186, 712 ->
+// 576, 3465 -> 2800 us.
 #pragma once
 #include "vb_kernels.hpp"
 
@@ -371,36 +371,60 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_pair(PairArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// The plane kernel where P and Q of a plane do not fit LDS together but one of
-// them does (FP64 at 128): the plane of P goes through y and x first, its v kept
-// in registers, then Q's, then the spectra of tmp1 and of s one after the other.
-// Two rows travel as one transform (k_pair's storage).  The same modes,
-// arguments and units as k_plane, but PL_SUMS takes one plane per workgroup.
-// One workgroup per CU and its phases in a row bound it, 45 us at 128^3 whether
-// 128 or 256 planes run; the three kernels take 50, and 100 for 256 planes: a
-// 128^3 FP64 drift step 627 -> 608 us, four of them batched 2026 -> 1607.  (FP32
-// at 192 fits as well but spills 78 registers: 76 us against 75.)
+// The prefix with two rows travelling as one transform (k_pair's storage): half
+// the rows and columns per array, so a workgroup has half the waves of k_plane's
+// and each has twice the phases.  Where both planes fit LDS (two) they go through
+// a phase together; else (FP64 at 128) the plane of P goes through y and x first,
+// its v kept in registers, then Q's, then the spectra of tmp1 and of s one after
+// the other.  The same arguments and units as k_plane.
+//
+// A workgroup does not get faster with fewer of them, so a launch whose last
+// round of planes fills at most half of the 256 CUs gives these planes two
+// workgroups each (nsplit): both invert P and Q and take the pointwise terms, one
+// transforms tmp1 and writes the sums, the other s; the second read of P and Q
+// comes from the XCD's L2.  What remains is latency and LDS: 9 000 of about
+// 45 000 cycles issue VALU.  Measured, us per step:
+//   128^3 FP64 drift: three kernels 627, one workgroup per plane 606, two 556;
+//     batches of 3 and 4 (the rest of 384 split; 512) 1375 -> 1303, 1594
+//   128^3 FP32 drift: k_plane 418, here 388; batches of 2, 3, 12: 572, 863,
+//     2832 -> 572, 832, 2800
+//   96^3 FP64: k_plane 414, here 380; batches of 2, 6: 605, 1445 -> 589, 1401
+//   64^3 FP32: 138 both; batches of 6, 16: 307, 617 -> 287, 577
+// k_plane stays at the others: 96^3 FP32 batches of 2 and 6 365, 829 against 391,
+// 884, 64^3 FP64 batch of 4 283 against 302, 32^3 and 48^3 5 % and more.  (FP32 at
+// 192 fits as well but spills 78 registers: 76 us against 75.)  PL_SUMS takes one
+// plane per workgroup here; it and PL_ROWSUMS run here only where k_plane does
+// not fit.
 // ---------------------------------------------------------------------------
 template <typename T, int N>
 struct Plane2Cfg {
-  static constexpr bool ok = sizeof(T) == 8 && N == 128;
+  static constexpr bool ok = N == 128 || N == (sizeof(T) == 4 ? 64 : 96);
+  static constexpr bool two = sizeof(T) == 4 || N <= 96;   // both planes do fit
 };
 
 // Planes from which the plane kernels are the faster ones: a workgroup's time
 // does not shrink with fewer of them.  128 x 128 x nz drift steps, plane kernels
-// against three kernels, us: FP32 nz = 16 237 / 186, 32 264 / 256, 64 343 / 345,
-// 128 416 / 459; FP64 nz = 64 (no drift) 273 / 190, 96 650 / 644, 128 608 / 627,
-// 192 878 / 1023.  At the shorter lengths they won at every depth measured (16
-// and up).
-template <typename T, int N> constexpr int plane_min_nz() { return Plane2Cfg<T, N>::ok ? 128 : N == 128 ? 64 : 0; }
+// against three kernels, us: FP32 nz = 16 213 / 160, 32 246 / 215, 48 297 / 285,
+// 64 (one workgroup per plane) 343 / 345, 128 388 / 459; FP64 nz = 32 351 / 262,
+// 64 399 / 361, 96 558 / 562, 128 556 / 627, 192 878 / 1023.  At the shorter
+// lengths they won at every depth measured (16 and up).
+template <typename T, int N> constexpr int plane_min_nz() { return N < 128 ? 0 : sizeof(T) == 8 ? 128 : 64; }
 
 template <typename T, int N, int MODE, bool TAB = false>
-__global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0, const PlaneArgs<T>* tab) {
+__global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0, const PlaneArgs<T>* tab,
+                                                                    int nsplit) {
   using C = PairCfg<T, N>;
   constexpr int E = C::E, TF = C::TF, LL = C::LL, PS = C::PS, V = C::V, CW = C::CW, NA = C::NA, H = N / 2;
-  const PlaneArgs<T> a = TAB ? tab[blockIdx.z] : a0;
+  // the last nsplit solves have two workgroups per plane: the first writes
+  // tmp1's spectra and the sums, the second, at the end of the grid, s's
+  const int lanes = int(gridDim.z) - nsplit, second = int(blockIdx.z) >= lanes;
+  const int lane_z = second ? int(blockIdx.z) - nsplit : int(blockIdx.z);
+  const bool split = lane_z >= lanes - nsplit;
+  const PlaneArgs<T> a = TAB ? tab[lane_z] : a0;
   const Geo& g = a.g;
-  __shared__ cpx<T> sm[H * LL];
+  // FP32: a plane each for P and Q, tmp1 and s; FP64: one, in turn
+  constexpr bool TWO = Plane2Cfg<T, N>::two;
+  __shared__ cpx<T> sm[(TWO ? 2 : 1) * H * LL];
   __shared__ cpx<T> tw[N];
   constexpr int K = (MODE == PL_ETD && sizeof(T) == 4) ? 5 : 3;
   __shared__ double red[K * (NA / 64)];
@@ -408,9 +432,11 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int cj = lane / CW, kx = wave * CW + lane % CW;    // column
   const int r = threadIdx.x / TF, j = threadIdx.x % TF;    // row pair
-  PlaneRow<T, PS> row{sm + (r < H ? r : 0) * LL};
+  constexpr int B2 = TWO ? H * LL : 0;
+  const PlaneRow<T, PS> row1{sm + (r < H ? r : 0) * LL}, row2{row1.base + B2};
   auto slot = [](int c) { return c + (c >> PS); };
-  const PairCol<T, LL> col{sm + slot(kx < H ? kx : N), kx < H ? slot(H + kx) - slot(kx) : slot(N + 1) - slot(N)};
+  const PairCol<T, LL> col1{sm + slot(kx < H ? kx : N), kx < H ? slot(H + kx) - slot(kx) : slot(N + 1) - slot(N)},
+      col2{col1.base + B2, col1.odd};
   const bool isrow = r < H, iscol = kx <= H;
   const long long pz = (long long)z * g.pp;
 
@@ -420,14 +446,14 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
       for (int e = 0; e < E; ++e) x[e] = src[unsigned(plane_pos(g, cj + TF * e, kx))];
     }
   };
-  auto col_inv = [&](cpx<T>* x) {
+  auto col_inv = [&](cpx<T>* x, const PairCol<T, LL>& col) {
     if (iscol) {
       fft<T, N, +1, V>(x, cj, tw, col);
 #pragma unroll
       for (int e = 0; e < E; ++e) col(cj + TF * e) = x[e];
     }
   };
-  auto row_inv = [&](cpx<T>* x) {   // two real rows, as re and im
+  auto row_inv = [&](cpx<T>* x, const PlaneRow<T, PS>& row) {   // two real rows, as re and im
     if (isrow) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
@@ -443,8 +469,7 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
       fft<T, N, +1, V>(x, j, tw, row);
     }
   };
-  // the plane of two real rows per lane group through x and y into out
-  auto forward = [&](cpx<T>* x, cpx<T>* out) {
+  auto row_fwd = [&](cpx<T>* x, const PlaneRow<T, PS>& row) {
     if (isrow) {
       constexpr int NH = H + 1, U = (NH + TF - 1) / TF;
       fft<T, N, -1, V>(x, j, tw, row);
@@ -471,7 +496,8 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
         }
       }
     }
-    __syncthreads();
+  };
+  auto col_fwd = [&](const PairCol<T, LL>& col, cpx<T>* out) {
     if (iscol) {
       cpx<T> y[E];
 #pragma unroll
@@ -492,18 +518,27 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
 
   cpx<T> v[E], x[E];
   col_load(x, a.P + pz);
+  if constexpr (TWO && MODE != PL_SUMS) col_load(v, a.Q + pz);
   for (int i = threadIdx.x; i < N; i += NA) tw[i] = a.tw[i];
   __syncthreads();
-  col_inv(x);
-  __syncthreads();
-  if constexpr (MODE != PL_SUMS) {
-    row_inv(v);
-    col_load(x, a.Q + pz);
-    __syncthreads();   // the rows of P are read
-    col_inv(x);
+  col_inv(x, col1);
+  if constexpr (MODE == PL_SUMS) {
     __syncthreads();
+    row_inv(x, row1);
+  } else if constexpr (TWO) {
+    col_inv(v, col2);
+    __syncthreads();
+    row_inv(v, row1);
+    row_inv(x, row2);    // lap v
+  } else {
+    __syncthreads();
+    row_inv(v, row1);
+    col_load(x, a.Q + pz);
+    __syncthreads();     // the rows of P are read
+    col_inv(x, col1);
+    __syncthreads();
+    row_inv(x, row1);
   }
-  row_inv(x);          // lap v (PL_SUMS: v)
   double acc[K] = {};
   if (isrow) {
     const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps, D = a.D;
@@ -543,13 +578,30 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
   }
   wave_part<K, NA>(acc, red);
   if constexpr (MODE == PL_ETD) {
-    forward(x, a.U);     // its barrier orders the sums' too
-    __syncthreads();
-    forward(v, a.U2);
+    // the barriers order the sums' partials too
+    if constexpr (TWO) {
+      if (!second) row_fwd(x, row1);
+      if (second || !split) row_fwd(v, row2);
+      __syncthreads();
+      if (!second) col_fwd(col1, a.U);
+      if (second || !split) col_fwd(col2, a.U2);
+    } else {
+      if (!second) {
+        row_fwd(x, row1);
+        __syncthreads();
+        col_fwd(col1, a.U);
+      }
+      if (!split) __syncthreads();
+      if (second || !split) {
+        row_fwd(v, row1);
+        __syncthreads();
+        col_fwd(col1, a.U2);
+      }
+    }
   } else {
     __syncthreads();
   }
-  if (threadIdx.x < K) {
+  if (threadIdx.x < K && !second) {
     const double s = wave_total<NA>(red, threadIdx.x);
     if (threadIdx.x < 3) a.part[3 * (long long)blockIdx.x + threadIdx.x] = s;
     else if (a.dcpart) a.dcpart[2 * (long long)blockIdx.x + threadIdx.x - 3] = s;

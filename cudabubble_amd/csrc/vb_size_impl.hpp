@@ -184,27 +184,38 @@ struct Launch {
     zs_dispatch<false>(sch, stg, gr, a, nullptr, s);
   }
 
+  // solves, of `lanes` with nz planes each, whose planes get two workgroups of
+  // k_plane2 each: those of a last round of planes that fills at most half of
+  // the compute units (measured at k_plane2)
+  static int plane2_split(int nz, int lanes) {
+    const int rest = nz * lanes % kCus;
+    return 2 * rest <= kCus ? rest / nz : 0;
+  }
   template <bool TAB>
   static void pl_launch(int mode, dim3 gr, const PlaneArgs<T>& a, const PlaneArgs<T>* tab, hipStream_t s) {
-    const dim3 bl(kPlaneThreads);
-    if constexpr (PlaneCfg<T, N>::ok) {
-      if (!TAB && mode == PL_EULER) {
-        hipLaunchKernelGGL((k_plane<T, N, PL_EULER>), gr, bl, 0, s, a, nullptr);
+    if constexpr (Plane2Cfg<T, N>::ok) {
+      if (mode == PL_ETD) {
+        const int k = plane2_split(int(gr.x), int(gr.z));
+        gr.z += unsigned(k);
+        hipLaunchKernelGGL((k_plane2<T, N, PL_ETD, TAB>), gr, dim3(PairCfg<T, N>::NA), 0, s, a, tab, k);
         return;
       }
-      if (mode == PL_ETD)
-        hipLaunchKernelGGL((k_plane<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
+    }
+    const dim3 bl(kPlaneThreads);
+    if constexpr (PlaneCfg<T, N>::ok) {
+      if (!TAB && mode == PL_EULER)
+        hipLaunchKernelGGL((k_plane<T, N, PL_EULER>), gr, bl, 0, s, a, nullptr);
       else if (mode == PL_SUMS)
         hipLaunchKernelGGL((k_plane<T, N, PL_SUMS, TAB>), gr, bl, 0, s, a, tab);
-      else
+      else if (mode == PL_ROWSUMS)
         hipLaunchKernelGGL((k_plane<T, N, PL_ROWSUMS, TAB>), gr, bl, 0, s, a, tab);
+      else if constexpr (!Plane2Cfg<T, N>::ok)
+        hipLaunchKernelGGL((k_plane<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
     } else if constexpr (Plane2Cfg<T, N>::ok) {
-      if (mode == PL_ETD)
-        hipLaunchKernelGGL((k_plane2<T, N, PL_ETD, TAB>), gr, bl, 0, s, a, tab);
-      else if (mode == PL_SUMS)
-        hipLaunchKernelGGL((k_plane2<T, N, PL_SUMS, TAB>), gr, bl, 0, s, a, tab);
+      if (mode == PL_SUMS)
+        hipLaunchKernelGGL((k_plane2<T, N, PL_SUMS, TAB>), gr, bl, 0, s, a, tab, 0);
       else
-        hipLaunchKernelGGL((k_plane2<T, N, PL_ROWSUMS, TAB>), gr, bl, 0, s, a, tab);
+        hipLaunchKernelGGL((k_plane2<T, N, PL_ROWSUMS, TAB>), gr, bl, 0, s, a, tab, 0);
     }
   }
   static constexpr int kPlaneThreads = PlaneCfg<T, N>::ok ? PlaneCfg<T, N>::NA : PairCfg<T, N>::NA;

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("prec", ["FP64", "FP32_MIXED"])
 @pytest.mark.parametrize("nx,nz", [(16, 16), (16, 48), (32, 16), (32, 32), (48, 48), (48, 16), (64, 16), (64, 96),
-                                   (96, 16), (96, 48), (128, 48), (128, 64), (128, 128)])
+                                   (96, 16), (96, 48), (128, 48), (128, 64), (128, 128), (128, 192)])
 def test_prefix_in_one_kernel(vb, gpu, oracle_mod, nx, nz, prec):
     flush_print("plane", nx, nz, prec)
     eps = 2.0 * 2 * np.pi / nx
@@ -42,6 +42,30 @@ def test_prefix_in_one_kernel(vb, gpu, oracle_mod, nx, nz, prec):
     assert rel(V, Vo) < 10 * tol and rel(A, Ao) < 10 * tol
     if prec == "FP64":
         assert rel(Eb, Ebo) < 1e-11
+
+
+# solves per batch such that all, the last ones or none of them have their planes
+# in two workgroups (a round is 256 planes)
+@pytest.mark.parametrize("nx,nz,count,prec", [(128, 128, 1, "FP64"), (128, 128, 2, "FP64"), (128, 128, 3, "FP32_MIXED"),
+                                              (96, 48, 6, "FP64"), (64, 64, 5, "FP32_MIXED"), (64, 16, 17, "FP32_MIXED")])
+def test_prefix_with_two_workgroups_per_plane(vb, gpu, nx, nz, count, prec):
+    """Which planes are shared out is not seen in the result: every solve of a
+    batch is its own run, bit for bit."""
+    flush_print("split planes", nx, nz, count, prec)
+    eps = 2.0 * 2 * np.pi / nx
+    ps, phis = [], []
+    for k in range(count):
+        phi, _ = vb.shape(vb.SHAPE_ELLIPSOID, 30 + k, nx, nz, 1.0, eps)
+        ps.append(vb.params_default(nx=nx, nz=nz, eps=eps, M1=1e4, M2=1e4, alpha=-1.0, beta=-1.0, time_step=1e-7,
+                                    fixed_time_step=1e-7, precision=getattr(vb, prec), phi_lut_mode=1))
+        phis.append(phi)
+    b = vb.Batch(ps, phis)
+    reps = b.step(3)
+    for i in {0, count - 2, count - 1} & set(range(count)):
+        assert reps[i]["status"] == 0
+        s = vb.Solver(ps[i], phis[i])
+        s.step(3)
+        assert np.array_equal(b.get_phi(i), s.get_phi()) and b.query(i) == s.query(), i
 
 
 @pytest.mark.parametrize("nx,nz", [(16, 16), (48, 32), (96, 16), (128, 16), (192, 16), (256, 16)])
