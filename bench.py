@@ -538,7 +538,9 @@ def main():
     roof["copy_variants_GBps"] = copy_each
     roof["copy_GBps_torch"] = copy_bandwidth() / 1e9
     roof["frac_of_copy"] = achieved / copy_bw if achieved else None
-    tfile = os.path.join(ROOT, "profiles", "traffic_%s_%d_fp32.json" % (name, n))
+    # the group-major forward y pass is the profile's y_fwd
+    tname = {"y_fwd2": "y_fwd"}.get(name, name)
+    tfile = os.path.join(ROOT, "profiles", "traffic_%s_%d_fp32.json" % (tname, n))
     if os.path.exists(tfile):
         with open(tfile) as f:
             roof["traffic"] = json.load(f).get("bytes_per_launch")
