@@ -76,6 +76,7 @@ template <> struct Plan<192, 1> { static constexpr int E = 24, NP = 2; static co
 template <> struct Plan<384, 3> { static constexpr int E = 12, NP = 4; static constexpr int R[4] = {12, 4, 4, 2}; };
 template <> struct Plan<32, 4>  { static constexpr int E = 4,  NP = 3; static constexpr int R[3] = {4, 4, 2}; };
 template <> struct Plan<64, 4>  { static constexpr int E = 4,  NP = 3; static constexpr int R[3] = {4, 4, 4}; };
+template <> struct Plan<128, 4> { static constexpr int E = 4,  NP = 4; static constexpr int R[4] = {4, 4, 4, 2}; };
 template <> struct Plan<48, 3>  { static constexpr int E = 12, NP = 2; static constexpr int R[2] = {12, 4}; };
 template <> struct Plan<96, 3>  { static constexpr int E = 12, NP = 3; static constexpr int R[3] = {12, 4, 2}; };
 template <> struct Plan<192, 3> { static constexpr int E = 12, NP = 3; static constexpr int R[3] = {12, 4, 4}; };

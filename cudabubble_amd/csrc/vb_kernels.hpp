@@ -89,11 +89,14 @@ template <typename T, int N> constexpr int colw() {
 // 499, 497 -> 499, 475, 476 us), and the short lengths with four elements per
 // thread: a combine there is one or two waves per SIMD of serial FP64 work, and
 // half the elements per thread halve it (a 32^3 FP64 drift step 104 -> 96 us,
-// 8 x 64^3 FP64 batched 506 -> 487).  At 256 the
+// 8 x 64^3 FP64 batched 506 -> 487).  FP64 at 128 takes 4 x 4 x 4 x 2 for the
+// same reason: its 2080 waves of 8 elements are one round of two per SIMD
+// (a 128^3 drift step 556 -> 549 us, an adaptive attempt 400 -> 397, batches of
+// three unchanged).  At 256 the
 // 16 x 16 plan needs 248-256 registers there and ran slower (stage 4 158 ->
 // 182 us), and so did 4 x 4 x 4 x 4 over 64 threads (100-128 registers).
 template <typename T, int N> constexpr int zsplan() {
-  return (sizeof(T) == 4 && (N == 192 || N == 384)) ? 3 : (N == 32 || (N == 64 && sizeof(T) == 8)) ? 4 : 0;
+  return (sizeof(T) == 4 && (N == 192 || N == 384)) ? 3 : (N == 32 || ((N == 64 || N == 128) && sizeof(T) == 8)) ? 4 : 0;
 }
 
 // Column tile of the z stage kernels (stage combines, z-prep, plain z
@@ -102,7 +105,8 @@ template <typename T, int N> constexpr int zsplan() {
 // was 9 workgroups of 256 threads): with the combine's operands and
 // coefficients loaded before its transforms (EARLY), 9.4 -> 6.4 us at 32^3 FP64
 // and 10.5 -> 8.6 us (stage 1 9.6 -> 6.4) at 64^3 FP32.  Above, the column
-// width, except FP32 at 256 and 512, 8 columns.  At 256 (256-thread workgroups,
+// width, except FP64 at 64 and 128 (whole 128-byte lines, with their plans of four
+// elements) and FP32 at 256 and 512, 8 columns.  At 256 in FP32 (256-thread workgroups,
 // two or three per CU) 8 measured 6-14 % faster per stage than 16: their inputs
 // are group-major, so only their P, Q outputs are written in 64-byte pieces.  At
 // 512, 16 columns make 1024-thread workgroups, whose 128-register budget
@@ -110,7 +114,7 @@ template <typename T, int N> constexpr int zsplan() {
 // from 1410-2358 to 1118-1440 us (the forward y pass, which writes the
 // 8-column groups, from 483 to 590 us) and a step from 25.7 to 23.2 ms.
 template <typename T, int N> constexpr int tbw() {
-  if (N == 64 && sizeof(T) == 8) return 8;
+  if ((N == 64 || N == 128) && sizeof(T) == 8) return 8;
   if (N <= 96) return 64 / TFof<N, zsplan<T, N>()>();
   return (sizeof(T) == 4 && (N == 256 || N == 512)) ? 8 : colw<T, N>();
 }
