@@ -542,7 +542,8 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
   double acc[K] = {};
   if (isrow) {
     const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps, D = a.D;
-    T ts[5] = {T(0), T(0), T(0), T(0), T(0)};
+    // as in k_xrow, a thread's E values of a row are added in T, the rows in FP64
+    T ts[2][5] = {};
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       T t1[2], sv[2];
@@ -560,7 +561,7 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
           t1[h] = q * (w - T(kappa));                                               // nld_kernel1, Calc.cu:270
           sv[h] = T(D) * t1[h] + (T(3 * eps) * q * q - T(eps * (D + 1))) * f;       // Calc.cu:282, times eps^3
           if constexpr (sizeof(T) == 4) {
-            ts[0] += q; ts[1] += w * w; ts[2] += f * f; ts[3] += t1[h]; ts[4] += sv[h];
+            ts[h][0] += q; ts[h][1] += w * w; ts[h][2] += f * f; ts[h][3] += t1[h]; ts[h][4] += sv[h];
           } else {
             acc[0] += double(q); acc[1] += double(w) * double(w); acc[2] += double(f) * double(f);
           }
@@ -573,7 +574,7 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
     }
     if constexpr (MODE != PL_SUMS && sizeof(T) == 4) {
 #pragma unroll
-      for (int q = 0; q < K; ++q) acc[q] = double(ts[q]);
+      for (int q = 0; q < K; ++q) acc[q] = double(ts[0][q]) + double(ts[1][q]);
     }
   }
   wave_part<K, NA>(acc, red);
