@@ -333,9 +333,19 @@ struct CalcImpl {
     inv_xy(f, f.w, (double*)out, ga);
   }
   void fftgradient(const void* fds, void* dx, void* dy, void* dz) {   // Calc.cu:344-356
-    c2r_t(fd(), (const cpx<double>*)fds, (double*)dx, ZM_DX);
-    c2r_t(fd(), (const cpx<double>*)fds, (double*)dy, ZM_DY);
-    c2r_t(fd(), (const cpx<double>*)fds, (double*)dz, ZM_DZ);
+    // fd is read once per component: where dx or dy covers part of it, from a copy
+    auto covers = [&](const void* r) {
+      const char *a = (const char*)r, *b = (const char*)fds;
+      return a < b + sizeof(cpx<double>) * (size_t)g.nc && b < a + sizeof(double) * (size_t)g.nr;
+    };
+    const cpx<double>* s = (const cpx<double>*)fds;
+    if (covers(dx) || covers(dy)) {
+      VB_HIP(hipMemcpyAsync(c2.p, fds, sizeof(cpx<double>) * (size_t)g.nc, hipMemcpyDeviceToDevice, st));
+      s = c2.p;
+    }
+    c2r_t(fd(), s, (double*)dx, ZM_DX);
+    c2r_t(fd(), s, (double*)dy, ZM_DY);
+    c2r_t(fd(), s, (double*)dz, ZM_DZ);
   }
   template <int OP>
   void pw(double* out, const void* a, const void* b, const void* c, const void* d, double s0, double s1 = 0,

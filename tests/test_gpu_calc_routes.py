@@ -1,0 +1,34 @@
+"""GPU: calls of the Calc operators that the timed cases do not make: outputs
+over their input, non-finite modes that the reference drops."""
+import numpy as np
+import pytest
+
+from conftest import flush_print, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _spectrum(oracle_mod, vb, nx, nz):
+    eps = 2.0 * 2 * np.pi / nx
+    d, _ = vb.shape(vb.SHAPE_TORUS, 5, nx, nz, 1.0, eps)
+    o = oracle_mod.Oracle(nx, nz, eps=eps)
+    return o, o.r2c(d)
+
+
+# one length with x and y in one kernel, two past it
+@pytest.mark.parametrize("nx,nz", [(48, 16), (192, 16), (256, 16)])
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_gradient_output_over_its_input(vb, gpu, oracle_mod, nx, nz, which):
+    """A component written over the spectrum (the storage reused) leaves the other
+    two components right."""
+    import torch
+    flush_print("gradient over fd", nx, nz, which)
+    o, fd = _spectrum(oracle_mod, vb, nx, nz)
+    ref = o.fftgradient(fd)
+    src = torch.from_numpy(fd).to(gpu)
+    g = [torch.empty((nz, nx, nx), dtype=torch.float64, device=gpu) for _ in range(3)]
+    g[which] = torch.view_as_real(src).reshape(-1)[:nz * nx * nx].view(nz, nx, nx)
+    vb.Calc(nx, nz).fftgradient(src, *g)
+    # the tolerance of the same operator with separate buffers (test_gpu_plane.py)
+    for a, b in zip(g, ref):
+        assert rel_l2(a.cpu().numpy(), b) < 1e-12
