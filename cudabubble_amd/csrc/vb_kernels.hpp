@@ -914,10 +914,12 @@ __global__ void __launch_bounds__((TB * TFof<N, V>())) k_zmul(ZmArgs<T> a) {
         const double c = g.kfac2, m = -(id.kx * id.kx * c + fy * fy * c + fz * fz * c);
         x[e] = mk<T>(T(double(x[e].x) * m), T(double(x[e].y) * m));
       } else {
-        const int k = OP == ZM_DX ? (id.kx == g.nx / 2 ? 0 : id.kx)
-                    : OP == ZM_DY ? (id.ky == g.ny / 2 ? 0 : sgnk(id.ky, g.ny)) : (kz == g.nz / 2 ? 0 : sgnk(kz, g.nz));
+        const int k = OP == ZM_DX ? id.kx : OP == ZM_DY ? sgnk(id.ky, g.ny) : sgnk(kz, g.nz);
+        const bool nyq = OP == ZM_DX ? id.kx == g.nx / 2 : OP == ZM_DY ? id.ky == g.ny / 2 : kz == g.nz / 2;
         const double f = g.kfac;
-        x[e] = mk<T>(T(-(double(x[e].y) * f) * k), T((double(x[e].x) * f) * k));
+        // (zero whatever the mode holds, not a product with zero)
+        const T re = T(-(double(x[e].y) * f) * k), im = T((double(x[e].x) * f) * k);
+        x[e] = mk<T>(nyq ? T(0) : re, nyq ? T(0) : im);
       }
     }
   }

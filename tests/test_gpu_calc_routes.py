@@ -32,3 +32,23 @@ def test_gradient_output_over_its_input(vb, gpu, oracle_mod, nx, nz, which):
     # the tolerance of the same operator with separate buffers (test_gpu_plane.py)
     for a, b in zip(g, ref):
         assert rel_l2(a.cpu().numpy(), b) < 1e-12
+
+
+@pytest.mark.parametrize("nx,nz", [(48, 16), (192, 16), (256, 16)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_gradient_drops_its_nyquist_modes(vb, gpu, oracle_mod, nx, nz, bad):
+    """gradient_kernel writes zero in a component's own Nyquist plane whatever the
+    mode holds (Calc.cu:310-339)."""
+    import torch
+    flush_print("gradient Nyquist", nx, nz, bad)
+    _, fd = _spectrum(oracle_mod, vb, nx, nz)
+    c = vb.Calc(nx, nz)
+    out = lambda: [torch.empty((nz, nx, nx), dtype=torch.float64, device=gpu) for _ in range(3)]
+    clean = out()
+    c.fftgradient(torch.from_numpy(fd).to(gpu), *clean)
+    for axis, plane in enumerate([np.s_[:, :, nx // 2], np.s_[:, nx // 2, :], np.s_[nz // 2, :, :]]):
+        f = fd.copy()
+        f[plane] = bad
+        g = out()
+        c.fftgradient(torch.from_numpy(f).to(gpu), *g)
+        assert torch.equal(g[axis], clean[axis]), axis
