@@ -164,11 +164,10 @@ struct Solver final : SolverBase {
   Scal* hs = nullptr;   // pinned host copy
   DBuf<double> rpart;   // block sums of the Euler residual
   int nxb = 0, nzb = 0;
-  // partial-sum sets of the last prefix's x (or plane) kernel, and which half
-  // of zpart and dc the prepared field's are in: the stage combines alternate
-  // (zprep and the last stage of either scheme use half 0), because one that
-  // evaluates the integrals itself reads one half while it writes the other
-  int nxlast = 0, zhalf = 0;
+  // zpart and dc have two halves: a stage combine that evaluates the integrals
+  // itself reads one while it writes the other.  Combine stg writes half stg & 1,
+  // so a state's partials (zprep, the Euler pass, the last stage of either
+  // scheme) are always in half 0.
   long long npairs = 0;
   int mmax = 0;
   // ETD coefficient tables: a fixed pool of slots allocated with the solver.
@@ -196,7 +195,6 @@ struct Solver final : SolverBase {
   bool prepped = false;     // P, Q hold zprep of uh[cur]
   bool prefixed = false;    // ETD prefix of uh[cur] done (scal; Tt, Ts: x,y-forward of tmp1, s)
   bool kept = false;        // scal_keep holds scal of uh[cur] (the drift double step starts from it)
-  bool fin_pending = false; // the last prefix left its integrals to the next stage combine
   bool prefixed_f = false;  // Euler prefix of uh[cur] done (scal; v, f; W: x-spectra of lap f)
   // driver state
   bool started = false;
@@ -493,13 +491,15 @@ struct Solver final : SolverBase {
     L("zprep", [&] { oz->zprep(vh, P.p, Q.p, zpart.p, dc.p, g, twz.p, st); });
     check_launch();
     prepped = true;
-    zhalf = 0;
   }
 
-  // the integrals of the prepared field from nx sets of x partials
-  FinArgs fin_of(int nx, int mode) {
-    return fin_args(xpart.p, nx, zpart.p + (size_t)zhalf * nzb, dc.p + zhalf, nzb, scal.p, fin_scratch.p, g, ph, mode);
+  // the integrals of a prepared field from nx sets of x partials and half `half`
+  // of the z partials
+  FinArgs fin_of(int nx, int mode, int half = 0) {
+    return fin_args(xpart.p, nx, zpart.p + (size_t)half * nzb, dc.p + half, nzb, scal.p, fin_scratch.p, g, ph, mode);
   }
+  // sets of x partials of an ETD and of an Euler prefix
+  int parts(bool withf) const { return by_plane(ox) && (!withf || ox->plane_euler) ? g.nz : nxb; }
 
   // fin: integrals to evaluate in the same launch as the z pass (extra
   // workgroups of it), or nullptr
@@ -540,7 +540,6 @@ struct Solver final : SolverBase {
     a.f = f.p;
     a.W = W.p;
     a.inv_n = 1.0 / double(g.nr);
-    nxlast = mode == PL_SUMS ? g.nz / ox->sums_planes : g.nz;
     L(mode == PL_SUMS ? "plane_sums" : mode == PL_EULER ? "plane_f" : "plane", [&] { ox->plane(a, mode, st); });
   }
 
@@ -551,19 +550,17 @@ struct Solver final : SolverBase {
   //  - Euler (withf = true): v, f and W = x-spectra of lap f (k_xe).
   // set 0: the prefix of the state (stage 1), kept in Tt, Ts; set 1: of a
   // later stage, in Tt1, Ts1 (so the state's survives an evaluation)
-  // defer (the stages inside an evaluation, where the next kernel is a stage
-  // combine): with a plane kernel the combine evaluates the integrals it needs.
+  // stg > 0: of the field that combine stg of an evaluation takes; with a plane
+  // kernel that combine evaluates the integrals it needs (suffix).
   // keep: the scalars also go to scal_keep.
-  void prefix(int mode, bool withf, int set = 0, bool defer = false, bool keep = false) {
+  void prefix(int mode, bool withf, int set = 0, int stg = 0, bool keep = false) {
     cpx<T>* tt = set ? Tt1.p : Tt.p;
     cpx<T>* ts = set ? Ts1.p : Ts.p;
     kept = false;
     if (by_plane(ox) && !withf) {
       plane(PL_ETD, tt, ts);
-      if (defer) {
-        fin_pending = true;
-      } else {
-        FinArgs fin = fin_of(nxlast, mode);
+      if (stg == 0) {
+        FinArgs fin = fin_of(parts(false), mode);
         fin.dcpart = kMixed ? xdc.p : nullptr;
         if (keep) fold_keep(fin);
         L("finalize", [&] { launch_finalize(fin, st); });
@@ -574,7 +571,6 @@ struct Solver final : SolverBase {
       prefixed_f = false;
       return;
     }
-    nxlast = nxb;
     XaArgs<T> a{};
     a.v = v.p;
     a.f = f.p;
@@ -587,13 +583,12 @@ struct Solver final : SolverBase {
     a.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
     // the integrals of this field (the x kernel's and the z kernel's partials)
     // are evaluated by extra workgroups of the next column pass
-    FinArgs fin = fin_of(nxb, mode);
+    FinArgs fin = fin_of(parts(withf), mode, stg > 0 ? (stg - 1) & 1 : 0);
     // FP32-mixed ETD prefix: FP64 sums of tmp1 and eps^3 s for the k = 0 modes
     fin.dcpart = (kMixed && !withf) ? xdc.p : nullptr;
     if (keep) fold_keep(fin);
     if (withf && by_plane(ox) && ox->plane_euler) {
       plane(PL_EULER, nullptr, nullptr);
-      fin.nxb = nxlast;
       spectral_lap(W.p, &fin, true);
     } else if (withf) {
       L("y_inv2", [&] { ox->ypass(P.p, Q.p, 2, +1, g, twx.p, nullptr, st); });
@@ -650,7 +645,7 @@ struct Solver final : SolverBase {
   void prefix_integrals(int mode, int fold) {
     if (by_plane(ox)) {
       plane(PL_SUMS, nullptr, nullptr);
-      refinalize(mode, nxlast, fold);
+      finalize(fin_of(g.nz / ox->sums_planes, mode), fold);
       prepped = prefixed = prefixed_f = false;
       return;
     }
@@ -667,22 +662,22 @@ struct Solver final : SolverBase {
     a.inv_n = 1.0 / double(g.nr);
     a.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
     L("xa_sums", [&] { ox->xa(a, XA_SUMS, st); });
-    refinalize(mode, (nxb + kXsLoop - 1) / kXsLoop, fold);
+    finalize(fin_of((nxb + kXsLoop - 1) / kXsLoop, mode), fold);
     prepped = false;
     prefixed = false;
     prefixed_f = false;
   }
 
-  // nx_parts: the x partials written by the last x kernel (k_xsums writes
-  // fewer); fold: FOLD_*
-  void refinalize(int mode, int nx_parts = -1, int fold = FOLD_NONE) {
-    FinArgs fin = fin_of(nx_parts < 0 ? nxlast : nx_parts, mode);
+  void finalize(FinArgs fin, int fold) {
     fin.fold = fold;
     fin.keep = scal_keep.p;
     kept = false;
     L("finalize", [&] { launch_finalize(fin, st); });
     check_launch();
   }
+  // the integrals of uh[cur] again, from the partials of its prefix, under the
+  // targets scal holds now
+  void refinalize(int mode) { finalize(fin_of(parts(prefixed_f), mode), FOLD_NONE); }
 
   // The combine of stage stg: z-forward of tmp1 and s, N^, the ETD combine,
   // and the z-inverse of the next stage field into P, Q.  probe (last ETDRK4
@@ -706,16 +701,15 @@ struct Solver final : SolverBase {
     z.Q = Q.p;
     z.xpart = xpart.p;
     z.dcpart = xdc.p;
-    z.zin = zpart.p + (size_t)zhalf * nzb;
-    z.dcin = dc.p + zhalf;
-    z.nxb = fin_pending ? nxlast : 0;
+    const int hin = (stg - 1) & 1, hout = stg & 1;
+    z.zin = zpart.p + (size_t)hin * nzb;
+    z.dcin = dc.p + hin;
+    z.nxb = stg > 1 && by_plane(ox) ? parts(false) : 0;   // as prefix left them
     z.nzb = nzb;
     z.M1 = p.M1;
     z.M2 = p.M2;
-    fin_pending = false;
-    zhalf = stg & 1;
-    z.part = zpart.p + (size_t)zhalf * nzb;
-    z.dc = dc.p + zhalf;
+    z.part = zpart.p + (size_t)hout * nzb;
+    z.dc = dc.p + hout;
     z.c1 = lt ? lt->c1 : chain_c1.p;
     z.c2 = lt ? lt->c2 : chain_c2.p;
     z.tw = twz.p;
@@ -751,7 +745,7 @@ struct Solver final : SolverBase {
     const int out = 1 - cur;
     ensure_prefixed();
     for (int stg = 1; stg <= sch; ++stg) {
-      if (stg > 1) prefix(FIN_PLAIN, false, 1, true);
+      if (stg > 1) prefix(FIN_PLAIN, false, 1, stg);
       suffix(sch, stg, lt, out, probe);
     }
     // after the last stage P, Q belong to uh[out]
@@ -788,7 +782,6 @@ struct Solver final : SolverBase {
     }
     // the new state, and P, Q prepared for it
     L("z_euler", [&] { oz->zeuler(W.p, uh[out].p, P.p, Q.p, zpart.p, dc.p, g, twz.p, st); });
-    zhalf = 0;
     prepped = true;
     check_launch();
     prefixed_f = false;   // W was consumed
@@ -818,7 +811,7 @@ struct Solver final : SolverBase {
       prefixed_f = false;
       out = eval(time_step);
       cur = out;
-      prefix(FIN_DRIFT, false, 0, false, true);   // and keep the new state's scalars
+      prefix(FIN_DRIFT, false, 0, 0, true);   // and keep the new state's scalars
       return 2;
     }
     ensure_prefixed();
@@ -1150,7 +1143,7 @@ struct Solver final : SolverBase {
       launch_chain_table(chain.p, chain_c1.p, chain_c2.p, mmax + 1, st);
       const int keep = cur, out = 1 - cur;
       for (int stg = 1; stg <= sch; ++stg) {
-        if (stg > 1) prefix(FIN_PLAIN, false, 1, true);
+        if (stg > 1) prefix(FIN_PLAIN, false, 1, stg);
         suffix(sch, stg, nullptr, out);
       }
       cur = out;

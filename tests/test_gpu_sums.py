@@ -30,3 +30,23 @@ def test_integral_sums_in_fp32_cover_one_row(vb, gpu, n, E):
     # first evaluation, whose sums are FP64, and by that of the new state
     A2 = 3.0 * target - s.state()["beta"] - A
     assert abs(A2 / A - 1.0) < E / 3.0 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n,prec", [(32, "FP64"), (64, "FP32_MIXED"), (128, "FP64")])
+def test_residual_between_attempts_changes_nothing(vb, gpu, n, prec):
+    """vb_residual leaves another prefix (and, at 128 in FP64, another number of
+    partial sums) than the attempts around it."""
+    flush_print("residual between attempts", n, prec)
+    eps = 2.0 * 2 * np.pi / n
+    phi, _ = vb.shape(vb.SHAPE_ELLIPSOID, 4, n, n, 1.0, eps)
+    p = vb.params_default(nx=n, nz=n, eps=eps, M1=1e3, M2=1e3, alpha=-1.0, beta=-1.0, time_step=1e-7,
+                          fixed_time_step=0.0, precision=getattr(vb, prec))
+    runs = []
+    for ask in (False, True):
+        s = vb.Solver(p, phi)
+        for k in range(3):
+            r = s.step(4)
+            if ask and k < 2:   # (a query right after it reads the Euler prefix's own sums)
+                assert np.isfinite(s.residual())
+        runs.append((r["energy"], s.query(), s.state(), s.get_phi()))
+    assert runs[0][:3] == runs[1][:3] and np.array_equal(runs[0][3], runs[1][3])
