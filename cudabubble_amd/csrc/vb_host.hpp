@@ -9,20 +9,9 @@
 
 #include "../../include/vesicle.h"
 #include "vb_device.hpp"
+#include "vb_hip.hpp"
 
 namespace vb {
-
-// Every HIP call is checked; a failure becomes VB_ERR_HIP with a message.
-struct HipError {
-  hipError_t err;
-  std::string where;
-};
-#define VB_HIP(call)                                                              \
-  do {                                                                            \
-    hipError_t e_ = (call);                                                       \
-    if (e_ != hipSuccess) throw ::vb::HipError{e_, std::string(#call) + " @ " +   \
-                                                  std::to_string(__LINE__)};      \
-  } while (0)
 
 void set_last_error(const std::string& msg);
 

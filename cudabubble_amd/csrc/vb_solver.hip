@@ -1683,11 +1683,12 @@ struct Solver final : SolverBase {
         s.check_launch();
       }
     } job(*this);
-    struct Held {
-      Staging* s;
-      ~Held() { staging_release(s); }
-    } held{staging_acquire(sizeof(double) * (size_t)g.nr)};
-    staging_copy_out(held.s, job, g.nz, sizeof(double) * (size_t)g.nx * g.ny, host, st);
+    if (staging_copy_out(job, g.nz, sizeof(double) * (size_t)g.nx * g.ny, host, st)) return;
+    // no pinned memory: through the device buffer
+    L("x_c2r", [&] { oxd->xc2r_d(S.p, phid.p, npairs, twxd.p, g, st); });
+    check_launch();
+    VB_HIP(hipMemcpyAsync(host, phid.p, sizeof(double) * (size_t)g.nr, hipMemcpyDeviceToHost, st));
+    VB_HIP(hipStreamSynchronize(st));
   }
 
   void set_phi(const double* host) override {

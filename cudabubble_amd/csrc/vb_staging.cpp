@@ -1,4 +1,4 @@
-// vb_staging.hip -- see vb_staging.hpp.
+// vb_staging.cpp -- see vb_staging.hpp.
 #include "vb_staging.hpp"
 
 #include <algorithm>
@@ -12,22 +12,30 @@
 namespace vb {
 
 namespace {
+struct Block {
+  static constexpr int kSlots = 8;
+  unsigned char* mem = nullptr;   // pinned
+  size_t slot = 0;                // bytes per slot
+  int device = 0;                 // the events' device
+  hipEvent_t ev[kSlots] = {};
+};
+
 constexpr size_t kSmall = (size_t)2 << 20, kLarge = (size_t)4 << 20;   // slot bytes
 constexpr int kThreads = 6, kKeep = 2;
 
 std::mutex g_mu;
-std::vector<Staging*> g_idle;
+std::vector<Block*> g_idle;
 int g_users = 0;
 
-void destroy(Staging* s) {
+void destroy(Block* s) {
   for (auto e : s->ev)
     if (e) (void)hipEventDestroy(e);
   if (s->mem) (void)hipHostFree(s->mem);
   delete s;
 }
-}  // namespace
 
-Staging* staging_acquire(size_t field_bytes) {
+// a block for a field of that size, nullptr where there is no pinned memory
+Block* acquire(size_t field_bytes) {
   const size_t slot = field_bytes <= kSmall ? kSmall : kLarge;
   int dev = 0;
   VB_HIP(hipGetDevice(&dev));
@@ -35,26 +43,25 @@ Staging* staging_acquire(size_t field_bytes) {
     std::lock_guard<std::mutex> l(g_mu);
     for (size_t i = 0; i < g_idle.size(); ++i)
       if (g_idle[i]->slot == slot && g_idle[i]->device == dev) {
-        Staging* s = g_idle[i];
+        Block* s = g_idle[i];
         g_idle.erase(g_idle.begin() + (long)i);
         return s;
       }
   }
-  Staging* s = new Staging;
+  Block* s = new Block;
   s->slot = slot;
   s->device = dev;
-  try {
-    VB_HIP(hipHostMalloc((void**)&s->mem, slot == kSmall ? slot : slot * Staging::kSlots, hipHostMallocDefault));
-    for (auto& e : s->ev) VB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  } catch (...) {
-    destroy(s);
-    throw;
-  }
-  return s;
+  hipError_t e = hipHostMalloc((void**)&s->mem, slot == kSmall ? slot : slot * Block::kSlots, hipHostMallocDefault);
+  if (e != hipSuccess) s->mem = nullptr;
+  for (auto& v : s->ev)
+    if (e == hipSuccess && (e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) != hipSuccess) v = nullptr;
+  if (e == hipSuccess) return s;
+  (void)hipGetLastError();   // not the next call's error
+  destroy(s);
+  return nullptr;
 }
 
-void staging_release(Staging* s) {
-  if (!s) return;
+void release(Block* s) {
   {
     std::lock_guard<std::mutex> l(g_mu);
     int same = 0;
@@ -70,8 +77,11 @@ void staging_release(Staging* s) {
   destroy(s);
 }
 
+void copy_out(Block* s, StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st);
+}  // namespace
+
 void staging_user(int d) {
-  std::vector<Staging*> drop;
+  std::vector<Block*> drop;
   {
     std::lock_guard<std::mutex> l(g_mu);
     g_users += d;
@@ -80,13 +90,28 @@ void staging_user(int d) {
   for (auto* s : drop) destroy(s);
 }
 
-void staging_copy_out(Staging* s, StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st) {
+bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st) {
+  Block* const s = acquire((size_t)items * item_bytes);
+  if (!s) return false;
+  try {
+    copy_out(s, job, items, item_bytes, dst, st);
+  } catch (...) {
+    (void)hipStreamSynchronize(st);   // the kernels launched write to the block
+    release(s);
+    throw;
+  }
+  release(s);
+  return true;
+}
+
+namespace {
+void copy_out(Block* s, StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st) {
   const long long per = std::max<long long>(1, (long long)(s->slot / item_bytes));
   const long long chunks = (items + per - 1) / per;
   unsigned char* const out = static_cast<unsigned char*>(dst);
   auto count = [&](long long c) { return std::min(per, items - c * per); };
   auto copy = [&](long long c) {
-    std::memcpy(out + (size_t)(c * per) * item_bytes, s->mem + (size_t)(c % Staging::kSlots) * s->slot,
+    std::memcpy(out + (size_t)(c * per) * item_bytes, s->mem + (size_t)(c % Block::kSlots) * s->slot,
                 (size_t)count(c) * item_bytes);
   };
   if (chunks == 1) {
@@ -137,18 +162,18 @@ void staging_copy_out(Staging* s, StagingJob& job, long long items, size_t item_
   try {
     long long issued = 0;
     for (long long c = 0; c < chunks; ++c) {
-      for (; issued < chunks && issued < c + Staging::kSlots; ++issued) {
-        if (issued >= Staging::kSlots) {
+      for (; issued < chunks && issued < c + Block::kSlots; ++issued) {
+        if (issued >= Block::kSlots) {
           std::unique_lock<std::mutex> l(mu);
-          const size_t prev = (size_t)(issued - Staging::kSlots);
+          const size_t prev = (size_t)(issued - Block::kSlots);
           // the slot's last chunk: wait for it only where nothing else is in flight
           if (!done[prev] && issued > c) break;
           cv.wait(l, [&] { return done[prev] != 0; });
         }
-        job.produce(issued * per, count(issued), s->mem + (size_t)(issued % Staging::kSlots) * s->slot);
-        VB_HIP(hipEventRecord(s->ev[issued % Staging::kSlots], st));
+        job.produce(issued * per, count(issued), s->mem + (size_t)(issued % Block::kSlots) * s->slot);
+        VB_HIP(hipEventRecord(s->ev[issued % Block::kSlots], st));
       }
-      VB_HIP(hipEventSynchronize(s->ev[c % Staging::kSlots]));
+      VB_HIP(hipEventSynchronize(s->ev[c % Block::kSlots]));
       if (th.empty()) {
         copy(c);
         done[(size_t)c] = 1;
@@ -162,10 +187,10 @@ void staging_copy_out(Staging* s, StagingJob& job, long long items, size_t item_
     }
   } catch (...) {
     join();
-    (void)hipStreamSynchronize(st);   // the kernels launched write to the block
     throw;
   }
   join();   // the workers finish what is ready
 }
+}  // namespace
 
 }  // namespace vb

@@ -11,33 +11,23 @@
 #pragma once
 #include <cstddef>
 
-#include "vb_host.hpp"
+#include "vb_hip.hpp"
 
 namespace vb {
 
-struct Staging {
-  static constexpr int kSlots = 8;
-  unsigned char* mem = nullptr;   // pinned
-  size_t slot = 0;                // bytes per slot
-  int device = 0;                 // the events' device
-  hipEvent_t ev[kSlots] = {};
-};
-
-// A block of one of two slot sizes (fields of up to 2 MB take the small one, a
-// single slot) for the current device; held by the caller until released.
-// Blocks are kept for reuse, at most two of each kind, and freed when the last
-// solver goes.
-Staging* staging_acquire(size_t field_bytes);
-void staging_release(Staging* s);
 void staging_user(int d);   // +1 / -1: a solver was created / destroyed
 
 // Copies a field of `items` items (planes) of item_bytes to dst.  produce(first,
 // count, p) launches on st the kernels that write items [first, first + count)
-// to pinned memory p.  Returns when dst is complete.
+// to pinned memory p.  Returns true when dst is complete, or false, with nothing
+// launched, where no pinned block can be had.
+// A call holds one block, of one of two slot sizes (fields of up to 2 MB take the
+// small one, a single slot), on the current device.  Blocks are kept for reuse,
+// at most two of each kind, and freed when the last solver goes.
 struct StagingJob {
   virtual void produce(long long first, long long count, void* p) = 0;
   virtual ~StagingJob() = default;
 };
-void staging_copy_out(Staging* s, StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st);
+bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st);
 
 }  // namespace vb
