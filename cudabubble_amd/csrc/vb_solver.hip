@@ -136,6 +136,7 @@ struct Solver final : SolverBase {
   hipStream_t st = nullptr;
   bool own_stream = false;
   bool staging_counted = false;
+  size_t phi_read = 0;   // bytes that get_phi has returned (staging_pays)
   const SizeOps<T>* ox = nullptr;
   const SizeOps<T>* oz = nullptr;
   // FP64 operations (state transforms, FP64 queries in mixed mode)
@@ -1683,8 +1684,11 @@ struct Solver final : SolverBase {
         s.check_launch();
       }
     } job(*this);
-    if (staging_copy_out(job, g.nz, sizeof(double) * (size_t)g.nx * g.ny, host, st)) return;
-    // no pinned memory: through the device buffer
+    const size_t plane = sizeof(double) * (size_t)g.nx * g.ny, bytes = plane * (size_t)g.nz;
+    const bool make = staging_pays(phi_read, bytes);
+    phi_read += bytes;
+    if (staging_copy_out(job, g.nz, plane, host, st, make)) return;
+    // no pinned block: through the device buffer
     L("x_c2r", [&] { oxd->xc2r_d(S.p, phid.p, npairs, twxd.p, g, st); });
     check_launch();
     VB_HIP(hipMemcpyAsync(host, phid.p, sizeof(double) * (size_t)g.nr, hipMemcpyDeviceToHost, st));

@@ -34,8 +34,8 @@ void destroy(Block* s) {
   delete s;
 }
 
-// a block for a field of that size, nullptr where there is no pinned memory
-Block* acquire(size_t field_bytes) {
+// a block for a field of that size, nullptr where there is none to be had
+Block* acquire(size_t field_bytes, bool make) {
   const size_t slot = field_bytes <= kSmall ? kSmall : kLarge;
   int dev = 0;
   VB_HIP(hipGetDevice(&dev));
@@ -48,6 +48,7 @@ Block* acquire(size_t field_bytes) {
         return s;
       }
   }
+  if (!make) return nullptr;
   Block* s = new Block;
   s->slot = slot;
   s->device = dev;
@@ -90,8 +91,8 @@ void staging_user(int d) {
   for (auto* s : drop) destroy(s);
 }
 
-bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st) {
-  Block* const s = acquire((size_t)items * item_bytes);
+bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st, bool make) {
+  Block* const s = acquire((size_t)items * item_bytes, make);
   if (!s) return false;
   try {
     copy_out(s, job, items, item_bytes, dst, st);

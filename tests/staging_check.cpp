@@ -142,14 +142,18 @@ struct Fill final : vb::StagingJob {
   }
 };
 
-static void one(long long items, size_t item, unsigned seed) {
+static bool one(long long items, size_t item, unsigned seed, bool make = true) {
   Stream s;
   Fill f(s, item, seed);
   std::vector<unsigned> out((size_t)items * item / 4 + 1, 0xdeadbeefu);
-  CHECK(vb::staging_copy_out(f, items, item, out.data(), reinterpret_cast<hipStream_t>(&s)));
+  if (!vb::staging_copy_out(f, items, item, out.data(), reinterpret_cast<hipStream_t>(&s), make)) {
+    CHECK(!make && f.calls == 0);
+    return false;
+  }
   for (long long i = 0; i < items; ++i)
     for (size_t j = 0; j < item / 4; ++j) CHECK(out[(size_t)i * (item / 4) + j] == pattern(i, j, seed));
   CHECK(out.back() == 0xdeadbeefu);
+  return true;
 }
 
 // sizes: one slot, exactly one, just past it, ragged last chunks, more chunks
@@ -207,7 +211,7 @@ static void launch_failure() {
     std::vector<unsigned> out((size_t)200 * 65536);
     bool threw = false;
     try {
-      (void)vb::staging_copy_out(f, 200, 262144, out.data(), reinterpret_cast<hipStream_t>(&s));
+      (void)vb::staging_copy_out(f, 200, 262144, out.data(), reinterpret_cast<hipStream_t>(&s), true);
     } catch (const std::runtime_error&) {
       threw = true;
     }
@@ -226,13 +230,28 @@ static void no_pinned() {
     Stream s;
     Fill f(s, 262144, 3);
     std::vector<unsigned> out((size_t)items * 65536, 7u);
-    CHECK(!vb::staging_copy_out(f, items, 262144, out.data(), reinterpret_cast<hipStream_t>(&s)));
+    CHECK(!vb::staging_copy_out(f, items, 262144, out.data(), reinterpret_cast<hipStream_t>(&s), true));
     CHECK(f.calls == 0 && out[0] == 7u && out.back() == 7u);
   }
   g_no_pinned = false;
   one(37, 262144, 5);
   vb::staging_user(-1);
   CHECK(g_blocks == 0 && g_events == 0);
+}
+
+// a block is made only where it pays; an idle one serves every reader
+static void make() {
+  vb::staging_user(1);
+  CHECK(!one(16, 131072, 1, false) && g_mallocs == 0);
+  CHECK(one(16, 131072, 1, true) && g_mallocs == 1);
+  CHECK(one(16, 131072, 2, false) && g_mallocs == 1);
+  CHECK(!one(37, 262144, 3, false) && g_mallocs == 1);   // the other kind
+  vb::staging_user(-1);
+  CHECK(g_blocks == 0);
+  const size_t M = (size_t)1 << 20;
+  CHECK(!vb::staging_pays(0, M / 4) && vb::staging_pays(M / 4, M / 4));
+  CHECK(!vb::staging_pays(0, 2 * M) && !vb::staging_pays(60 * M, 2 * M) && vb::staging_pays(62 * M, 2 * M));
+  CHECK(!vb::staging_pays(0, 57 * M) && vb::staging_pays(57 * M, 57 * M) && vb::staging_pays(0, 128 * M));
 }
 
 int main(int argc, char** argv) {
@@ -242,6 +261,7 @@ int main(int argc, char** argv) {
   else if (what == "pool") pool();
   else if (what == "launch_failure") launch_failure();
   else if (what == "no_pinned") no_pinned();
+  else if (what == "make") make();
   else return 2;
   std::printf("ok\n");
   return 0;

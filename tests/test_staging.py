@@ -20,7 +20,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["sizes", "threads", "pool", "launch_failure", "no_pinned"])
+@pytest.mark.parametrize("what", ["sizes", "threads", "pool", "launch_failure", "no_pinned", "make"])
 def test_staging(check, what):
     r = subprocess.run([check, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr[-3000:]
