@@ -52,3 +52,26 @@ def test_gradient_drops_its_nyquist_modes(vb, gpu, oracle_mod, nx, nz, bad):
         g = out()
         c.fftgradient(torch.from_numpy(f).to(gpu), *g)
         assert torch.equal(g[axis], clean[axis]), axis
+
+
+@pytest.mark.parametrize("nx,nz", [(16, 16), (96, 96), (192, 192)])
+def test_get_phi_into_pinned_memory(vb, gpu, nx, nz):
+    """The caller's own pinned buffer, whole or from its middle, gets what a pageable
+    one gets, on the first read and on those that use a staging block."""
+    import ctypes as C
+    import torch
+    flush_print("get_phi pinned", nx, nz)
+    eps = 2.0 * 2 * np.pi / nx
+    phi, _ = vb.shape(vb.SHAPE_TORUS, 5, nx, nz, 1.0, eps)
+    s = vb.Solver(vb.params_default(nx=nx, nz=nz, eps=eps, M1=1e3, M2=1e3, time_step=1e-8, fixed_time_step=1e-8), phi)
+    n = nx * nx * nz
+    buf = torch.full((2 * n + 64,), -7.0, dtype=torch.float64, pin_memory=True)
+    ref = s.get_phi()
+    for off in (0, 3, n):
+        buf.fill_(-7.0)
+        assert vb.lib().vb_get_phi(s.h, C.c_void_p(buf.data_ptr() + 8 * off)) == 0
+        out = buf.numpy()
+        assert np.array_equal(out[off:off + n].reshape(ref.shape), ref)
+        assert (out[:off] == -7.0).all() and (out[off + n:] == -7.0).all()
+        for _ in range(3):
+            assert np.array_equal(s.get_phi(), ref)
