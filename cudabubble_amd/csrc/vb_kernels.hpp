@@ -1165,7 +1165,7 @@ constexpr int zs_lds_bytes() {
 // The stage combine of column group `tile` of one solve, with the
 // workgroup's LDS passed in (smraw: zs_lds_bytes, red: (TB * TF) / 64
 // doubles), so that a launch can run the groups of solves of several sizes.
-template <typename T, int N, int SCH, int STG, int TB, int V, bool PROBE>
+template <typename T, int N, int SCH, int STG, int TB, int V, bool PROBE, bool TAB = false>
 __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, int tid, unsigned char* smraw, double* red,
                                             double* fred) {
   static_assert(!PROBE || (SCH == 4 && STG == 4), "the probe form is the last ETDRK4 stage");
@@ -1211,6 +1211,11 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, int ti
   // The operands of the combine (EH elements at a time, see below)
   constexpr int NH = (!EARLY && (sizeof(T) == 8 || E >= 12 || PROBE) && STG == SCH) ? 2 : 1, EH = E / NH;
   constexpr bool C1 = SCH == 2 || STG != 4, C2 = STG == SCH;
+  // In the table form ETDRK4 stage 2 loads the state whether a lane's column is
+  // there or not: as a branch per element, the compiler waits for each load before
+  // the next branch (4 x 192^3 in one launch 203 -> 219 us).  By value the branches
+  // are the faster form (192^3 FP32 1015 against 1023 us a step).
+  constexpr bool PLAIN = TAB && SCH == 4 && STG == 2 && !EARLY;
   cpx<double> ur[USES_U ? EH : 1];
   cpx<T> pa[(SCH == 4 && STG >= 3) || (SCH == 2 && STG == 2) ? EH : 1];
   cpx<T> pb[(SCH == 4 && STG == 4) ? EH : 1];
@@ -1222,7 +1227,12 @@ __device__ __forceinline__ void zstage_body(const ZsArgs<T>& a, int tile, int ti
     for (int iq = 0; iq < EH; ++iq) {
       const int e = hh * EH + iq;
       const long long ib = ib0 + (long long)(j + TF * e) * TB;
-      if constexpr (USES_U) ur[iq] = id.valid ? ld_nt(a.uh + ib) : mk<double>(0.0, 0.0);
+      if constexpr (USES_U && PLAIN) {
+        const cpx<double> u = ld_nt(a.uh + ib);   // (the group's whole run is there)
+        ur[iq] = mk<double>(id.valid ? u.x : 0.0, id.valid ? u.y : 0.0);
+      } else if constexpr (USES_U) {
+        ur[iq] = id.valid ? ld_nt(a.uh + ib) : mk<double>(0.0, 0.0);
+      }
       if constexpr (SCH == 4 && STG == 3) pa[iq] = ld_nt(a.pre + ib);
       if constexpr (SCH == 4 && STG == 4) { pa[iq] = ld_nt(a.Na + ib); pb[iq] = ld_nt(a.Nb + ib); }
       if constexpr (SCH == 2 && STG == 2) pa[iq] = ld_nt(a.Na + ib);
@@ -1431,7 +1441,7 @@ __global__ void __launch_bounds__((TB * TFof<N, V>())) k_zstage(ZsArgs<T> a0, co
   __shared__ __align__(16) unsigned char smraw[zs_lds_bytes<T, N, SCH, STG, TB, V>()];
   __shared__ double red[(TB * TFof<N, V>()) / 64];
   __shared__ double fred[4 * ((TB * TFof<N, V>()) / 64)];
-  zstage_body<T, N, SCH, STG, TB, V, PROBE>(a, pair_item(int(blockIdx.x), int(gridDim.x)), int(threadIdx.x), smraw,
+  zstage_body<T, N, SCH, STG, TB, V, PROBE, TAB>(a, pair_item(int(blockIdx.x), int(gridDim.x)), int(threadIdx.x), smraw,
                                                 red, fred);
 }
 
