@@ -33,7 +33,13 @@ namespace vb {
 // and a line that two XCDs write in parts is worse still.  So the prefix kernels
 // give plane z to XCD (z / 2) mod 8 in all of them, and the column groups that
 // share 128-byte lines (two planes of a group-major spectrum, two 8-column tiles
-// of a row) run on one XCD.
+// of a row) run on one XCD.  Past a cache's size a batch's own locality
+// goes by the order instead (in_order): with P and Q of all its solves past the
+// L2s (32 MB) the x kernel takes rows in memory order, past the memory-side cache
+// (256 MB) the y passes take columns so.  us per step, both on their XCDs / x in
+// order / both in order: 2, 3, 4 x 256^3 FP32 (270, 405, 540 MB) 4586, 6976, 9589 /
+// 4534, 6970, 9534 / 4420, 6892, 9427; 4 x 192^3 (229 MB) 3476 / 3472 / 3511; 8 x
+// 192^3 7420 / 7368 / 7420; 4 x 128 x 128 x 32 (18 MB) 420 / 461 / 461.
 constexpr int kXcds = 8;
 constexpr int kCus = 256;    // compute units
 // item of workgroup b (of n) when items 2i and 2i + 1 are to share an XCD; a
@@ -292,6 +298,7 @@ struct XaArgs {
   long long npairs;
   double eps, kappa, D, inv_n;
   Rows rl;
+  int in_order;      // table form, read from the by-value struct: rows in memory order (see kXcds)
 };
 
 // Every pipeline kernel takes its argument struct by value, or (TAB, a
@@ -432,7 +439,8 @@ template <typename T, int N> constexpr int xrwaves() { return (sizeof(T) == 4 &&
 // state (T = double).
 template <typename T, int N, bool TAB = false, int XP = xrplan<T, N>(), bool SUMS = false>
 __global__ void __launch_bounds__((xrthreads<T, N, XP>()), (xrwaves<T, N>())) k_xrow(XaArgs<T> a0, const XaArgs<T>* tab) {
-  const XaArgs<T> a = TAB ? tab[blockIdx.z] : a0;
+  // (a batch: the last solve first, its arrays are the ones still cached)
+  const XaArgs<T> a = TAB ? tab[gridDim.z - 1 - blockIdx.z] : a0;
   constexpr int E = Plan<N, XP>::E, TF = N / E, RL = 2 * xlanes<T, N>(), LL = row_lds_len<N>(),
                 NT = xrthreads<T, N, XP>();
   static_assert(NT % 64 == 0, "whole waves");
@@ -441,7 +449,10 @@ __global__ void __launch_bounds__((xrthreads<T, N, XP>()), (xrwaves<T, N>())) k_
   const int lane = threadIdx.x / TF, j = threadIdx.x % TF;
   RowLds<T> lds{sm + lane * LL};
   const long long nrows = 2 * a.npairs;
-  long long row = (long long)xgroup<RL>(a.rl, nrows) * RL + lane;
+  const bool in_order = TAB && a0.in_order;
+  // (the partials go by row group, the same for a solve alone and in a batch)
+  const unsigned grp = in_order ? blockIdx.x : xgroup<RL>(a.rl, nrows);
+  long long row = (long long)grp * RL + lane;
   const bool valid = row < nrows;
   if (!valid) row = nrows - 1;
   const double eps = a.eps, kappa = a.kappa, ieps = 1.0 / eps;
@@ -490,7 +501,7 @@ __global__ void __launch_bounds__((xrthreads<T, N, XP>()), (xrwaves<T, N>())) k_
     }
   }
   if constexpr (SUMS) {
-    block_sum_store<3, NT>(acc, red, a.part + 3 * (long long)blockIdx.x);
+    block_sum_store<3, NT>(acc, red, a.part + 3 * (long long)grp);
     return;
   }
   if constexpr (DCS && NT == 64) {
@@ -500,21 +511,21 @@ __global__ void __launch_bounds__((xrthreads<T, N, XP>()), (xrwaves<T, N>())) k_
                                   a.Ts + a.rl.nyq(row, N / 2), T(1), valid);
     __shared__ double wred[5 * 64];
     const double v5[5] = {acc[0], acc[1], acc[2], dcs[0], dcs[1]};
-    double* const o3 = a.part + 3 * (long long)blockIdx.x;
-    double* const o2 = a.dcpart ? a.dcpart + 2 * (long long)blockIdx.x : nullptr;
+    double* const o3 = a.part + 3 * (long long)grp;
+    double* const o2 = a.dcpart ? a.dcpart + 2 * (long long)grp : nullptr;
     wave_sum_store<5>(v5, wred, o3, o2);
     return;
   }
   if constexpr (DCS) {
     if (a.dcpart) {
       __shared__ double red2[2 * (NT / 64)];
-      block_sum_store<2, NT>(dcs, red2, a.dcpart + 2 * (long long)blockIdx.x);
+      block_sum_store<2, NT>(dcs, red2, a.dcpart + 2 * (long long)grp);
     }
   }
   fft<T, N, -1, XP>(x, j, a.tw, lds);   // tmp1 + i s
   unpack_store<T, N, XP, false>(x, j, lds, a.Tt + a.rl.off(row), a.Tt + a.rl.nyq(row, N / 2), a.Ts + a.rl.off(row),
                                 a.Ts + a.rl.nyq(row, N / 2), T(1), valid);
-  block_sum_store<3, NT>(acc, red, a.part + 3 * (long long)blockIdx.x);
+  block_sum_store<3, NT>(acc, red, a.part + 3 * (long long)grp);
 }
 
 // The partial sums of v and (v^2-1)^2 from P alone, for the targets' drift in
@@ -639,7 +650,7 @@ struct YIdx {
 // t: the workgroup's column group (blockIdx.x unless the launch has extra
 // workgroups in front)
 template <int TB>
-__device__ __forceinline__ YIdx yidx(const Geo& g, long long t) {
+__device__ __forceinline__ YIdx yidx(const Geo& g, long long t, bool in_order) {
   const int c = threadIdx.x % TB;
   YIdx r;
   int z, kx;
@@ -649,10 +660,15 @@ __device__ __forceinline__ YIdx yidx(const Geo& g, long long t) {
     const int tpr = (g.nx / 2) / TB;
     const int nnyq = (g.nz + TB - 1) / TB;
     if (t >= nnyq) {
-      // two planes at a time per XCD, their tiles alternating
-      const unsigned i = unsigned(t - nnyq), q = i / kXcds, t2 = 2 * unsigned(tpr), q2 = q % t2;
-      z = int(((q / t2) * kXcds + i % kXcds) * 2 + q2 % 2);
-      kx = int(q2 / 2) * TB + c;
+      const unsigned i = unsigned(t - nnyq);
+      if (in_order) {
+        z = int(i / unsigned(tpr));
+        kx = int(i % unsigned(tpr)) * TB + c;
+      } else {   // two planes at a time per XCD, their tiles alternating
+        const unsigned q = i / kXcds, t2 = 2 * unsigned(tpr), q2 = q % t2;
+        z = int(((q / t2) * kXcds + i % kXcds) * 2 + q2 % 2);
+        kx = int(q2 / 2) * TB + c;
+      }
       r.valid = true;
     } else {   // Nyquist column of TB planes
       z = int(t * TB + c);
@@ -677,7 +693,7 @@ __device__ __forceinline__ YIdx yidx(const Geo& g, long long t) {
 }
 template <int TB>
 __device__ __forceinline__ YIdx yidx(const Geo& g) {
-  return yidx<TB>(g, blockIdx.x);
+  return yidx<TB>(g, blockIdx.x, false);
 }
 
 template <typename T>
@@ -693,6 +709,7 @@ struct YArgs {
   cpx<T>* o1;
   int ztb;      // GM: the z kernels' column tile
   int nzt;      // GM: planes of the whole grid (g may be a slab of it)
+  int in_order; // table form, read from the by-value struct: columns in memory order (see kXcds)
 };
 
 // Position of spectral element (z, ky, kx) in the group-major layout of the z
@@ -741,7 +758,7 @@ __global__ void __launch_bounds__((TB * TFof<N, V>())) k_ypass(YArgs<T> a0, cons
   cpx<T>* buf = blockIdx.y ? a.b1 : a.b0;
   const int j = threadIdx.x / TB;
   ColLds<T, TB> lds{sm + threadIdx.x % TB};
-  const YIdx id = yidx<TB>(g, (long long)blockIdx.x - a.fin_on - a.pad);
+  const YIdx id = yidx<TB>(g, (long long)blockIdx.x - a.fin_on - a.pad, TAB && a0.in_order);
   if ((int)blockIdx.x < a.fin_on + a.pad) return;
   cpx<T>* col = buf + id.base;
   cpx<T> x[E];

@@ -79,7 +79,7 @@ struct Launch {
     const int nf = fin_groups(fin);
     const int pad = ypad(g, nf);
     const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf + pad), unsigned(narr)), bl(CT);
-    YArgs<T> a{b0, b1, tw, g, fin ? *fin : FinArgs{}, nf, pad, nullptr, nullptr, 0, g.nz};
+    YArgs<T> a{b0, b1, tw, g, fin ? *fin : FinArgs{}, nf, pad, nullptr, nullptr, 0, g.nz, 0};
     if (g_recorder) return record_launch(&launch_tab, sign < 0 ? OP_Y_FWD : OP_Y_INV, a, grid, bl);
     if (sign < 0)
       hipLaunchKernelGGL((k_ypass<T, N, -1, CB, false, CV>), grid, bl, 0, s, a, nullptr);
@@ -93,7 +93,7 @@ struct Launch {
     const int nf = fin_groups(fin);
     const int pad = ypad(g, nf);
     const dim3 grid(unsigned(ygroups(g, CB)) + unsigned(nf + pad), 2u), bl(CT);
-    YArgs<T> a{const_cast<cpx<T>*>(b0), const_cast<cpx<T>*>(b1), tw, g, fin ? *fin : FinArgs{}, nf, pad, o0, o1, ztb, nzt};
+    YArgs<T> a{const_cast<cpx<T>*>(b0), const_cast<cpx<T>*>(b1), tw, g, fin ? *fin : FinArgs{}, nf, pad, o0, o1, ztb, nzt, 0};
     if (g_recorder) return record_launch(&launch_tab, OP_Y_FWD_GM, a, grid, bl);
     hipLaunchKernelGGL((k_ypass<T, N, -1, CB, false, CV, true>), grid, bl, 0, s, a, nullptr);
   }
@@ -229,25 +229,31 @@ struct Launch {
   // the table form of a recorded launch, over `lanes` solves (blockIdx.z)
   static void launch_tab(int op, const void* tab, dim3 gr, dim3 bl, int lanes, hipStream_t s) {
     gr.z = unsigned(lanes);
+    // the workgroups' order (see kXcds): by the bytes of the batch's P and Q
+    auto past = [&](double modes, int mb) { return int(2.0 * sizeof(cpx<T>) * modes * lanes > double(mb << 20)); };
+    XaArgs<T> xa{};
+    YArgs<T> ya{};
+    xa.in_order = past(double(gr.x) * 2 * G * (N / 2), 32);
+    ya.in_order = past(double(gr.x) * CB * N, 256);
     switch (op) {
       case OP_XA_RS:
-        hipLaunchKernelGGL((k_xrow<T, N, true, XR, true>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab);
+        hipLaunchKernelGGL((k_xrow<T, N, true, XR, true>), gr, bl, 0, s, xa, (const XaArgs<T>*)tab);
         break;
       case OP_XA_F: hipLaunchKernelGGL((k_xa<T, N, true>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab); break;
       case OP_XA_S:
-        hipLaunchKernelGGL((k_xrow<T, N, true, XR>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab);
+        hipLaunchKernelGGL((k_xrow<T, N, true, XR>), gr, bl, 0, s, xa, (const XaArgs<T>*)tab);
         break;
       case OP_XA_SUMS:
         hipLaunchKernelGGL((k_xsums<T, N, true>), gr, bl, 0, s, XaArgs<T>{}, (const XaArgs<T>*)tab);
         break;
       case OP_Y_FWD:
-        hipLaunchKernelGGL((k_ypass<T, N, -1, CB, true, CV>), gr, bl, 0, s, YArgs<T>{}, (const YArgs<T>*)tab);
+        hipLaunchKernelGGL((k_ypass<T, N, -1, CB, true, CV>), gr, bl, 0, s, ya, (const YArgs<T>*)tab);
         break;
       case OP_Y_INV:
-        hipLaunchKernelGGL((k_ypass<T, N, +1, CB, true, CV>), gr, bl, 0, s, YArgs<T>{}, (const YArgs<T>*)tab);
+        hipLaunchKernelGGL((k_ypass<T, N, +1, CB, true, CV>), gr, bl, 0, s, ya, (const YArgs<T>*)tab);
         break;
       case OP_Y_FWD_GM:
-        hipLaunchKernelGGL((k_ypass<T, N, -1, CB, true, CV, true>), gr, bl, 0, s, YArgs<T>{}, (const YArgs<T>*)tab);
+        hipLaunchKernelGGL((k_ypass<T, N, -1, CB, true, CV, true>), gr, bl, 0, s, ya, (const YArgs<T>*)tab);
         break;
       case OP_ZLAP:
         hipLaunchKernelGGL((k_zlap<T, N, CB, true, CV>), gr, bl, 0, s, ZlArgs<T>{}, (const ZlArgs<T>*)tab);
