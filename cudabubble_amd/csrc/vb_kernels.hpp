@@ -110,7 +110,8 @@ template <typename T, int N> constexpr int zsplan() {
 // workgroup barrier and a short grid spreads over more CUs (a 32^3 FP64 combine
 // was 9 workgroups of 256 threads): with the combine's operands and
 // coefficients loaded before its transforms (EARLY), 9.4 -> 6.4 us at 32^3 FP64
-// and 10.5 -> 8.6 us (stage 1 9.6 -> 6.4) at 64^3 FP32.  Above, the column
+// and 10.5 -> 8.6 us (stage 1 9.6 -> 6.4) at 64^3 FP32 (under planes of 192^2 and
+// more tbw_wide instead).  Above, the column
 // width, except FP64 at 64 and 128 (whole 128-byte lines, with their plans of four
 // elements) and FP32 at 256 and 512, 8 columns.  At 256 in FP32 (256-thread workgroups,
 // two or three per CU) 8 measured 6-14 % faster per stage than 16: their inputs
@@ -127,6 +128,10 @@ template <typename T, int N> constexpr int tbw() {
 // The other z tile a kernel schedule can select: the column width where tbw
 // is narrower, else half of it.
 template <typename T, int N> constexpr int tbw_alt() { return tbw<T, N>() < colw<T, N>() ? colw<T, N>() : tbw<T, N>() / 2; }
+
+// The z tile that short lengths take under a large plane, on the default plan
+// (get_zops); 0 where there is none.
+template <typename T, int N> constexpr int tbw_wide() { return N == 32 || N == 64 ? 32 : N == 128 && sizeof(T) == 8 ? 16 : 0; }
 
 // Z_p = A_ext(p) + i * B_ext(p): Hermitian extension along x of two half
 // spectra (rows A and B, whose Nyquist elements are at An and Bn).  The

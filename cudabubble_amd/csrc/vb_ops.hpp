@@ -176,6 +176,28 @@ inline const SizeOps<T>* get_ops(int N) {
   return get_ops<T>(N, sc);
 }
 
+// The z kernels' table of a grid: under a large plane the short lengths take the
+// wide tile on the default plan (kWideZ, tbw_wide) in place of one wave's columns.
+// There the combines stream from memory, and 64-byte pieces of P and Q cost more
+// than the barriers and the longer threads.  us per step, the narrow tile / this:
+//   FP32 192 x 64 480 / 466, 256 x 64 661 / 645, 512 x 64 2485 / 2300, batches of 8
+//   of 192 x 64 2490 / 2375, 4 of 256 x 64 2225 / 2100; 256 x 32 447 / 436;
+//   128 x 32 215 / 255
+//   FP64 192 x 64 710 / 704, 512 x 64 4290 / 4010; 256 x 128 1797 / 1801, 384 x 128
+//   4590 / 4395, two of 256 x 128 3890 / 3750, but 192 x 128 1209 / 1222; 512 x 32
+//   2155 / 2120, but 256 x 32 562 / 592
+// mixed: the FP64 integrals of a mixed solver, whose tile should be the FP32 one's
+// (a pass regroups the state where it is not).
+constexpr int kWideZ = 8;   // a schedule number past those that can be selected
+template <typename T>
+inline const SizeOps<T>* get_zops(int nx, int nz, bool mixed) {
+  const SizeOps<T>* const o = get_ops<T>(nz);
+  const int from = sizeof(T) == 4 || mixed || nz == 64 ? 192 : nz == 128 ? 256 : 384;
+  if (nx < from || o != get_ops<T>(nz, 0)) return o;   // (a schedule that was chosen stays)
+  const SizeOps<T>* const w = get_ops<T>(nz, kWideZ);
+  return w ? w : o;
+}
+
 inline bool size_supported(int N) {
   switch (N) {
 #define VB_CASE(n) case n: return true;

@@ -22,9 +22,10 @@ template <typename T, int N, int SC = 0>
 struct Launch {
   static constexpr int TF = TFof<N>();
   static constexpr int G = xlanes<T, N>();
-  static constexpr int TB = (SC & 1) ? tbw_alt<T, N>() : tbw<T, N>();
+  static constexpr int TB = (SC & kWideZ) ? tbw_wide<T, N>() : (SC & 1) ? tbw_alt<T, N>() : tbw<T, N>();
+  static constexpr int ZV = (SC & kWideZ) ? 0 : zsplan<T, N>();   // plan of the z kernels
   static constexpr int XR = (SC & 2) ? xrplan_alt<T, N>() : xrplan<T, N>();
-  static constexpr int YT = TB * TFof<N, zsplan<T, N>()>();
+  static constexpr int YT = TB * TFof<N, ZV>();
   static constexpr int CV = colplan<T, N>();          // plan of the y passes and the z Laplacian
   static constexpr int CB = colw<T, N>();             // their columns per workgroup
   static constexpr int CT = CB * TFof<N, CV>();       // and threads per workgroup
@@ -100,9 +101,9 @@ struct Launch {
   static unsigned zgrid(const Geo& g) { return unsigned(zgroups(g, TB)); }
   static void zpass(cpx<T>* b, int sign, const Geo& g, const cpx<T>* tw, hipStream_t s) {
     if (sign < 0)
-      hipLaunchKernelGGL((k_zpass<T, N, -1, TB>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
+      hipLaunchKernelGGL((k_zpass<T, N, -1, TB, ZV>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
     else
-      hipLaunchKernelGGL((k_zpass<T, N, +1, TB>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
+      hipLaunchKernelGGL((k_zpass<T, N, +1, TB, ZV>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
   }
   // (FP32 at 192 would spill its 24 elements' v and f: a step 199 -> 209 us)
   static constexpr bool kXePlane = PairCfg<T, N>::ok && N <= 128;
@@ -112,7 +113,7 @@ struct Launch {
   }
   static void zeuler(const cpx<T>* W, cpx<double>* uh, cpx<T>* P, cpx<T>* Q, double* part, double* dc, const Geo& g,
                      const cpx<T>* tw, hipStream_t s) {
-    hipLaunchKernelGGL((k_zeuler<T, N, TB>), dim3(zgrid(g)), dim3(YT), 0, s, W, uh,
+    hipLaunchKernelGGL((k_zeuler<T, N, TB, ZV>), dim3(zgrid(g)), dim3(YT), 0, s, W, uh,
                        (ZprArgs<T>{nullptr, P, Q, part, dc, tw, g}));
   }
   static void zmul(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,
@@ -120,15 +121,15 @@ struct Launch {
     const ZmArgs<T> a{in, out, tw, gi, go};
     const dim3 gr(unsigned(zgroups(go.aligned ? go : gi, TB))), bl(YT);
     if (sign < 0) {
-      hipLaunchKernelGGL((k_zmul<T, N, -1, TB, ZM_ONE>), gr, bl, 0, s, a);
+      hipLaunchKernelGGL((k_zmul<T, N, -1, TB, ZM_ONE, ZV>), gr, bl, 0, s, a);
       return;
     }
     switch (op) {
-      case ZM_LAP: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_LAP>), gr, bl, 0, s, a); break;
-      case ZM_DX: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DX>), gr, bl, 0, s, a); break;
-      case ZM_DY: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DY>), gr, bl, 0, s, a); break;
-      case ZM_DZ: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DZ>), gr, bl, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_ONE>), gr, bl, 0, s, a); break;
+      case ZM_LAP: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_LAP, ZV>), gr, bl, 0, s, a); break;
+      case ZM_DX: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DX, ZV>), gr, bl, 0, s, a); break;
+      case ZM_DY: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DY, ZV>), gr, bl, 0, s, a); break;
+      case ZM_DZ: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DZ, ZV>), gr, bl, 0, s, a); break;
+      default: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_ONE, ZV>), gr, bl, 0, s, a); break;
     }
   }
   static void pair_r2c(const T* u, cpx<T>* so, double scl, const Geo& g, const cpx<T>* tw, hipStream_t s) {
@@ -153,12 +154,11 @@ struct Launch {
     const dim3 gr(zgrid(g)), bl(YT);
     ZprArgs<T> a{vh, P, Q, part, dc, tw, g};
     if (g_recorder) return record_launch(&launch_tab, OP_ZPREP, a, gr, bl);
-    hipLaunchKernelGGL((k_zprep<T, N, TB>), gr, bl, 0, s, a, nullptr);
+    hipLaunchKernelGGL((k_zprep<T, N, TB, false, ZV>), gr, bl, 0, s, a, nullptr);
   }
   template <int SCH, int STG, bool TAB, bool PROBE = false>
   static void zs_launch(dim3 gr, const ZsArgs<T>& a, const ZsArgs<T>* tab, hipStream_t s) {
-    hipLaunchKernelGGL((k_zstage<T, N, SCH, STG, TB, TAB, zsplan<T, N>(), PROBE>), gr,
-                       dim3(TB * TFof<N, zsplan<T, N>()>()), 0, s, a, tab);
+    hipLaunchKernelGGL((k_zstage<T, N, SCH, STG, TB, TAB, ZV, PROBE>), gr, dim3(YT), 0, s, a, tab);
   }
   template <bool TAB>
   static void zs_dispatch(int sch, int stg, dim3 gr, const ZsArgs<T>& a, const ZsArgs<T>* tab, hipStream_t s) {
@@ -180,7 +180,7 @@ struct Launch {
     const dim3 gr(zgrid(a.g));
     if (g_recorder)
       return record_launch(&launch_tab, stg == 5 ? OP_ZS44P : (sch == 4 ? OP_ZS41 : OP_ZS21) + (stg - 1), a, gr,
-                           dim3(TB * TFof<N, zsplan<T, N>()>()));
+                           dim3(YT));
     zs_dispatch<false>(sch, stg, gr, a, nullptr, s);
   }
 
@@ -259,7 +259,7 @@ struct Launch {
         hipLaunchKernelGGL((k_zlap<T, N, CB, true, CV>), gr, bl, 0, s, ZlArgs<T>{}, (const ZlArgs<T>*)tab);
         break;
       case OP_ZPREP:
-        hipLaunchKernelGGL((k_zprep<T, N, TB, true>), gr, bl, 0, s, ZprArgs<T>{}, (const ZprArgs<T>*)tab);
+        hipLaunchKernelGGL((k_zprep<T, N, TB, true, ZV>), gr, bl, 0, s, ZprArgs<T>{}, (const ZprArgs<T>*)tab);
         break;
       case OP_ZS41: case OP_ZS42: case OP_ZS43: case OP_ZS44:
         zs_dispatch<true>(4, op - OP_ZS41 + 1, gr, ZsArgs<T>{}, (const ZsArgs<T>*)tab, s);
@@ -316,6 +316,13 @@ namespace vb {
 // the launch table of schedule sc of length N (nullptr: not compiled)
 template <typename T, int N>
 const SizeOps<T>* ops_table(int sc) {
+  if (sc == kWideZ) {
+    if constexpr (tbw_wide<T, N>() != 0) {
+      static const SizeOps<T> w = Launch<T, N, kWideZ>::table();
+      return &w;
+    }
+    return nullptr;
+  }
   if (sc < 0 || sc >= schedules<T, N>()) return nullptr;
   static const SizeOps<T> t[4] = {
       Launch<T, N, 0>::table(), Launch<T, N, (schedules<T, N>() > 1 ? 1 : 0)>::table(),

@@ -275,9 +275,9 @@ struct Solver final : SolverBase {
   Solver(const vb_params& pp, hipStream_t shared) {
     p = pp;
     ox = get_ops<T>(p.nx);
-    oz = get_ops<T>(p.nz);
+    oz = get_zops<T>(p.nx, p.nz, kMixed);
     oxd = get_ops<double>(p.nx);
-    ozd = get_ops<double>(p.nz);
+    ozd = get_zops<double>(p.nx, p.nz, kMixed);
     setup_geo();
     if (shared) {
       st = shared;
