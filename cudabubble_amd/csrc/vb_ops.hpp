@@ -114,8 +114,10 @@ struct SizeOps {
   int plane_min_nz;   // the planes from which it is used
   void (*plane)(const PlaneArgs<T>& a, int mode, hipStream_t s);
   // The Forward-Euler update with x and y of a plane in one kernel (nullptr
-  // where a plane does not fit; nz partials of rhs^2), and the z pass that
+  // where a plane does not fit; nz partials of rhs^2), used from xe_min_nz planes
+  // on, and the z pass that
   // follows it: the new state from W, and the prepared field's P, Q
+  int xe_min_nz;
   void (*xe_plane)(const XeArgs<T>& a, const Geo& g, hipStream_t s);
   void (*zeuler)(const cpx<T>* W, cpx<double>* uh, cpx<T>* P, cpx<T>* Q, double* part, double* dc, const Geo& g,
                  const cpx<T>* tw, hipStream_t s);

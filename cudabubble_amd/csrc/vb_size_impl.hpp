@@ -105,8 +105,10 @@ struct Launch {
     else
       hipLaunchKernelGGL((k_zpass<T, N, +1, TB, ZV>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
   }
-  // (FP32 at 192 would spill its 24 elements' v and f: a step 199 -> 209 us)
-  static constexpr bool kXePlane = PairCfg<T, N>::ok && N <= 128;
+  // FP32 at 192 would spill its 24 elements' v and f (a step 199 -> 209 us); FP64 at
+  // 128 spilled 60 registers: nz = 16, 64, 128, 256 62, 84, 110, 169 us a step against
+  // 46, 76, 106, 158 with separate kernels.  FP32 at 128 spills 18 and is faster.
+  static constexpr bool kXePlane = PairCfg<T, N>::ok && (N <= 96 || (N == 128 && sizeof(T) == 4));
   static void xe_plane(const XeArgs<T>& a, const Geo& g, hipStream_t s) {
     if constexpr (kXePlane)
       hipLaunchKernelGGL((k_xe_plane<T, N>), dim3(unsigned(g.nz)), dim3(PairCfg<T, N>::NA), 0, s, a, g);
@@ -302,6 +304,11 @@ struct Launch {
     o.plane_min_nz = plane_min_nz<T, N>();
     o.plane_euler = PlaneCfg<T, N>::ok;
     o.xe_plane = kXePlane ? &xe_plane : nullptr;
+    // few planes leave the chip idle.  us per step (and with a residual after it),
+    // one kernel / separate ones: FP32 128 nz = 16 43.8 (101.5) / 39.1 (87.9), 48 59.0
+    // (117) / 54.4 (103), 64 61.9 (121) / 62.1 (112), 96 67.6 / 70.0, 128 69.8 / 75.2;
+    // FP64 96 nz = 16 50.9 (106) / 50.2 (99), 32 56.3 / 57.6; FP32 96 nz = 16 35.3 / 37.6
+    o.xe_min_nz = N == 128 ? 96 : N == 96 && sizeof(T) == 8 ? 32 : 0;
     o.zeuler = &zeuler;
     o.zmul = &zmul;
     o.pair_r2c = PairCfg<T, N>::ok ? &pair_r2c : nullptr;

@@ -509,7 +509,7 @@ struct Solver final : SolverBase {
   void spectral_lap(cpx<T>* b, const FinArgs* fin, bool y_done) {
     if (!y_done) L("y_fwd", [&] { ox->ypass(b, nullptr, 1, -1, g, twx.p, nullptr, st); });
     L(fin ? "z_lap_fin" : "z_lap", [&] { oz->zlap(b, g, twz.p, fin, st); });
-    if (!ox->xe_plane) L("y_inv", [&] { ox->ypass(b, nullptr, 1, +1, g, twx.p, nullptr, st); });
+    if (!xe_by_plane()) L("y_inv", [&] { ox->ypass(b, nullptr, 1, +1, g, twx.p, nullptr, st); });
   }
 
   void fold_keep(FinArgs& fin) {
@@ -521,6 +521,8 @@ struct Solver final : SolverBase {
   // whether a whole plane at a time is the way (SizeOps::plane)
   template <typename X>
   bool by_plane(const SizeOps<X>* o) const { return o->plane && g.nz >= o->plane_min_nz; }
+
+  bool xe_by_plane() const { return ox->xe_plane && g.nz >= ox->xe_min_nz; }
 
   // one plane kernel over the prepared field (PlaneMode)
   void plane(int mode, cpx<T>* tt, cpx<T>* ts) {
@@ -775,7 +777,7 @@ struct Solver final : SolverBase {
     e.rl = Rows{g.ny, g.pitch, g.pp, g.nq};
     e.part = nullptr;
     e.tp = tdev;
-    if (ox->xe_plane) {
+    if (xe_by_plane()) {
       L("xe_plane", [&] { ox->xe_plane(e, g, st); });
     } else {
       L("xe", [&] { ox->xe(e, st); });
@@ -1767,7 +1769,7 @@ struct Solver final : SolverBase {
     if (!W.p) W.alloc((size_t)g.ncp);
     if (!v.p) v.alloc((size_t)g.nr);
     if (!f.p) f.alloc((size_t)g.nr);
-    const int nres = ox->xe_plane ? g.nz : nxb;
+    const int nres = xe_by_plane() ? g.nz : nxb;
     if (!rpart.p) rpart.alloc((size_t)nres);
     ensure_prefixed(true);
     XeArgs<T> e;
@@ -1787,7 +1789,7 @@ struct Solver final : SolverBase {
     e.part = rpart.p;
     e.tp = nullptr;
     L("xe_resid", [&] {
-      if (ox->xe_plane) ox->xe_plane(e, g, st);
+      if (xe_by_plane()) ox->xe_plane(e, g, st);
       else ox->xe(e, st);
     });
     check_launch();
