@@ -280,13 +280,13 @@ struct CalcImpl {
   template <typename T>
   void fwd_xy(const Fft<T>& f, const T* u, cpx<T>* s, const Geo& gl) {
     const double n = 1.0 / double(g.nr);
-    if (f.ox->pair_r2c && !gl.aligned) return f.ox->pair_r2c(u, s, n, gl, f.twx, st);
+    if (f.ox->pair_r2c && !gl.aligned && g.nz >= f.ox->pair_r2c_nz) return f.ox->pair_r2c(u, s, n, gl, f.twx, st);
     f.ox->xr2c(u, s, npairs, f.twx, n, gl, st);
     f.ox->ypass(s, nullptr, 1, -1, gl, f.twx, nullptr, st);
   }
   template <typename T>
   void inv_xy(const Fft<T>& f, cpx<T>* s, T* u, const Geo& gl) {   // s is overwritten
-    if (f.ox->pair_c2r && !gl.aligned) return f.ox->pair_c2r(s, u, gl, f.twx, st);
+    if (f.ox->pair_c2r && !gl.aligned && g.nz >= f.ox->pair_c2r_nz) return f.ox->pair_c2r(s, u, gl, f.twx, st);
     f.ox->ypass(s, nullptr, 1, +1, gl, f.twx, nullptr, st);
     f.ox->xc2r(s, u, npairs, f.twx, gl, st);
   }

@@ -126,7 +126,9 @@ struct SizeOps {
   void (*zmul)(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,
                hipStream_t s);
   // x and y transforms of whole planes in LDS (k_pair), real rows to half
-  // spectra times scl and back; nullptr where a plane does not fit
+  // spectra times scl and back; nullptr where a plane does not fit.  Used from
+  // pair_r2c_nz and pair_c2r_nz planes on.
+  int pair_r2c_nz, pair_c2r_nz;
   void (*pair_r2c)(const T* u, cpx<T>* so, double scl, const Geo& g, const cpx<T>* tw, hipStream_t s);
   void (*pair_c2r)(const cpx<T>* si, T* uo, const Geo& g, const cpx<T>* tw, hipStream_t s);
 };

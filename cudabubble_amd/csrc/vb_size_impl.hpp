@@ -311,6 +311,13 @@ struct Launch {
     o.xe_min_nz = N == 128 ? 96 : N == 96 && sizeof(T) == 8 ? 32 : 0;
     o.zeuler = &zeuler;
     o.zmul = &zmul;
+    // few planes leave the chip idle.  A call, separate kernels / by plane, us: r2c FP64
+    // 128 nz = 16 23.1 / 27.0, 32 27.0 / 28.5, 48 31.4 / 30.5; FP32 128 nz = 16 21.6 /
+    // 22.2, 32 23.4 / 23.9, 48 26.2 / 24.1; FP32 192 nz = 16 25.2 / 29.5, 32 30.3 / 33.3,
+    // 48 36.1 / 33.6; c2r FP32 192 nz = 16 28.9 / 29.4, 32 35.0 / 31.0 (96 and shorter:
+    // by plane at 16 too)
+    o.pair_r2c_nz = N < 128 ? 0 : 48;
+    o.pair_c2r_nz = N < 128 ? 0 : 32;
     o.pair_r2c = PairCfg<T, N>::ok ? &pair_r2c : nullptr;
     o.pair_c2r = PairCfg<T, N>::ok ? &pair_c2r : nullptr;
     return o;

@@ -3,7 +3,7 @@ over their input, non-finite modes that the reference drops."""
 import numpy as np
 import pytest
 
-from conftest import flush_print, rel_l2
+from conftest import flush_print, rel, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +75,23 @@ def test_get_phi_into_pinned_memory(vb, gpu, nx, nz):
         assert (out[:off] == -7.0).all() and (out[off + n:] == -7.0).all()
         for _ in range(3):
             assert np.array_equal(s.get_phi(), ref)
+
+
+# planes on either side of the rules between one kernel per plane and separate ones
+@pytest.mark.parametrize("nx,nz,prec", [(128, 16, "FP64"), (128, 32, "FP64"), (128, 48, "FP64"), (128, 32, "FP32_MIXED"),
+                                        (192, 16, "FP32_MIXED"), (192, 32, "FP32_MIXED"), (192, 48, "FP32_MIXED")])
+def test_transforms_of_few_planes(vb, gpu, oracle_mod, nx, nz, prec):
+    import torch
+    flush_print("few planes", nx, nz, prec)
+    fp64 = prec == "FP64"
+    u = np.random.default_rng(nx + nz).standard_normal((nz, nx, nx)).astype(np.float64 if fp64 else np.float32)
+    c = vb.Calc(nx, nz, precision=getattr(vb, prec))
+    ud = torch.from_numpy(u).to(gpu)
+    s = torch.empty((nz, nx, nx // 2 + 1), dtype=torch.complex128 if fp64 else torch.complex64, device=gpu)
+    c.r2c(ud, s)
+    # the bounds of the round trips in test_gpu_calc.py and test_gpu_plane.py
+    tol = 1e-14 if fp64 else 2e-6
+    assert rel_l2(s.cpu().numpy().astype(np.complex128), oracle_mod.Oracle(nx, nz).r2c(u.astype(np.float64))) < tol
+    keep, back = s.clone(), torch.empty_like(ud)
+    c.c2r(s, back)
+    assert rel_l2(back.cpu().numpy(), u) < tol and torch.equal(s, keep)
