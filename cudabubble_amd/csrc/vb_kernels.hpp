@@ -105,8 +105,8 @@ template <typename T, int N> constexpr int zsplan() {
   return (sizeof(T) == 4 && (N == 192 || N == 384)) ? 3 : (N == 32 || ((N == 64 || N == 128) && sizeof(T) == 8)) ? 4 : 0;
 }
 
-// Column tile of the z stage kernels (stage combines, z-prep, plain z
-// passes).  Up to 96, one wave's columns, so that the combines need no
+// Column tile of the z stage kernels (stage combines, z-prep; the plain z passes:
+// zpassw).  Up to 96, one wave's columns, so that the combines need no
 // workgroup barrier and a short grid spreads over more CUs (a 32^3 FP64 combine
 // was 9 workgroups of 256 threads): with the combine's operands and
 // coefficients loaded before its transforms (EARLY), 9.4 -> 6.4 us at 32^3 FP64
@@ -132,6 +132,15 @@ template <typename T, int N> constexpr int tbw_alt() { return tbw<T, N>() < colw
 // The z tile that short lengths take under a large plane, on the default plan
 // (get_zops); 0 where there is none.
 template <typename T, int N> constexpr int tbw_wide() { return N == 32 || N == 64 ? 32 : N == 128 && sizeof(T) == 8 ? 16 : 0; }
+
+// Column tile of the plain z passes (row layouts): the stage kernels' (TB), except
+// 16 columns, whole 128-byte lines, on the default plan in FP32 at 32, 64 and 96
+// (r2c of 384 x 96 99 -> 81 us, of 384 x 64 74 -> 62; in FP64 their 8 columns are
+// whole lines: c2r of 192 x 64 46 against 47 us) and in FP64 at 128 (a pass at
+// 128^3 11.1 us against 13.7 with four elements per thread).
+template <typename T, int N, int TB> constexpr int zpassw() {
+  return (sizeof(T) == 4 && (N == 32 || N == 64 || N == 96)) || (sizeof(T) == 8 && N == 128) ? 16 : TB;
+}
 
 // Z_p = A_ext(p) + i * B_ext(p): Hermitian extension along x of two half
 // spectra (rows A and B, whose Nyquist elements are at An and Bn).  The

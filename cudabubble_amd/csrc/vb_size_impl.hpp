@@ -26,6 +26,10 @@ struct Launch {
   static constexpr int ZV = (SC & kWideZ) ? 0 : zsplan<T, N>();   // plan of the z kernels
   static constexpr int XR = (SC & 2) ? xrplan_alt<T, N>() : xrplan<T, N>();
   static constexpr int YT = TB * TFof<N, ZV>();
+  // tile, plan and threads of the plain z passes (k_zpass, k_zmul)
+  static constexpr int PB = zpassw<T, N, TB>();
+  static constexpr int PV = PB == TB ? ZV : 0;
+  static constexpr int PT = PB * TFof<N, PV>();
   static constexpr int CV = colplan<T, N>();          // plan of the y passes and the z Laplacian
   static constexpr int CB = colw<T, N>();             // their columns per workgroup
   static constexpr int CT = CB * TFof<N, CV>();       // and threads per workgroup
@@ -101,9 +105,9 @@ struct Launch {
   static unsigned zgrid(const Geo& g) { return unsigned(zgroups(g, TB)); }
   static void zpass(cpx<T>* b, int sign, const Geo& g, const cpx<T>* tw, hipStream_t s) {
     if (sign < 0)
-      hipLaunchKernelGGL((k_zpass<T, N, -1, TB, ZV>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
+      hipLaunchKernelGGL((k_zpass<T, N, -1, PB, PV>), dim3(unsigned(zgroups(g, PB))), dim3(PT), 0, s, b, g, tw);
     else
-      hipLaunchKernelGGL((k_zpass<T, N, +1, TB, ZV>), dim3(zgrid(g)), dim3(YT), 0, s, b, g, tw);
+      hipLaunchKernelGGL((k_zpass<T, N, +1, PB, PV>), dim3(unsigned(zgroups(g, PB))), dim3(PT), 0, s, b, g, tw);
   }
   // FP32 at 192 would spill its 24 elements' v and f (a step 199 -> 209 us); FP64 at
   // 128 spilled 60 registers: nz = 16, 64, 128, 256 62, 84, 110, 169 us a step against
@@ -121,17 +125,17 @@ struct Launch {
   static void zmul(const cpx<T>* in, cpx<T>* out, int sign, int op, const Geo& gi, const Geo& go, const cpx<T>* tw,
                    hipStream_t s) {
     const ZmArgs<T> a{in, out, tw, gi, go};
-    const dim3 gr(unsigned(zgroups(go.aligned ? go : gi, TB))), bl(YT);
+    const dim3 gr(unsigned(zgroups(go.aligned ? go : gi, PB))), bl(PT);
     if (sign < 0) {
-      hipLaunchKernelGGL((k_zmul<T, N, -1, TB, ZM_ONE, ZV>), gr, bl, 0, s, a);
+      hipLaunchKernelGGL((k_zmul<T, N, -1, PB, ZM_ONE, PV>), gr, bl, 0, s, a);
       return;
     }
     switch (op) {
-      case ZM_LAP: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_LAP, ZV>), gr, bl, 0, s, a); break;
-      case ZM_DX: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DX, ZV>), gr, bl, 0, s, a); break;
-      case ZM_DY: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DY, ZV>), gr, bl, 0, s, a); break;
-      case ZM_DZ: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_DZ, ZV>), gr, bl, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_zmul<T, N, +1, TB, ZM_ONE, ZV>), gr, bl, 0, s, a); break;
+      case ZM_LAP: hipLaunchKernelGGL((k_zmul<T, N, +1, PB, ZM_LAP, PV>), gr, bl, 0, s, a); break;
+      case ZM_DX: hipLaunchKernelGGL((k_zmul<T, N, +1, PB, ZM_DX, PV>), gr, bl, 0, s, a); break;
+      case ZM_DY: hipLaunchKernelGGL((k_zmul<T, N, +1, PB, ZM_DY, PV>), gr, bl, 0, s, a); break;
+      case ZM_DZ: hipLaunchKernelGGL((k_zmul<T, N, +1, PB, ZM_DZ, PV>), gr, bl, 0, s, a); break;
+      default: hipLaunchKernelGGL((k_zmul<T, N, +1, PB, ZM_ONE, PV>), gr, bl, 0, s, a); break;
     }
   }
   static void pair_r2c(const T* u, cpx<T>* so, double scl, const Geo& g, const cpx<T>* tw, hipStream_t s) {

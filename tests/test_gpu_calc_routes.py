@@ -79,7 +79,8 @@ def test_get_phi_into_pinned_memory(vb, gpu, nx, nz):
 
 # planes on either side of the rules between one kernel per plane and separate ones
 @pytest.mark.parametrize("nx,nz,prec", [(128, 16, "FP64"), (128, 32, "FP64"), (128, 48, "FP64"), (128, 32, "FP32_MIXED"),
-                                        (192, 16, "FP32_MIXED"), (192, 32, "FP32_MIXED"), (192, 48, "FP32_MIXED")])
+                                        (192, 16, "FP32_MIXED"), (192, 32, "FP32_MIXED"), (192, 48, "FP32_MIXED"),
+                                        (96, 64, "FP32_MIXED"), (256, 96, "FP32_MIXED"), (192, 128, "FP64")])
 def test_transforms_of_few_planes(vb, gpu, oracle_mod, nx, nz, prec):
     import torch
     flush_print("few planes", nx, nz, prec)
