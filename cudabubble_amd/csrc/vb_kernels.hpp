@@ -242,7 +242,8 @@ __device__ __forceinline__ void st_nt(cpx<T>* p, cpx<T> v) {
 // ---------------------------------------------------------------------------
 // plain x transforms (pairs of rows)
 // ---------------------------------------------------------------------------
-template <typename TI, typename T, int N>
+// NT: the input is read past the caches
+template <typename TI, typename T, int N, bool NT>
 __global__ void __launch_bounds__(XWG) k_xr2c(const TI* __restrict__ in, cpx<T>* __restrict__ out,
                                                long long npairs, const cpx<T>* __restrict__ tw, double scl,
                                                Rows rl) {
@@ -258,7 +259,10 @@ __global__ void __launch_bounds__(XWG) k_xr2c(const TI* __restrict__ in, cpx<T>*
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int p = j + TF * e;
-    x[e] = mk<T>(T(__builtin_nontemporal_load(in + r0 * N + p)), T(__builtin_nontemporal_load(in + (r0 + 1) * N + p)));
+    if constexpr (NT)
+      x[e] = mk<T>(T(__builtin_nontemporal_load(in + r0 * N + p)), T(__builtin_nontemporal_load(in + (r0 + 1) * N + p)));
+    else
+      x[e] = mk<T>(T(in[r0 * N + p]), T(in[(r0 + 1) * N + p]));
   }
   fft<T, N, -1, XP>(x, j, tw, lds);
   unpack_store<T, N, XP>(x, j, lds, out + rl.off(r0), out + rl.nyq(r0, N / 2), out + rl.off(r0 + 1),
