@@ -96,3 +96,29 @@ def test_transforms_of_few_planes(vb, gpu, oracle_mod, nx, nz, prec):
     keep, back = s.clone(), torch.empty_like(ud)
     c.c2r(s, back)
     assert rel_l2(back.cpu().numpy(), u) < tol and torch.equal(s, keep)
+
+
+# with x and y in one kernel, in two, in two with aligned scratch rows
+@pytest.mark.parametrize("nx,nz", [(48, 16), (128, 16), (192, 16), (256, 32)])
+def test_etd41_is_the_inverse_of_its_combine(vb, gpu, oracle_mod, nx, nz):
+    """vb_calc_etd41 is the combine of vb_calc_etd42 and its inverse transform
+    (Calc.cu:488-517); its inputs are preserved, also where the output lies over one."""
+    import torch
+    flush_print("etd41", nx, nz)
+    _, f = _spectrum(oracle_mod, vb, nx, nz)
+    rng = np.random.default_rng(nx)
+    fd = torch.from_numpy(f).to(gpu)
+    nl = torch.from_numpy(oracle_mod.Oracle(nx, nz).r2c(rng.standard_normal((nz, nx, nx)))).to(gpu)
+    c, eps, h = vb.Calc(nx, nz), 4 * np.pi / nx, 1e-5
+    b = torch.empty_like(fd)
+    c.etd42(b, fd, nl, eps, h)
+    real = lambda: torch.empty((nz, nx, nx), dtype=torch.float64, device=gpu)
+    ref, out, kf, kn = real(), real(), fd.clone(), nl.clone()
+    c.c2r(b, ref)
+    c.etd41(out, fd, nl, eps, h)
+    # one inverse transform's rounding either way
+    assert rel_l2(out.cpu().numpy(), ref.cpu().numpy()) < 1e-14
+    assert torch.equal(fd, kf) and torch.equal(nl, kn)
+    over = torch.view_as_real(nl).reshape(-1)[:nz * nx * nx].view(nz, nx, nx)
+    c.etd41(over, fd, nl, eps, h)
+    assert torch.equal(over, out)
