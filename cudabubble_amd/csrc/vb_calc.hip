@@ -98,12 +98,15 @@ __global__ void __launch_bounds__(256) k_sum(const double* __restrict__ u, long 
   __shared__ double red[4];
   const long long b0 = (long long)blockIdx.x * chunk;
   const long long e = b0 + chunk < n ? b0 + chunk : n;
-  double s[4] = {};   // four loads in flight
-  for (long long i = b0 + threadIdx.x; i < e; i += 1024) {
+  double s[4] = {};   // four loads in flight, the guarded last round apart
+  long long i = b0 + threadIdx.x;
+  for (; i + 768 < e; i += 1024) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (i + 256 * k < e) s[k] += u[i + 256 * k];
+    for (int k = 0; k < 4; ++k) s[k] += u[i + 256 * k];
   }
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (i + 256 * k < e) s[k] += u[i + 256 * k];
   double acc[1] = {(s[0] + s[1]) + (s[2] + s[3])};
   block_sum_store<1, 256>(acc, red, part + blockIdx.x);
 }

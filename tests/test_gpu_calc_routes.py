@@ -122,3 +122,20 @@ def test_etd41_is_the_inverse_of_its_combine(vb, gpu, oracle_mod, nx, nz):
     over = torch.view_as_real(nl).reshape(-1)[:nz * nx * nx].view(nz, nx, nx)
     c.etd41(over, fd, nl, eps, h)
     assert torch.equal(over, out)
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 768, 769, 1023, 1024, 1025, 4095, 4096, 4097, 100003,
+                               4096 * 4096, 4096 * 4096 + 1, 2 * 4096 * 4096 + 4099])
+def test_integral_of_any_length(vb, gpu, n):
+    """Lengths that no chunk, round of four loads or workgroup divides, on either side
+    of the chunk's first doubling."""
+    import torch
+    flush_print("intf_static", n)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    u = torch.rand(n, generator=g, dtype=torch.float64, device=gpu) + 0.5
+    val = torch.zeros(1, dtype=torch.float64, device=gpu)
+    vb.intf_static(u, 2.0, 0.25, 3.0, val)
+    torch.cuda.synchronize()
+    # partial sums of at most 65536 / 1024 rounds, the rest pairwise: far below 200 ulps
+    ref = (float(np.mean(u.cpu().numpy())) + 0.25) * 3.0 * 8.0
+    assert rel(float(val), ref) < 200 * 2.0 ** -53
