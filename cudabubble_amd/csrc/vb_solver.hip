@@ -1418,6 +1418,10 @@ struct Solver final : SolverBase {
       VB_HIP(hipStreamSynchronize(st));
       if (c.status != SHAPE_RUN) break;
     }
+    // the state's prefix is in place, but the partial sums are those of the chain's
+    // last attempt, rejected or past the end: whoever needs the state's integrals
+    // under other targets takes the prefix again
+    prefixed_f = false;
     hs_state = false;
   }
 

@@ -36,3 +36,24 @@ def test_euler_steps_and_residual(vb, gpu, oracle_mod, nx, nz, prec):
         o.set_targets(s.state()["alpha"], s.state()["beta"])
         ref = np.mean(o.sum_fgq(d) ** 2) * (2 * np.pi) ** 3
         assert rel(s.residual(), ref) < (1e-11 if fp64 else 1e-4) * max(1.0, (nx / 32.0) ** 2)
+
+
+@pytest.mark.parametrize("prec", ["FP64", "FP32_MIXED"])
+@pytest.mark.parametrize("n", [32, 96])
+def test_euler_after_shape_adjustment_on_the_device(vb, gpu, n, prec):
+    """The shape loop with its decisions on the device ends behind attempts that were
+    rejected or did not run; the driver that follows starts from the state's own
+    integrals, as after the loop on the host."""
+    flush_print("euler after shape chain", n, prec)
+    eps = 2.0 * 2 * np.pi / n
+    phi, _ = vb.shape(1, 20260002, n, n, 1.0, eps)
+    runs = []
+    for chain in (0, 8):
+        s = vb.Solver(vb.params_default(nx=n, nz=n, eps=eps, scheme=vb.EULER, shape_adjust=1, M1=1e4, M2=1e4, alpha=-1.0,
+                                        beta=-1.0, time_step=1e-7, fixed_time_step=1e-7, accept_chain=chain,
+                                        precision=getattr(vb, prec)), phi)
+        s.step(0)
+        q = s.query()
+        s.step(2)
+        runs.append((q, s.state(), s.query(), s.get_phi()))
+    assert runs[0][:3] == runs[1][:3] and np.array_equal(runs[0][3], runs[1][3])
