@@ -20,9 +20,6 @@
 #include <type_traits>
 
 #include "vb_device.hpp"
-#ifndef VB_XREV
-#define VB_XREV true
-#endif
 
 namespace vb {
 
