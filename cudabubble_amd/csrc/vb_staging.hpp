@@ -26,16 +26,17 @@ void staging_user(int d);   // +1 / -1: a solver was created / destroyed
 // small one, a single slot), on the current device.  Blocks are kept for reuse,
 // at most two of each kind, and freed when the last solver goes.
 // A new block costs its allocation and the page faults of its first pass: 0.02 ms
-// for a 32^3 field, 0.75 at 64^3, 2 at 96^3 and 128^3, where a read saves 0.01,
-// 0.02, 0.13, 0.45.  staging_pays says when the reads of one solver have come to
-// about that: `before` bytes so far, this one of `bytes`.
+// for a 32^3 field, 0.75 at 64^3, up to 2 at 96^3 and 128^3, 3.5 at 256 x 64 and
+// 192^3 (much less where the runtime still has the memory of a freed one), where a
+// read saves 0.01, 0.02, 0.13, 0.45, 2.0, 3.8.  staging_pays says when the reads of
+// one solver have come to about that: `before` bytes so far, this one of `bytes`.
 struct StagingJob {
   virtual void produce(long long first, long long count, void* p) = 0;
   virtual ~StagingJob() = default;
 };
 bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st, bool make);
 inline bool staging_pays(size_t before, size_t bytes) {
-  return bytes <= (size_t)1 << 20 ? before > 0 : before + bytes >= (size_t)64 << 20;
+  return bytes <= (size_t)1 << 20 ? before > 0 : before + bytes >= (size_t)32 << 20;
 }
 
 }  // namespace vb

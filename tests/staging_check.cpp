@@ -250,8 +250,8 @@ static void make() {
   CHECK(g_blocks == 0);
   const size_t M = (size_t)1 << 20;
   CHECK(!vb::staging_pays(0, M / 4) && vb::staging_pays(M / 4, M / 4));
-  CHECK(!vb::staging_pays(0, 2 * M) && !vb::staging_pays(60 * M, 2 * M) && vb::staging_pays(62 * M, 2 * M));
-  CHECK(!vb::staging_pays(0, 57 * M) && vb::staging_pays(57 * M, 57 * M) && vb::staging_pays(0, 128 * M));
+  CHECK(!vb::staging_pays(0, 2 * M) && !vb::staging_pays(28 * M, 2 * M) && vb::staging_pays(30 * M, 2 * M));
+  CHECK(!vb::staging_pays(0, 16 * M) && vb::staging_pays(16 * M, 16 * M) && vb::staging_pays(0, 54 * M));
 }
 
 int main(int argc, char** argv) {
