@@ -382,19 +382,23 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_pair(PairArgs<T> a) {
 // round of planes fills at most half of the 256 CUs gives these planes two
 // workgroups each (nsplit): both invert P and Q and take the pointwise terms, one
 // transforms tmp1 and writes the sums, the other s; the second read of P and Q
-// comes from the XCD's L2.  What remains is latency and LDS: 9 000 of about
-// 45 000 cycles issue VALU.  Measured, us per step:
+// comes from the XCD's L2.  What remains is arithmetic, latency and LDS: in a
+// batch of 12 x 128^3 FP32 the SIMDs issue VALU work in 48 % of the cycles and the
+// waves wait in 35 % of theirs (one solve: 37 and 29).  FP64 at 128 spills 25
+// registers: nine waves, the Nyquist column's being the ninth, leave 168 each.
+// Measured, us per step:
 //   128^3 FP64 drift: three kernels 627, one workgroup per plane 606, two 556;
 //     batches of 3 and 4 (the rest of 384 split; 512) 1375 -> 1303, 1594
 //   128^3 FP32 drift: k_plane 418, here 388; batches of 2, 3, 12: 572, 863,
 //     2832 -> 572, 832, 2800
 //   96^3 FP64: k_plane 414, here 380; batches of 2, 6: 605, 1445 -> 589, 1401
 //   64^3 FP32: 138 both; batches of 6, 16: 307, 617 -> 287, 577
-// k_plane stays at the others: 96^3 FP32 batches of 2 and 6 365, 829 against 391,
-// 884, 64^3 FP64 batch of 4 283 against 302, 32^3 and 48^3 5 % and more.  (FP32 at
-// 192 fits as well but spills 78 registers: 76 us against 75.)  PL_SUMS takes one
-// plane per workgroup here; it and PL_ROWSUMS run here only where k_plane does
-// not fit.
+// k_plane stays at the others, k_plane / here: 96^3 FP32 288 / 287, batches of 2
+// and 6 363, 822 / 385, 880; 64^3 FP64 172 / 171, a batch of 4 284 / 299; 48^3 FP64
+// 171 / 181, FP32 156 / 167, 4 of FP64 242 / 269; 32^3 FP64 98 / 104, FP32 97 / 103,
+// 16 of FP64 232 / 247.  (FP32 at 192 fits as well but spills 78 registers: 76 us a
+// launch against 75.)  PL_SUMS takes one plane per workgroup here; it and
+// PL_ROWSUMS run here only where k_plane does not fit.
 // ---------------------------------------------------------------------------
 template <typename T, int N>
 struct Plane2Cfg {
@@ -613,7 +617,8 @@ __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_plane2(PlaneArgs<T> a0,
 // The Forward-Euler update of a plane in LDS: the y and x inverse of W (x and y
 // spectra of lap f), k_xe's update, the x and y forward of the new field over W.
 // With PL_EULER and k_zeuler a fixed-dt Euler step is four kernels instead of
-// ten: 64^3 FP64 53 -> 33 us, 32^3 FP32 38 -> 19, 128^3 FP32 98 -> 68.
+// ten: 64^3 FP64 53 -> 33 us, 32^3 FP32 38 -> 19, 128^3 FP32 98 -> 68.  Used where
+// it is the faster form (kXePlane, xe_min_nz).
 // ---------------------------------------------------------------------------
 template <typename T, int N>
 __global__ void __launch_bounds__((PairCfg<T, N>::NA)) k_xe_plane(XeArgs<T> a, Geo g) {

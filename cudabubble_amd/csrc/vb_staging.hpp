@@ -6,8 +6,8 @@
 // by a few host threads as their events complete, so the transfer, the copies
 // and the page faults of a fresh destination overlap.  (A copy from device
 // memory into pageable memory went through the runtime's own staging in 1 MB
-// pieces on one thread.)  vb_get_phi, ms: 32^3 0.15 -> 0.04, 128^3 1.20 -> 0.75,
-// 256^3 13.0 -> 3.3, 384^3 43.9 -> 10.7.
+// pieces on one thread.)  vb_get_phi, ms, once a block is there: 32^3 0.046 -> 0.036,
+// 128^3 1.22 -> 0.75, 256^3 12.8 -> 3.3, 384^3 43.6 -> 10.3.
 #pragma once
 #include <cstddef>
 
