@@ -139,3 +139,33 @@ def test_integral_of_any_length(vb, gpu, n):
     # partial sums of at most 65536 / 1024 rounds, the rest pairwise: far below 200 ulps
     ref = (float(np.mean(u.cpu().numpy())) + 0.25) * 3.0 * 8.0
     assert rel(float(val), ref) < 200 * 2.0 ** -53
+
+
+def test_get_phi_from_several_threads(vb, gpu):
+    """Solvers of several sizes created, read (past the reads that make a pinned
+    block) and destroyed by four threads at a time."""
+    import threading
+    errors = []
+
+    def work(t):
+        try:
+            for r, n in enumerate([(32, 64, 96, 128)[(t + r) % 4] for r in range(4)]):
+                eps = 2.0 * 2 * np.pi / n
+                phi, _ = vb.shape(vb.SHAPE_ELLIPSOID, 100 * t + r, n, n, 1.0, eps)
+                s = vb.Solver(vb.params_default(nx=n, nz=n, eps=eps, M1=1e3, M2=1e3, time_step=1e-7,
+                                                fixed_time_step=1e-7), phi)
+                first = s.get_phi()
+                assert rel_l2(first, phi) < 1e-14      # the round trip of the transforms
+                for _ in range(5):
+                    assert np.array_equal(s.get_phi(), first)
+                s.close()
+        except BaseException as e:   # re-raised below, in the test's thread
+            errors.append((t, e))
+
+    flush_print("get_phi from threads")
+    th = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors, errors
