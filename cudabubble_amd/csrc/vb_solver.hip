@@ -136,7 +136,6 @@ struct Solver final : SolverBase {
   hipStream_t st = nullptr;
   bool own_stream = false;
   bool staging_counted = false;
-  size_t phi_read = 0;   // bytes that get_phi has returned (staging_pays)
   const SizeOps<T>* ox = nullptr;
   const SizeOps<T>* oz = nullptr;
   // FP64 operations (state transforms, FP64 queries in mixed mode)
@@ -1698,15 +1697,10 @@ struct Solver final : SolverBase {
         s.check_launch();
       }
     } job(*this);
-    const size_t plane = sizeof(double) * (size_t)g.nx * g.ny, bytes = plane * (size_t)g.nz;
     // pageable memory only: to memory the runtime knows (pinned, or a device's) one
     // copy from the device buffer does it, faster (to pinned memory 64^3 71 us against
     // 129 through a block, 128^3 356 against 524, 256^3 2.54 ms against 2.91)
-    if (pageable(host)) {
-      const bool make = staging_pays(phi_read, bytes);
-      phi_read += bytes;
-      if (staging_copy_out(job, g.nz, plane, host, st, make)) return;
-    }
+    if (pageable(host) && staging_copy_out(job, g.nz, sizeof(double) * (size_t)g.nx * g.ny, host, st)) return;
     // through the device buffer
     L("x_c2r", [&] { oxd->xc2r_d(S.p, phid.p, npairs, twxd.p, g, st); });
     check_launch();

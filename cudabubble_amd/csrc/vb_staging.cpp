@@ -26,6 +26,7 @@ constexpr int kThreads = 6, kKeep = 2;
 std::mutex g_mu;
 std::vector<Block*> g_idle;
 int g_users = 0;
+size_t g_read = 0;   // bytes that copies were asked for since the first solver
 
 void destroy(Block* s) {
   for (auto e : s->ev)
@@ -35,7 +36,7 @@ void destroy(Block* s) {
 }
 
 // a block for a field of that size, nullptr where there is none to be had
-Block* acquire(size_t field_bytes, bool make) {
+Block* acquire(size_t field_bytes) {
   const size_t slot = field_bytes <= kSmall ? kSmall : kLarge;
   int dev = 0;
   VB_HIP(hipGetDevice(&dev));
@@ -45,10 +46,13 @@ Block* acquire(size_t field_bytes, bool make) {
       if (g_idle[i]->slot == slot && g_idle[i]->device == dev) {
         Block* s = g_idle[i];
         g_idle.erase(g_idle.begin() + (long)i);
+        g_read += field_bytes;
         return s;
       }
+    const bool pays = staging_pays(g_read, field_bytes);
+    g_read += field_bytes;
+    if (!pays) return nullptr;
   }
-  if (!make) return nullptr;
   Block* s = new Block;
   s->slot = slot;
   s->device = dev;
@@ -86,13 +90,16 @@ void staging_user(int d) {
   {
     std::lock_guard<std::mutex> l(g_mu);
     g_users += d;
-    if (g_users <= 0) drop.swap(g_idle);
+    if (g_users <= 0) {
+      drop.swap(g_idle);
+      g_read = 0;
+    }
   }
   for (auto* s : drop) destroy(s);
 }
 
-bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st, bool make) {
-  Block* const s = acquire((size_t)items * item_bytes, make);
+bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st) {
+  Block* const s = acquire((size_t)items * item_bytes);
   if (!s) return false;
   try {
     copy_out(s, job, items, item_bytes, dst, st);

@@ -20,21 +20,22 @@ void staging_user(int d);   // +1 / -1: a solver was created / destroyed
 // Copies a field of `items` items (planes) of item_bytes to dst.  produce(first,
 // count, p) launches on st the kernels that write items [first, first + count)
 // to pinned memory p.  Returns true when dst is complete, or false, with nothing
-// launched, where no pinned block can be had: none is idle, and `make` does not
-// allow a new one or there is no memory for it.
+// launched, where there is no pinned block for it: none is idle, and a new one
+// does not pay yet (staging_pays) or cannot be had.
 // A call holds one block, of one of two slot sizes (fields of up to 2 MB take the
 // small one, a single slot), on the current device.  Blocks are kept for reuse,
 // at most two of each kind, and freed when the last solver goes.
-// A new block costs its allocation and the page faults of its first pass: 0.02 ms
-// for a 32^3 field, 0.75 at 64^3, up to 2 at 96^3 and 128^3, 3.5 at 256 x 64 and
-// 192^3 (much less where the runtime still has the memory of a freed one), where a
-// read saves 0.01, 0.02, 0.13, 0.45, 2.0, 3.8.  staging_pays says when the reads of
-// one solver have come to about that: `before` bytes so far, this one of `bytes`.
 struct StagingJob {
   virtual void produce(long long first, long long count, void* p) = 0;
   virtual ~StagingJob() = default;
 };
-bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st, bool make);
+bool staging_copy_out(StagingJob& job, long long items, size_t item_bytes, void* dst, hipStream_t st);
+
+// A new block costs its allocation and the page faults of its first pass: 0.02 ms
+// for a 32^3 field, 0.75 at 64^3, up to 2 at 96^3 and 128^3, 3.5 at 256 x 64 and
+// 192^3 (much less where the runtime still has the memory of a freed one), where a
+// read saves 0.01, 0.02, 0.13, 0.45, 2.0, 3.8.  So one is made when the reads since
+// the first solver have come to about that: `before` bytes, and this one of `bytes`.
 inline bool staging_pays(size_t before, size_t bytes) {
   return bytes <= (size_t)1 << 20 ? before > 0 : before + bytes >= (size_t)32 << 20;
 }

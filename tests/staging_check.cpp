@@ -142,12 +142,13 @@ struct Fill final : vb::StagingJob {
   }
 };
 
-static bool one(long long items, size_t item, unsigned seed, bool make = true) {
+// false: there was no block, and nothing was launched
+static bool one(long long items, size_t item, unsigned seed) {
   Stream s;
   Fill f(s, item, seed);
   std::vector<unsigned> out((size_t)items * item / 4 + 1, 0xdeadbeefu);
-  if (!vb::staging_copy_out(f, items, item, out.data(), reinterpret_cast<hipStream_t>(&s), make)) {
-    CHECK(!make && f.calls == 0);
+  if (!vb::staging_copy_out(f, items, item, out.data(), reinterpret_cast<hipStream_t>(&s))) {
+    CHECK(f.calls == 0 && out[0] == 0xdeadbeefu);
     return false;
   }
   for (long long i = 0; i < items; ++i)
@@ -156,19 +157,23 @@ static bool one(long long items, size_t item, unsigned seed, bool make = true) {
   return true;
 }
 
+// a first read large enough for blocks to pay from here on
+static void warm() { CHECK(one(32, (size_t)1 << 20, 77)); }
+
 // sizes: one slot, exactly one, just past it, ragged last chunks, more chunks
 // than slots, one item per slot
 static void sizes() {
   vb::staging_user(1);
+  warm();
   const size_t M = (size_t)1 << 20;
-  one(1, 4096, 1);
-  one(16, 16 * 16 * 8, 2);
-  one(2, M, 3);
-  one(3, M, 4);
-  one(17, M, 5);
-  one(67, M / 2, 6);
-  one(41, 4 * M, 7);
-  one(13, 3 * M, 8);
+  CHECK(one(1, 4096, 1));
+  CHECK(one(16, 16 * 16 * 8, 2));
+  CHECK(one(2, M, 3));
+  CHECK(one(3, M, 4));
+  CHECK(one(17, M, 5));
+  CHECK(one(67, M / 2, 6));
+  CHECK(one(41, 4 * M, 7));
+  CHECK(one(13, 3 * M, 8));
   vb::staging_user(-1);
   CHECK(g_blocks == 0 && g_events == 0);
 }
@@ -180,7 +185,7 @@ static void threads() {
     th.emplace_back([t] {
       for (int r = 0; r < 4; ++r) {
         vb::staging_user(1);
-        one(t % 2 ? 9 : 37, t % 2 ? 65536 : 262144, unsigned(16 * t + r));
+        (void)one(t % 2 ? 9 : 37, t % 2 ? 65536 : 262144, unsigned(16 * t + r));
         vb::staging_user(-1);
       }
     });
@@ -191,12 +196,13 @@ static void threads() {
 // blocks are kept while a solver lives, at most two of a kind, then freed
 static void pool() {
   vb::staging_user(1);
+  warm();
   std::vector<std::thread> th;
-  for (int t = 0; t < 5; ++t) th.emplace_back([t] { one(37, 262144, unsigned(t)); });
+  for (int t = 0; t < 5; ++t) th.emplace_back([t] { CHECK(one(37, 262144, unsigned(t))); });
   for (auto& t : th) t.join();
   CHECK(g_blocks <= 2);
   const int n = g_mallocs;
-  one(37, 262144, 9);
+  CHECK(one(37, 262144, 9));
   CHECK(g_mallocs == n);
   vb::staging_user(-1);
   CHECK(g_blocks == 0);
@@ -204,6 +210,7 @@ static void pool() {
 
 static void launch_failure() {
   vb::staging_user(1);
+  warm();
   for (long long at : {0, 1, 9}) {
     Stream s;
     Fill f(s, 262144, 3);
@@ -211,13 +218,13 @@ static void launch_failure() {
     std::vector<unsigned> out((size_t)200 * 65536);
     bool threw = false;
     try {
-      (void)vb::staging_copy_out(f, 200, 262144, out.data(), reinterpret_cast<hipStream_t>(&s), true);
+      (void)vb::staging_copy_out(f, 200, 262144, out.data(), reinterpret_cast<hipStream_t>(&s));
     } catch (const std::runtime_error&) {
       threw = true;
     }
     CHECK(threw);
   }
-  one(37, 262144, 5);
+  CHECK(one(37, 262144, 5));
   vb::staging_user(-1);
   CHECK(g_blocks == 0 && g_events == 0);
 }
@@ -230,25 +237,34 @@ static void no_pinned() {
     Stream s;
     Fill f(s, 262144, 3);
     std::vector<unsigned> out((size_t)items * 65536, 7u);
-    CHECK(!vb::staging_copy_out(f, items, 262144, out.data(), reinterpret_cast<hipStream_t>(&s), true));
+    CHECK(!vb::staging_copy_out(f, items, 262144, out.data(), reinterpret_cast<hipStream_t>(&s)));
     CHECK(f.calls == 0 && out[0] == 7u && out.back() == 7u);
   }
   g_no_pinned = false;
-  one(37, 262144, 5);
+  CHECK(one(37, 262144, 5));
   vb::staging_user(-1);
   CHECK(g_blocks == 0 && g_events == 0);
 }
 
-// a block is made only where it pays; an idle one serves every reader
+// a block is made when it pays, over all solvers there are; an idle one serves
+// every reader
 static void make() {
+  const size_t M = (size_t)1 << 20;
   vb::staging_user(1);
-  CHECK(!one(16, 131072, 1, false) && g_mallocs == 0);
-  CHECK(one(16, 131072, 1, true) && g_mallocs == 1);
-  CHECK(one(16, 131072, 2, false) && g_mallocs == 1);
-  CHECK(!one(37, 262144, 3, false) && g_mallocs == 1);   // the other kind
+  CHECK(!one(16, M / 64, 1) && g_mallocs == 0);   // 256 KB: the first read
+  CHECK(one(16, M / 64, 1) && g_mallocs == 1);    // and the second
+  CHECK(one(16, M / 8, 2) && g_mallocs == 1);     // 2 MB: the idle one
+  CHECK(!one(40, M / 8, 3) && g_mallocs == 1);    // the other kind
+  vb::staging_user(1);
+  CHECK(one(32, M, 3) && g_mallocs == 2);
+  CHECK(one(40, M / 8, 3) && g_mallocs == 2);
+  vb::staging_user(-1);
+  CHECK(g_blocks == 2);
   vb::staging_user(-1);
   CHECK(g_blocks == 0);
-  const size_t M = (size_t)1 << 20;
+  vb::staging_user(1);   // counted from the first solver again
+  CHECK(!one(40, M / 8, 3) && g_mallocs == 2);
+  vb::staging_user(-1);
   CHECK(!vb::staging_pays(0, M / 4) && vb::staging_pays(M / 4, M / 4));
   CHECK(!vb::staging_pays(0, 2 * M) && !vb::staging_pays(28 * M, 2 * M) && vb::staging_pays(30 * M, 2 * M));
   CHECK(!vb::staging_pays(0, 16 * M) && vb::staging_pays(16 * M, 16 * M) && vb::staging_pays(0, 54 * M));
